@@ -389,6 +389,13 @@ struct bfmx_system {
 	float* d_mp_h[4] = {nullptr, nullptr, nullptr, nullptr};   // hidden features (FP32, 64 per node)
 	double* d_mp_z = nullptr;          // its output (FP64, 2 per node)
 
+	// register-resident PCG (resident.hip): its workgroups (-1: not looked at,
+	// 0: the system does not fit), the nodes of their widest window, the
+	// blocks of the longest row
+	int res_groups = -1;
+	int res_window = 0;
+	int res_width = 0;
+
 	bool assembled = false;
 	bool finalized = false;
 	bool borrowed = false;   // belongs to a batch built from meshes: device arrays inside its arenas
@@ -555,6 +562,12 @@ struct PcgBuffers {
 // graph capture); *out receives the final scalars, the solution stays in
 // w.x (internal node order). The system's own solver buffers are untouched.
 int pcg_in_buffers(bfmx_system* s, PcgBuffers const& w, int precond, double rtol, int64_t cap, Scalars* out);
+// resident.hip: point or block Jacobi PCG of s->d_bsolve in the solver's
+// buffers, with the matrix held in registers, from x = 0 or (warm) from
+// s->d_x; *ran is false (and nothing but the buffers changed) when the system
+// does not fit or the device could not run it. *out: the final scalars.
+int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double delta2, int64_t cap, bool warm,
+                 Scalars* out, bool* ran);
 // noalloc.hip: bfmx_system_solve_noalloc, and the largest system (nodes) its
 // fixed scratch array holds.
 int solve_noalloc(bfmx_system* s, const double* b_in, double* u_out, int precond, double rtol, size_t max_iter,

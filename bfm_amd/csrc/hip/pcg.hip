@@ -1,5 +1,10 @@
 // Preconditioned conjugate gradients on the device.
 //
+// Point and block Jacobi PCG of a system whose matrix fits the GPU's registers
+// (up to 262,144 nodes, rows of at most nine blocks) runs in one launch
+// (resident.hip, three to five times as fast); the kernels here take the
+// larger systems and those it refuses.
+//
 // One CG iteration is four kernels:
 //   k_cg_spmv    p_new = z + beta p_old and q = A p_new for its rows, gathering
 //                z and p_old at the block columns (so the direction update
@@ -44,7 +49,7 @@
 #include <cmath>
 #include <cstdlib>
 
-#include "internal.h"
+#include "resident.h"
 
 namespace bfmx {
 
@@ -265,24 +270,6 @@ __device__ __forceinline__ dbl2 row_spmv(const int32_t* __restrict__ slice_ptr, 
 		y1 += u.x * xv.x + u.y * xv.y;
 	}
 	return dbl2{y0, y1};
-}
-
-// s - a x accumulated without losing its rounding errors: s carries the
-// running sum and c the sum of the errors, so that s + c is the row's
-// b - sum A_ij x_j as accurately as if it were summed in twice the working
-// precision and then rounded (the product's error exactly from an FMA,
-// Knuth's TwoSum for the difference; Ogita, Rump and Oishi, SIAM J. Sci.
-// Comput. 26 (2005) 1955-1988, Algorithm Dot2). Contraction is off here: a
-// fused s - a x would not be the rounded difference the error terms assume.
-__device__ __forceinline__ void sub_exact(double& s, double& c, double a, double x) {
-#pragma clang fp contract(off)
-	double const p = a * x;
-	double const pe = fma(a, x, -p);   // a x = p + pe exactly
-	double const t = s - p;
-	double const z = t - s;
-	double const e = (s - (t - z)) + (-p - z);   // s - p = t + e exactly
-	s = t;
-	c += e - pe;
 }
 
 // b - A x for one block row, compensated (sub_exact).
@@ -978,6 +965,14 @@ int run_chunks(bfmx_system* s, int precond, bool mixed, double rtol2, int64_t ca
                Scalars* out) {
 	int64_t const n = s->n_nodes;
 	hipStream_t const st = s->stream;
+	if (!is_fcg(precond)) {
+		// in one launch, where the matrix fits the GPU's registers
+		bool ran = false;
+		BFMX_CHECK(resident_pcg(s, precond, mixed, rtol2, mixed ? kDelta2 : 0.0, cap, warm, out, &ran));
+		if (ran) {
+			return BFMX_OK;
+		}
+	}
 	// Chunks go through captured graphs from a system's second solve with a
 	// preconditioner on: capturing and instantiating them costs about as much
 	// as a large system's whole launch overhead (2M-DOF beam, multigrid FCG:
@@ -1671,6 +1666,11 @@ int pcg_in_buffers(bfmx_system* s, PcgBuffers const& w, int precond, double rtol
 	s->partial_cap = w.partial_cap;
 	s->d_scal = w.scal;
 	double const rtol2 = rtol * rtol;
+	bool ran = false;
+	BFMX_CHECK(resident_pcg(s, precond, false, rtol2, 0.0, cap, false, out, &ran));
+	if (ran) {
+		return BFMX_OK;
+	}
 	k_precond<<<grid(n), kBlock, 0, st>>>(static_cast<int>(n), precond, s->d_diag_blk, s->d_val, s->d_dinv);
 	for (double* v : {w.x, w.q, w.p0, w.p1}) {
 		k_zero<<<grid(2 * n), kBlock, 0, st>>>(2 * n, v);

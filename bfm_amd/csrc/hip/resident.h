@@ -1,0 +1,648 @@
+// PCG with the matrix held in registers (device code shared by the solve of
+// one system and by batches).
+//
+// The streaming kernels of pcg.hip read the whole matrix from memory in every
+// iteration and end each of its two dot products at a kernel boundary: below
+// some 260,000 nodes an iteration is then bound by four launches and by the
+// latency of its loads, not by bandwidth (13 us an iteration from 451 to
+// 23,000 nodes, 32 us at 251,000). Here a cluster of G workgroups runs the
+// whole iteration loop in one launch:
+//   * one block row per thread, its blocks in registers (a CU's 512 KB of
+//     registers hold 1024 rows of nine FP64 blocks), x, r, z and the inverse
+//     diagonal beside them;
+//   * the direction p of a workgroup's own rows and of the nodes their columns
+//     reach (a contiguous window, since the nodes are in RCM order) in LDS;
+//     every workgroup forms p = z + beta p for its whole window, so that only
+//     z is exchanged;
+//   * z and the partial dot products travel through memory in 8-byte words of
+//     32 data bits and the 32-bit number of the exchange, written and read with
+//     agent-scope relaxed atomics (which pass by the XCDs' incoherent L2s). A
+//     reader polls the word itself until it carries the expected number, so an
+//     exchange costs one store-to-load latency (1.4 us up to 8 workgroups, 3.7
+//     at 256) and needs no fence, no flag and no wait for the stores.
+// Measured on one MI355X, microseconds an iteration, streaming -> here: 451 nodes
+// (one workgroup) 13.8 -> 1.7; 1,105 (two) 13.3 -> 4.4; 5,124 (six) 13.3 -> 4.8;
+// 22,952 (23) 13.4 -> 4.8; 63,126 (62) 16.4 -> 5.3; 251,251 (246) 32.7 -> 10.0,
+// point Jacobi on Q1 beams (22,952: block Jacobi, FP32 matrix, P1). Above one
+// workgroup the two all-gathers bound it.
+// A word is overwritten two exchanges later at the earliest, after an
+// all-gather to which every workgroup contributed past its last read of it.
+// Every workgroup forms the same sums in the same order, so all of them take
+// the same branches; the result does not depend on scheduling.
+//
+// The workgroups of a cluster must be resident together: launches are
+// cooperative, and every wait is bounded (kSpinLimit polls), so that each
+// workgroup ends whatever happens; the caller then solves with the streaming
+// kernels.
+#pragma once
+
+#include "internal.h"
+
+namespace bfmx {
+
+// s - a x accumulated without losing its rounding errors: s carries the
+// running sum and c the sum of the errors, so that s + c is the row's
+// b - sum A_ij x_j as accurately as if it were summed in twice the working
+// precision and then rounded (the product's error exactly from an FMA,
+// Knuth's TwoSum for the difference; Ogita, Rump and Oishi, SIAM J. Sci.
+// Comput. 26 (2005) 1955-1988, Algorithm Dot2). Contraction is off here: a
+// fused s - a x would not be the rounded difference the error terms assume.
+__device__ __forceinline__ void sub_exact(double& s, double& c, double a, double x) {
+#pragma clang fp contract(off)
+	double const p = a * x;
+	double const pe = fma(a, x, -p);   // a x = p + pe exactly
+	double const t = s - p;
+	double const z = t - s;
+	double const e = (s - (t - z)) + (-p - z);   // s - p = t + e exactly
+	s = t;
+	c += e - pe;
+}
+
+namespace resident {
+
+typedef double dbl2 __attribute__((ext_vector_type(2)));
+typedef float flt2 __attribute__((ext_vector_type(2)));
+typedef unsigned long long u64;
+
+constexpr uint32_t kSpinLimit = 1u << 22;   // polls of one wait (seconds)
+constexpr int kSlotWords = 8;               // words of one workgroup's contribution to an all-gather
+constexpr int kMaxGroup = 256;              // workgroups of a cluster
+constexpr int kMaxWindow = 3900;            // nodes of a window (62 KB of the CU's 160 KB of LDS, beside 96 KB of row blocks)
+constexpr int kMaxWidth = 9;                // blocks of a row held in registers
+constexpr int kCheckEvery = 16;             // iterations between true-residual checks once one has failed
+constexpr int kStall = 8;                   // such checks without halving before the run counts as stalled
+constexpr int kFailed = 5;                  // status: a bounded wait ran out
+
+// One system's arrays. The exchange uses the solver's vector buffers (16
+// bytes a node each): words 0 and 1, 2 and 3 of the two parities in w[0..3],
+// the all-gather slots in slots. All five are zeroed before the launch.
+struct View {
+	const int32_t* slice_ptr;
+	const int32_t* col;
+	const int32_t* diag_blk;
+	const double* val;      // FP64 matrix
+	const float* val32;     // FP32 copy (mixed precision)
+	const double* b;
+	double* x;
+	u64* w[4];
+	u64* slots;
+	double* save;           // 4 doubles a node: r and p of a run cut at its iteration limit
+	int64_t n;
+};
+
+// Scalars of a run, the same in every workgroup.
+struct Run {
+	double rz, rr, bb, tol2, beta, rr_true, rr_ref, rr_best, pq;
+	int64_t iter;
+	int32_t status;    // 0 running (limit reached), 1 converged, 2 breakdown, 3 stalled, kFailed
+	int32_t stall, checking, updates, checks;
+};
+
+__device__ __forceinline__ dbl2 ld2(const double* p) {
+	return *reinterpret_cast<const dbl2*>(p);
+}
+__device__ __forceinline__ void st2(double* p, dbl2 v) {
+	*reinterpret_cast<dbl2*>(p) = v;
+}
+__device__ __forceinline__ void put(u64* p, u64 v) {
+	__hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ u64 get(const u64* p) {
+	return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ u64 word_hi(double v, uint32_t ep) {
+	return (static_cast<u64>(__double_as_longlong(v)) & 0xffffffff00000000ull) | ep;
+}
+__device__ __forceinline__ u64 word_lo(double v, uint32_t ep) {
+	return (static_cast<u64>(__double_as_longlong(v)) << 32) | ep;
+}
+__device__ __forceinline__ double join(u64 hi, u64 lo) {
+	return __longlong_as_double(static_cast<long long>((hi & 0xffffffff00000000ull) | (lo >> 32)));
+}
+
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v) {
+	int const lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+	int const hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+	return __hiloint2double(hi, lo);
+}
+
+// Sum over each row of 16 lanes, in all of them (register moves between
+// lanes: a shuffle through LDS takes several times as long).
+__device__ __forceinline__ double row_sum(double v) {
+	v += dpp<0xB1>(v);    // lanes 1 0 3 2
+	v += dpp<0x4E>(v);    // lanes 2 3 0 1
+	v += dpp<0x141>(v);   // the other four of each eight
+	v += dpp<0x140>(v);   // the other eight of each sixteen
+	return v;
+}
+
+__device__ __forceinline__ double lane_value(double v, int lane) {
+	return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+	                        __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// Sum over the wavefront, in all lanes.
+__device__ __forceinline__ double wave_total(double v) {
+	v = row_sum(v);
+	return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
+}
+
+// A value that is the same in all lanes, held in scalar registers.
+__device__ __forceinline__ double uniform(double v) {
+	return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+	                        __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
+template <typename MT>
+__device__ __forceinline__ const MT* matrix(View const& V) {
+	if constexpr (sizeof(MT) == 4) {
+		return V.val32;
+	} else {
+		return V.val;
+	}
+}
+
+struct Shared {
+	double part[3][3][16];   // per kind of all-gather: the waves' partial sums
+	double tot[3][3][4];     // the gathered sums of up to four polling waves
+	int lo, hi;
+	int failed;
+};
+
+// Blocks of a row held in registers, by threads of the workgroup: six FP64
+// blocks (48 registers) fit beside the vectors in the 128 registers a thread
+// of 1024 has (with seven the compiler spills); the others go to LDS.
+template <typename MT, int W, int NT>
+constexpr int register_blocks() {
+	return sizeof(MT) == 8 && NT > 512 && W > 6 ? 6 : W;
+}
+template <typename MT, int W, int NT>
+constexpr int spare_bytes() {
+	return (W - register_blocks<MT, W, NT>()) * 4 * static_cast<int>(sizeof(MT)) * NT;
+}
+
+// One cluster's run, called by all NT threads of its workgroup g of G. On
+// return R holds the run's scalars (in every thread) and V.x the solution of
+// the workgroup's rows. win: LDS for the window's directions. mode 0 starts
+// from x = 0, 1 from the x in V.x, 2 continues a run cut at its limit (R as it
+// was left, r and p in V.save). Runs until R.iter >= stop.
+template <typename MT, int W, int PRE, int NT>
+__device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, double delta2, int64_t stop,
+                        bool final_check, Shared& sh, dbl2* lds, Run& R) {
+	constexpr int NW = NT / 64;
+	constexpr int kAhead = 1;
+	constexpr int WR = register_blocks<MT, W, NT>();
+	// the row's last W - WR blocks, two 16-byte halves each, then the window
+	typedef MT mt2 __attribute__((ext_vector_type(2)));
+	mt2* const spare = reinterpret_cast<mt2*>(lds);
+	dbl2* const win = lds + spare_bytes<MT, W, NT>() / sizeof(dbl2);
+	int t = threadIdx.x;
+	int const lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+	int const n = static_cast<int>(V.n);
+	int const rows = ((n + G - 1) / G + 63) / 64 * 64;   // per workgroup (at most NT)
+	int const r0 = min(g * rows, n), r1 = min(r0 + rows, n);
+	int row = r0 + t;
+	bool const live = row < r1;
+	if (t == 0) {
+		sh.lo = r0;
+		sh.hi = r1;
+		sh.failed = 0;
+	}
+	__syncthreads();
+	// the row's blocks into registers, columns as offsets into the window
+	MT m[WR][4];
+	uint32_t at[(W + 1) / 2];
+	int cols[W];
+	dbl2 dinv0 = {0, 0}, dinv1 = {0, 0};
+	int clo = r0, chi = r0;
+#pragma unroll
+	for (int k = 0; k < W; k++) {
+		cols[k] = r0;
+	}
+	int const s = row >> 6, r64 = row & 63;
+	int beg = 0, len = 0;
+	if (live) {
+		beg = V.slice_ptr[s] + r64;
+		len = (V.slice_ptr[s + 1] - beg + 63) >> 6;
+		clo = chi = row;
+	}
+#pragma unroll
+	for (int k = 0; k < W; k++) {
+		mt2 a = {0, 0}, c = {0, 0};
+		if (live) {
+			cols[k] = row;
+			if (k < len) {
+				int64_t const blk = beg + k * kSlice;
+				int64_t const o = 4 * blk - 2 * r64;
+				const MT* const from = matrix<MT>(V) + o;
+				cols[k] = V.col[blk];
+				a = *reinterpret_cast<const mt2*>(from);
+				c = *reinterpret_cast<const mt2*>(from + 2 * kSlice);
+				clo = min(clo, cols[k]);
+				chi = max(chi, cols[k]);
+			}
+		}
+		if (k < WR) {
+			m[k < WR ? k : 0][0] = a.x;
+			m[k < WR ? k : 0][1] = a.y;
+			m[k < WR ? k : 0][2] = c.x;
+			m[k < WR ? k : 0][3] = c.y;
+		} else {
+			spare[(2 * (k - WR)) * NT + t] = a;
+			spare[(2 * (k - WR) + 1) * NT + t] = c;
+		}
+	}
+	if (live) {
+		const double* top = V.val + 4 * static_cast<int64_t>(V.diag_blk[row]) - 2 * r64;
+		double const a00 = top[0], a01 = top[1], a10 = top[2 * kSlice], a11 = top[2 * kSlice + 1];
+		if (PRE == BFMX_PRECOND_JACOBI) {
+			dinv0 = dbl2{1.0 / a00, 1.0 / a11};
+		} else {
+			double const det = a00 * a11 - a01 * a10;
+			dinv0 = dbl2{a11 / det, -a01 / det};
+			dinv1 = dbl2{-a10 / det, a00 / det};
+		}
+		atomicMin(&sh.lo, clo);
+		atomicMax(&sh.hi, chi + 1);
+	}
+	__syncthreads();
+	int const lo = __builtin_amdgcn_readfirstlane(sh.lo), nwin = __builtin_amdgcn_readfirstlane(sh.hi) - lo, left = r0 - lo, own = r1 - r0, halo = nwin - own;
+#pragma unroll
+	for (int k = 0; k < W; k += 2) {
+		uint32_t const a = static_cast<uint32_t>(cols[k] - lo);
+		uint32_t const c = k + 1 < W ? static_cast<uint32_t>(cols[k + 1 < W ? k + 1 : k] - lo) : 0;
+		at[k / 2] = a | (c << 16);
+	}
+	auto precond = [&](dbl2 r) {
+		if (PRE == BFMX_PRECOND_JACOBI) {
+			return dbl2{dinv0.x * r.x, dinv0.y * r.y};
+		}
+		return dbl2{dinv0.x * r.x + dinv0.y * r.y, dinv1.x * r.x + dinv1.y * r.y};
+	};
+
+	uint32_t ep = 0;   // exchanges of a vector so far
+	uint32_t sep = 0;  // all-gathers so far
+	// word k (0 .. 3) of node i in the current exchange (byte offsets below
+	// 2^32: a uniform base and one 32-bit register)
+	auto word_at = [&](int k, int i) {
+		u64* const base = (ep & 1 ? V.w[2 + k / 2] : V.w[k / 2]) + (k & 1 ? n : 0);
+		return reinterpret_cast<u64*>(reinterpret_cast<char*>(base) + static_cast<uint32_t>(i) * 8u);
+	};
+	auto publish = [&](dbl2 v) {
+		ep++;
+		if (G > 1 && live) {
+			put(word_at(0, row), word_hi(v.x, ep));
+			put(word_at(1, row), word_lo(v.x, ep));
+			put(word_at(2, row), word_hi(v.y, ep));
+			put(word_at(3, row), word_lo(v.y, ep));
+		}
+	};
+	// the last published vector at node i
+	auto receive = [&](int i) {
+		u64 q0, q1, q2, q3;
+		uint32_t spin = 0;
+#pragma unroll 1
+		while (true) {
+			q0 = get(word_at(0, i));
+			q1 = get(word_at(1, i));
+			q2 = get(word_at(2, i));
+			q3 = get(word_at(3, i));
+			if (static_cast<uint32_t>(q0) == ep && static_cast<uint32_t>(q1) == ep &&
+			    static_cast<uint32_t>(q2) == ep && static_cast<uint32_t>(q3) == ep) {
+				break;
+			}
+			if (++spin >= kSpinLimit) {
+				sh.failed = 1;
+				break;
+			}
+		}
+		return dbl2{join(q0, q1), join(q2, q3)};
+	};
+	// halo node k (of the window without the own rows) and its place
+	auto halo_at = [&](int k) { return k < left ? k : k + own; };
+
+	// Sums v over the cluster (the same value everywhere); meanwhile `work`
+	// runs between the posting of the contribution and the wait for the
+	// others'. set: the LDS arrays used (callers alternate, so that no array is
+	// written while a wave may still read it). NV <= 3.
+	auto gather = [&](auto& v, int set, auto&& work) {
+		constexpr int NV = sizeof(v) / sizeof(double);
+#pragma unroll
+		for (int k = 0; k < NV; k++) {
+			double const s = wave_total(v[k]);
+			if (lane == 0) {
+				sh.part[set][k][wave] = s;
+			}
+		}
+		__syncthreads();
+		auto total = [&](int k) { return row_sum((lane & 15) < NW ? sh.part[set][k][lane & 15] : 0.0); };
+		if (G == 1) {
+#pragma unroll
+			for (int k = 0; k < NV; k++) {
+				v[k] = uniform(total(k));
+			}
+			work();
+			return;
+		}
+		sep++;
+		u64* const base = V.slots + static_cast<int64_t>(sep & 1) * G * kSlotWords;
+		if (wave == 0) {
+			double s[NV];
+#pragma unroll
+			for (int k = 0; k < NV; k++) {
+				s[k] = total(k);
+			}
+#pragma unroll
+			for (int k = 0; k < NV; k++) {
+				if (lane == 2 * k) {
+					put(base + g * kSlotWords + lane, word_hi(s[k], sep));
+				}
+				if (lane == 2 * k + 1) {
+					put(base + g * kSlotWords + lane, word_lo(s[k], sep));
+				}
+			}
+		}
+		work();
+		if (wave < (G + 63) / 64) {
+			u64 q[2 * NV];
+#pragma unroll
+			for (int k = 0; k < 2 * NV; k++) {
+				q[k] = 0;
+			}
+			if (t < G) {
+				const u64* const from = base + t * kSlotWords;
+				uint32_t spin = 0;
+#pragma unroll 1
+				while (true) {
+					bool ok = true;
+#pragma unroll
+					for (int k = 0; k < 2 * NV; k++) {
+						q[k] = get(from + k);
+					}
+#pragma unroll
+					for (int k = 0; k < 2 * NV; k++) {
+						ok = ok && static_cast<uint32_t>(q[k]) == sep;
+					}
+					if (ok) {
+						break;
+					}
+					if (++spin >= kSpinLimit) {
+						sh.failed = 1;
+						break;
+					}
+				}
+			}
+#pragma unroll
+			for (int k = 0; k < NV; k++) {
+				double const s = wave_total(join(q[2 * k], q[2 * k + 1]));
+				if (lane == 0) {
+					sh.tot[set][k][wave] = s;
+				}
+			}
+		}
+		__syncthreads();
+#pragma unroll
+		for (int k = 0; k < NV; k++) {
+			double s = sh.tot[set][k][0];
+			for (int w = 1; w < (G + 63) / 64; w++) {
+				s += sh.tot[set][k][w];
+			}
+			v[k] = uniform(s);
+		}
+	};
+	auto nothing = [] {};
+	auto failed = [&] { return __builtin_amdgcn_readfirstlane(sh.failed) != 0; };
+
+	// b - A x of the own row with the FP64 matrix, compensated (row_residual in
+	// pcg.hip); x is published for it
+	dbl2 x = {0, 0}, r = {0, 0}, z = {0, 0}, pn = {0, 0};
+	auto true_residual = [&]() {
+		publish(x);
+		dbl2 res = {0, 0};
+		if (G == 1) {
+			// through the window's LDS: its directions are kept in registers
+			__syncthreads();
+			if (live) {
+				win[row - lo] = x;
+			}
+			__syncthreads();
+		}
+		if (live) {
+			dbl2 const bv = ld2(V.b + 2 * static_cast<int64_t>(row));
+			int const end = beg + len * kSlice;
+			double s0 = bv.x, s1 = bv.y, c0 = 0, c1 = 0;
+#pragma unroll 1
+			for (int blk = beg; blk < end; blk += kSlice) {
+				int const c = V.col[blk];
+				int64_t const o = 4 * static_cast<int64_t>(blk) - 2 * r64;
+				dbl2 const a = ld2(V.val + o), d = ld2(V.val + o + 2 * kSlice);
+				dbl2 const xv = G == 1 ? win[c - lo] : c == row ? x : receive(c);
+				sub_exact(s0, c0, a.x, xv.x);
+				sub_exact(s0, c0, a.y, xv.y);
+				sub_exact(s1, c1, d.x, xv.x);
+				sub_exact(s1, c1, d.y, xv.y);
+			}
+			res = dbl2{s0 + c0, s1 + c1};
+		}
+		if (G == 1) {
+			__syncthreads();
+			if (live) {
+				win[row - lo] = pn;
+			}
+		}
+		return res;
+	};
+
+	double beta = 0;
+	int status = 0;
+	for (int k = t; k < nwin; k += NT) {
+		win[k] = mode == 2 ? ld2(V.save + 2 * (static_cast<int64_t>(n) + lo + k)) : dbl2{0, 0};
+	}
+	if (mode == 2) {
+		if (live) {
+			x = ld2(V.x + 2 * static_cast<int64_t>(row));
+			r = ld2(V.save + 2 * static_cast<int64_t>(row));
+			z = precond(r);
+		}
+		beta = R.beta;
+		__syncthreads();
+	} else {
+		__syncthreads();
+		if (live) {
+			if (mode == 1) {
+				x = ld2(V.x + 2 * static_cast<int64_t>(row));
+			} else {
+				r = ld2(V.b + 2 * static_cast<int64_t>(row));
+			}
+		}
+		if (mode == 1) {
+			r = true_residual();
+		}
+		z = precond(r);
+		dbl2 const bv = live ? ld2(V.b + 2 * static_cast<int64_t>(row)) : dbl2{0, 0};
+		double v[3] = {r.x * z.x + r.y * z.y, r.x * r.x + r.y * r.y, bv.x * bv.x + bv.y * bv.y};
+		gather(v, 2, nothing);
+		R.rz = v[0];
+		R.rr = R.rr_true = R.rr_ref = v[1];
+		R.bb = v[2];
+		R.tol2 = uniform(rtol2 * v[2]);
+		R.rr_best = R.pq = 0;
+		R.iter = 0;
+		R.stall = R.checking = R.checks = 0;
+		R.updates = 1;
+		status = failed() ? kFailed : R.rr <= R.tol2 ? 1 : 0;
+	}
+	if (status == 0 && R.iter < stop) {
+		publish(z);
+	}
+	dbl2 hz[kAhead];   // z of this thread's first halo nodes
+	auto halo_first = [&] {
+#pragma unroll
+		for (int u = 0; u < kAhead; u++) {
+			int const k = t + u * NT;
+			if (k < halo) {
+				hz[u] = receive(lo + halo_at(k));
+			}
+		}
+	};
+	if (status == 0 && R.iter < stop) {
+		halo_first();
+	}
+	while (status == 0 && R.iter < stop) {
+		// addresses are formed anew in every iteration: held in registers they
+		// would push the matrix out
+		asm volatile("" : "+v"(t), "+v"(row));
+		// p = z + beta p over the window
+		if (live) {
+			pn = z + beta * win[row - lo];
+			win[row - lo] = pn;
+		}
+#pragma unroll
+		for (int u = 0; u < kAhead; u++) {
+			int const k = t + u * NT;
+			if (k < halo) {
+				int const a = halo_at(k);
+				win[a] = hz[u] + beta * win[a];
+			}
+		}
+		for (int k = t + kAhead * NT; k < halo; k += NT) {
+			int const a = halo_at(k);
+			win[a] = receive(lo + a) + beta * win[a];
+		}
+		__syncthreads();
+		// q = A p
+		dbl2 q = {0, 0};
+#pragma unroll
+		for (int k = 0; k < (W + 1) / 2; k++) {
+			asm volatile("" : "+v"(at[k]));   // unpacked in every iteration, not held unpacked
+		}
+#pragma unroll
+		for (int k = 0; k < W; k++) {
+			dbl2 const pv = win[(at[k / 2] >> (16 * (k & 1))) & 0xffffu];
+			mt2 a, c;
+			if (k < WR) {
+				int const kr = k < WR ? k : 0;
+				if constexpr (sizeof(MT) == 4) {
+					// converted in every iteration: kept as FP64 they would not fit
+					asm volatile("" : "+v"(m[kr][0]), "+v"(m[kr][1]), "+v"(m[kr][2]), "+v"(m[kr][3]));
+				}
+				a = mt2{m[kr][0], m[kr][1]};
+				c = mt2{m[kr][2], m[kr][3]};
+			} else {
+				a = spare[(2 * (k - WR)) * NT + t];
+				c = spare[(2 * (k - WR) + 1) * NT + t];
+			}
+			q.x += static_cast<double>(a.x) * pv.x + static_cast<double>(a.y) * pv.y;
+			q.y += static_cast<double>(c.x) * pv.x + static_cast<double>(c.y) * pv.y;
+		}
+		double v1[1] = {pn.x * q.x + pn.y * q.y};
+		gather(v1, 0, nothing);
+		R.pq = v1[0];
+		if (failed()) {
+			status = kFailed;
+			break;
+		}
+		if (!(v1[0] > 0) || !isfinite(v1[0])) {
+			status = 2;
+			break;
+		}
+		double const alpha = uniform(R.rz / v1[0]);
+		x += alpha * pn;
+		r -= alpha * q;
+		z = precond(r);
+		publish(z);
+		double v2[2] = {r.x * z.x + r.y * z.y, r.x * r.x + r.y * r.y};
+		gather(v2, 1, halo_first);
+		if (failed()) {
+			status = kFailed;
+			break;
+		}
+		R.iter++;
+		double const rz_prev = R.rz;
+		beta = uniform(v2[0] / rz_prev);
+		R.rz = v2[0];
+		R.rr = v2[1];
+		bool const at_tol = R.rr <= R.tol2;
+		bool const every = R.iter % kCheckEvery == 0;
+		if ((at_tol && !R.checking) || (every && (R.checking || R.rr <= delta2 * R.rr_ref))) {
+			// the true residual replaces the recursive one (the directions are
+			// kept) and decides about the end
+			r = true_residual();
+			z = precond(r);
+			double v3[2] = {r.x * z.x + r.y * z.y, r.x * r.x + r.y * r.y};
+			gather(v3, 2, nothing);
+			if (failed()) {
+				status = kFailed;
+				break;
+			}
+			beta = rz_prev != 0 ? uniform(v3[0] / rz_prev) : 0.0;
+			R.rz = v3[0];
+			R.rr = R.rr_true = R.rr_ref = v3[1];
+			R.updates++;
+			R.checks++;
+			if (R.rr <= R.tol2) {
+				status = 1;
+			} else {
+				if (at_tol || R.checking) {
+					R.checking = 1;
+					if (R.rr_best == 0 || R.rr < 0.25 * R.rr_best) {
+						R.rr_best = R.rr;
+						R.stall = 0;
+					} else if (++R.stall >= kStall) {
+						status = 3;
+					}
+				}
+				if (status == 0) {
+					publish(z);
+					halo_first();
+				}
+			}
+		}
+	}
+	R.beta = beta;
+	if (status == 0 && final_check && R.checks == 0) {
+		dbl2 const rt = true_residual();
+		double v[1] = {rt.x * rt.x + rt.y * rt.y};
+		gather(v, 2, nothing);
+		R.rr_true = v[0];
+		if (failed()) {
+			status = kFailed;
+		}
+	}
+	R.status = status;
+	if (live) {
+		st2(V.x + 2 * static_cast<int64_t>(row), x);
+		if (status == 0) {
+			st2(V.save + 2 * static_cast<int64_t>(row), r);
+			st2(V.save + 2 * (static_cast<int64_t>(n) + row), pn);
+		}
+	}
+}
+
+// True when the system's rows and windows fit the clusters above; then *groups
+// workgroups of at most kRows rows and *window nodes at most.
+bool fits(const bfmx_system* s, int* groups, int* window);
+
+}  // namespace resident
+}  // namespace bfmx

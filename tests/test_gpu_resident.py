@@ -1,0 +1,144 @@
+"""Jacobi PCG with the matrix in registers (bfm_amd/csrc/hip/resident.hip)
+against the streaming kernels (BFMX_RESIDENT=0), at the edges of its
+workgroups and of what it takes. Both runs meet the same true residual rtol,
+which bounds each solution's error in the A-norm; the displacements are
+compared to 1e-6, a hundred times what was seen, and the residual of the
+register-resident solution is formed again from the matrix."""
+
+import threading
+
+import numpy as np
+import pytest
+
+from conftest import rel_err
+
+from bfm_amd import device as D
+from bfm_amd import meshgen
+
+pytestmark = pytest.mark.gpu
+
+RTOL = 1e-9
+
+
+def strip(n, kind, het, seed=5):
+    """A beam of exactly n nodes: a grid h nodes high, cut off along its last column."""
+    h = 4 if n < 256 else 16 if n < 1000 else 32
+    nx = -(-n // h)
+    m = meshgen.beam(nx, h - 1, kind=kind, length=nx / h, height=1.0, jitter=0.2, seed=seed)
+    # nodes column by column, so that the first n of them are a prefix of the grid
+    j, i = np.divmod(np.arange(m.n_nodes), nx + 1)
+    order = np.argsort(i * h + j, kind="stable")
+    new = np.empty_like(order)
+    new[order] = np.arange(order.size)
+    elems = new[m.elems.astype(np.int64)]
+    elems = elems[(elems < n).all(axis=1)]
+    edges = new[m.edges.astype(np.int64)]
+    edges = edges[(edges < n).all(axis=1)]
+    used = np.zeros(n, bool)
+    used[elems.ravel()] = True
+    assert used.all()
+    sets = {k: v[order][:n] for k, v in m.node_sets.items()}
+    out = meshgen.Mesh(kind, m.coords[order][:n].copy(), elems.astype(np.uint64), edges.astype(np.uint64),
+                       -np.ones(len(edges), np.int64), sets)
+    if het:
+        out.elem_E = meshgen.loguniform_E(out.n_elems, seed=seed)
+    return out
+
+
+def both(monkeypatch, s, **kw):
+    monkeypatch.setenv("BFMX_RESIDENT", "0")
+    ref, st_ref = s.solve(**kw)
+    monkeypatch.delenv("BFMX_RESIDENT")
+    u, st = s.solve(**kw)
+    return ref, st_ref, u, st
+
+
+def check(s, u, ref, st, rtol):
+    assert st["status"] == 0 and st["rel_residual"] <= rtol
+    A, b = s.get_csr_scipy(), s.get_rhs()
+    assert np.linalg.norm(b - A @ u) <= 1.1 * rtol * np.linalg.norm(b)
+    assert rel_err(u, ref) <= 1e-6
+
+
+# one workgroup of 512 and of 1024 threads, then clusters: full, one row over, an uneven last one
+@pytest.mark.parametrize("n", [8, 64, 511, 512, 514, 1022, 1024, 1026, 2048, 2050, 3200])
+@pytest.mark.parametrize("kind,pre,precision", [(4, D.PRECOND_JACOBI, D.FP64), (3, D.PRECOND_BLOCK_JACOBI, D.FP64),
+                                                (4, D.PRECOND_BLOCK_JACOBI, D.MIXED)])
+def test_workgroup_edges(monkeypatch, n, kind, pre, precision):
+    if precision == D.MIXED and n < 512:
+        pytest.skip("the FP32 operator stalls above rtol on the smallest strips, on either path")
+    m = strip(n + n % 2, kind, het=pre == D.PRECOND_BLOCK_JACOBI and precision == D.FP64)
+    s = D.beam_system(m)
+    rtol = 1e-8 if precision == D.MIXED else RTOL
+    ref, st_ref, u, st = both(monkeypatch, s, precond=pre, precision=precision, rtol=rtol)
+    print(f"{m.n_nodes} nodes: {st_ref['iterations']} / {st['iterations']} iterations, difference {rel_err(u, ref):.1e}")
+    check(s, u, ref, st, rtol)
+    again, st2 = s.solve(precond=pre, precision=precision, rtol=rtol)
+    assert np.array_equal(u, again) and st2["iterations"] == st["iterations"]
+
+
+@pytest.mark.parametrize("nx,ny,precision", [(24, 6, D.FP64), (80, 20, D.FP64), (80, 20, D.MIXED)])
+def test_a_run_cut_into_launches_is_the_same_run(monkeypatch, nx, ny, precision):
+    s = D.beam_system(meshgen.beam(nx, ny, kind=4, jitter=0.2, seed=3))
+    u, st = s.solve(precision=precision, rtol=1e-8)
+    monkeypatch.setenv("BFMX_RESIDENT_ITERS", "48")
+    u2, st2 = s.solve(precision=precision, rtol=1e-8)
+    assert st["iterations"] > 96 and st2["iterations"] == st["iterations"] and np.array_equal(u, u2)
+
+
+def test_what_does_not_fit_takes_the_streaming_kernels(monkeypatch):
+    # a fan: the middle node's row has 13 blocks, more than the registers hold
+    k = 12
+    a = 2 * np.pi * np.arange(k) / k
+    coords = np.concatenate([[[0.0, 0.0]], np.stack([np.cos(a), np.sin(a)], 1)])
+    elems = np.array([[0, 1 + i, 1 + (i + 1) % k] for i in range(k)], np.uint64)
+    s = D.System(3, coords, elems)
+    s.assemble(1, 2e11, 0.3, 7850.0, g=(0.0, -9.81))
+    fix = np.zeros(k + 1, np.uint8)
+    fix[1:4] = 1
+    s.apply_conditions([0, 1], [0.0, 0.0], [fix, fix])
+    ref, _, u, st = both(monkeypatch, s, rtol=RTOL)
+    assert np.array_equal(u, ref)
+    # an order of the nodes that reaches over more than a window holds
+    m = meshgen.beam(120, 50, kind=4, jitter=0.2, seed=4)
+    p = np.random.default_rng(1).permutation(m.n_nodes)
+    q = np.empty_like(p)
+    q[p] = np.arange(p.size)
+    m.coords, m.elems, m.edges = m.coords[p], q[m.elems.astype(np.int64)].astype(np.uint64), q[m.edges.astype(np.int64)]
+    m.node_sets = {name: v[p] for name, v in m.node_sets.items()}
+    s = D.beam_system(m, renumber=False)
+    ref, _, u, st = both(monkeypatch, s, rtol=RTOL)
+    assert np.array_equal(u, ref)
+    s = D.beam_system(m)                    # renumbered, it fits
+    ref, _, u, st = both(monkeypatch, s, rtol=RTOL)
+    check(s, u, ref, st, RTOL)
+
+
+def test_zero_load_limit_and_floor():
+    s = D.beam_system(meshgen.beam(80, 20, kind=4, jitter=0.2, seed=3))
+    u, st = s.solve(b=np.zeros(2 * s.n_nodes))
+    assert st["iterations"] == 0 and np.array_equal(u, np.zeros_like(u))
+    with pytest.raises(D.BfmxError) as e:
+        s.solve(max_iter=20)
+    assert e.value.code == -5 and "32 iterations" in str(e.value)   # whole rounds of 16
+    with pytest.raises(D.BfmxError) as e:
+        s.solve(rtol=1e-17)
+    assert e.value.code == -8
+
+
+def test_clusters_on_several_threads():
+    """More workgroups than the GPU holds at once, from several threads: each system's run is its own."""
+    systems = [D.beam_system(meshgen.beam(400 + 10 * k, 180, kind=4, jitter=0.2, seed=k)) for k in range(4)]
+    alone = [s.solve(rtol=1e-6)[0] for s in systems]
+    got = [None] * len(systems)
+
+    def work(k):
+        for _ in range(2):
+            got[k] = systems[k].solve(rtol=1e-6)[0]
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(systems))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(np.array_equal(a, g) for a, g in zip(alone, got))

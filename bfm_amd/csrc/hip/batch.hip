@@ -1,8 +1,13 @@
-// Batched solves: many independent planar systems of uneven sizes solved by
-// one persistent kernel launch per size class, the launches captured in one
-// HIP graph.
+// Batched solves: many independent planar systems of uneven sizes.
 //
-// One workgroup runs the whole Jacobi or block-Jacobi PCG of one system: its
+// Systems whose matrix fits the registers of a cluster of workgroups (rows of
+// at most nine blocks, up to 262,144 nodes) are solved by resident.hip: all
+// clusters in one launch, each taking one system after another. The others,
+// and all of them where the device refuses that launch, are solved by the
+// streaming kernel below, one persistent launch per size class (captured in
+// one HIP graph when it solves the whole batch).
+//
+// In the streaming kernel one workgroup runs the whole Jacobi or block-Jacobi PCG of one system: its
 // passes over the rows (SpMV with the direction update folded into the
 // gathers, the vector updates, the residual recomputation) are separated by
 // workgroup barriers, and its dot products are workgroup reductions in a
@@ -27,6 +32,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <cstdlib>
 #include <numeric>
 
 #include <atomic>
@@ -35,6 +41,7 @@
 #include <thread>
 
 #include "assemble_dev.h"
+#include "resident.h"
 
 namespace bfmx {
 
@@ -89,13 +96,7 @@ struct BatchInst {
 	double* vfirst;
 };
 
-struct BatchOut {
-	int64_t iter;
-	double rr_true;
-	double bb;
-	int32_t status;   // 1 converged, 2 breakdown, 3 stagnated, 0 iteration limit
-	int32_t checks;
-};
+using BatchOut = resident::Out;
 
 // Configurations: workgroup size x rows per thread per step.
 constexpr int kConfigs = 5;
@@ -553,6 +554,12 @@ struct bfmx_batch {
 	};
 	std::vector<Exec> graphs;
 	hipEvent_t ev[2] = {};
+	// clusters with the matrix in registers (resident.h) for the systems that
+	// fit, made at the first solve; the streaming kernel takes the others
+	bool planned = false;
+	bfmx::resident::Plan* plan = nullptr;
+	int32_t* d_rest = nullptr;              // those others, by class, largest first
+	int rest_count[bfmx::kClasses] = {};
 	// batches built from meshes: the systems are the batch's own (host
 	// topology plus device arrays inside the arenas below), assembled by every
 	// solve launch
@@ -630,6 +637,8 @@ void batch_destroy(bfmx_batch* b) {
 		(void) hipStreamSynchronize(b->stream);
 	}
 	union_release(b);
+	resident::plan_destroy(b->plan);
+	dfree(b->d_rest);
 	for (auto& g : b->graphs) {
 		(void) hipGraphExecDestroy(g.exec);
 	}
@@ -1002,29 +1011,76 @@ int batch_solve_amg(bfmx_batch* b, double rtol, int64_t max_iter, bfmx_stats_t* 
 
 }  // namespace
 
-int batch_solve(bfmx_batch* b, int pre, double rtol, int64_t max_iter, const int32_t* picks_in, bfmx_stats_t* stats,
-                double* total_ms) {
-	if (pre == BFMX_PRECOND_AMG) {
-		return batch_solve_amg(b, rtol, max_iter, stats, total_ms);
+namespace {
+
+// The batch's clusters (at its first Jacobi solve): the systems that fit, and
+// the rest by class for the streaming kernel.
+int make_plan(bfmx_batch* b) {
+	if (b->planned) {
+		return BFMX_OK;
 	}
-	if (pre != BFMX_PRECOND_JACOBI && pre != BFMX_PRECOND_BLOCK_JACOBI) {
-		set_error("batched solves use Jacobi or block-Jacobi PCG, or the multigrid mode");
-		return BFMX_E_UNSUPPORTED;
+	std::vector<BatchInst> h(b->systems.size());
+	BFMX_HIP(hipMemcpy(h.data(), b->d_inst, h.size() * sizeof(BatchInst), hipMemcpyDeviceToHost));
+	std::vector<resident::View> views;
+	auto words = [](double* p) { return reinterpret_cast<resident::u64*>(p); };
+	for (auto const& I : h) {
+		views.push_back(resident::View{I.slice_ptr, I.col, I.diag_blk, I.val, nullptr, I.b, I.x,
+		                               {words(I.r), words(I.z), words(I.q), words(I.p0)}, words(I.p1), I.dinv, I.n});
 	}
-	int picks[kClasses];
-	for (int c = 0; c < kClasses; c++) {
-		picks[c] = picks_in ? picks_in[c] : kDefaultPick[c];
-		if (picks[c] < 0 || picks[c] >= kConfigs) {
-			set_error("configuration %d out of range", picks[c]);
-			return BFMX_E_ARG;
+	BFMX_CHECK(resident::plan_create(&b->plan, b->systems, views, b->stream));
+	if (b->plan && !resident::plan_rest(b->plan).empty()) {
+		std::vector<int32_t> rest = resident::plan_rest(b->plan);
+		std::stable_sort(rest.begin(), rest.end(),
+		                 [&](int32_t a, int32_t c) { return size_class(h[a].n) > size_class(h[c].n); });
+		for (int32_t const k : rest) {
+			b->rest_count[size_class(h[k].n)]++;
+		}
+		BFMX_CHECK(dalloc(&b->d_rest, rest.size()));
+		BFMX_HIP(hipMemcpy(b->d_rest, rest.data(), rest.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+	}
+	b->planned = true;
+	return BFMX_OK;
+}
+
+// Assembles the batch and solves it with the clusters, the systems that do not
+// fit with the streaming kernel; *ran is false when the streaming kernel has
+// to take them all.
+int solve_resident(bfmx_batch* b, int pre, double rtol2, int64_t max_iter, const int* picks, bool* ran) {
+	*ran = false;
+	const char* e = std::getenv("BFMX_RESIDENT");
+	if (e && e[0] == '0') {
+		return BFMX_OK;
+	}
+	BFMX_CHECK(make_plan(b));
+	if (!b->plan) {
+		return BFMX_OK;
+	}
+	BFMX_HIP(hipEventRecord(b->ev[0], b->stream));
+	launch_assemble(b);
+	bool launched = false;
+	BFMX_CHECK(resident::plan_launch(b->plan, b->stream, pre, rtol2, max_iter, b->d_out, &launched));
+	if (!launched) {
+		return BFMX_OK;
+	}
+	const int32_t* at = b->d_rest;
+	for (int c = kClasses - 1; c >= 0; c--) {
+		if (b->rest_count[c] > 0) {
+			launch(pre, picks[c], b->rest_count[c], b->stream, b->d_inst, at, rtol2, max_iter, b->d_out);
+			at += b->rest_count[c];
 		}
 	}
-	if (max_iter == 0) {
-		for (auto* s : b->systems) {
-			max_iter = std::max<int64_t>(max_iter, 20 * 2 * s->n_nodes);
-		}
-	}
-	double const rtol2 = rtol * rtol;
+	BFMX_HIP(hipGetLastError());
+	BFMX_HIP(hipEventRecord(b->ev[1], b->stream));
+	BFMX_HIP(hipMemcpyAsync(b->h_out.data(), b->d_out, b->h_out.size() * sizeof(BatchOut), hipMemcpyDeviceToHost,
+	                        b->stream));
+	BFMX_HIP(hipStreamSynchronize(b->stream));
+	*ran = std::none_of(b->h_out.begin(), b->h_out.end(),
+	                    [](BatchOut const& o) { return o.status == resident::kFailed; });
+	return BFMX_OK;
+}
+
+// The whole batch through the streaming kernel, from a captured graph.
+int solve_streaming(bfmx_batch* b, int pre, double rtol2, int64_t max_iter, const int* picks) {
 	hipGraphExec_t exec = nullptr;
 	bool const use_graph = graphs_enabled();
 	for (auto const& g : b->graphs) {
@@ -1061,6 +1117,39 @@ int batch_solve(bfmx_batch* b, int pre, double rtol, int64_t max_iter, const int
 	BFMX_HIP(hipMemcpyAsync(b->h_out.data(), b->d_out, b->h_out.size() * sizeof(BatchOut), hipMemcpyDeviceToHost,
 	                        b->stream));
 	BFMX_HIP(hipStreamSynchronize(b->stream));
+	return BFMX_OK;
+}
+
+}  // namespace
+
+int batch_solve(bfmx_batch* b, int pre, double rtol, int64_t max_iter, const int32_t* picks_in, bfmx_stats_t* stats,
+                double* total_ms) {
+	if (pre == BFMX_PRECOND_AMG) {
+		return batch_solve_amg(b, rtol, max_iter, stats, total_ms);
+	}
+	if (pre != BFMX_PRECOND_JACOBI && pre != BFMX_PRECOND_BLOCK_JACOBI) {
+		set_error("batched solves use Jacobi or block-Jacobi PCG, or the multigrid mode");
+		return BFMX_E_UNSUPPORTED;
+	}
+	int picks[kClasses];
+	for (int c = 0; c < kClasses; c++) {
+		picks[c] = picks_in ? picks_in[c] : kDefaultPick[c];
+		if (picks[c] < 0 || picks[c] >= kConfigs) {
+			set_error("configuration %d out of range", picks[c]);
+			return BFMX_E_ARG;
+		}
+	}
+	if (max_iter == 0) {
+		for (auto* s : b->systems) {
+			max_iter = std::max<int64_t>(max_iter, 20 * 2 * s->n_nodes);
+		}
+	}
+	double const rtol2 = rtol * rtol;
+	bool ran = false;
+	BFMX_CHECK(solve_resident(b, pre, rtol2, max_iter, picks, &ran));
+	if (!ran) {
+		BFMX_CHECK(solve_streaming(b, pre, rtol2, max_iter, picks));
+	}
 	mark_assembled(b);
 	float ms = 0;
 	BFMX_HIP(hipEventElapsedTime(&ms, b->ev[0], b->ev[1]));

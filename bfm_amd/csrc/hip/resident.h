@@ -18,11 +18,11 @@
 //     32 data bits and the 32-bit number of the exchange, written and read with
 //     agent-scope relaxed atomics (which pass by the XCDs' incoherent L2s). A
 //     reader polls the word itself until it carries the expected number, so an
-//     exchange costs one store-to-load latency (1.4 us up to 8 workgroups, 3.7
-//     at 256) and needs no fence, no flag and no wait for the stores.
+//     exchange costs one store-to-load latency (1.3 us up to 4 workgroups, 1.8
+//     at 32, 2.7 at 256) and needs no fence, no flag and no wait for the stores.
 // Measured on one MI355X, microseconds an iteration, streaming -> here: 451 nodes
-// (one workgroup) 13.8 -> 1.7; 1,105 (two) 13.3 -> 4.4; 5,124 (six) 13.3 -> 4.8;
-// 22,952 (23) 13.4 -> 4.8; 63,126 (62) 16.4 -> 5.3; 251,251 (246) 32.7 -> 10.0,
+// (one workgroup) 13.8 -> 1.7; 1,105 (two) 13.4 -> 4.3; 5,124 (six) 13.3 -> 4.6;
+// 22,952 (23) 13.4 -> 4.7; 63,126 (62) 16.2 -> 5.0; 251,251 (246) 32.7 -> 10.0,
 // point Jacobi on Q1 beams (22,952: block Jacobi, FP32 matrix, P1). Above one
 // workgroup the two all-gathers bound it.
 // A word is overwritten two exchanges later at the earliest, after an
@@ -65,7 +65,8 @@ typedef float flt2 __attribute__((ext_vector_type(2)));
 typedef unsigned long long u64;
 
 constexpr uint32_t kSpinLimit = 1u << 22;   // polls of one wait (seconds)
-constexpr int kSlotWords = 8;               // words of one workgroup's contribution to an all-gather
+constexpr int kSlotWords = 16;              // a 128-byte line for each workgroup's contribution to an all-gather
+                                            // (several in a line cost 0.4 us more at 32 workgroups)
 constexpr int kMaxGroup = 256;              // workgroups of a cluster
 constexpr int kMaxWindow = 3900;            // nodes of a window (62 KB of the CU's 160 KB of LDS, beside 96 KB of row blocks)
 constexpr int kMaxWidth = 9;                // blocks of a row held in registers
@@ -166,7 +167,8 @@ __device__ __forceinline__ const MT* matrix(View const& V) {
 struct Shared {
 	double part[3][3][16];   // per kind of all-gather: the waves' partial sums
 	double tot[3][3][4];     // the gathered sums of up to four polling waves
-	int lo, hi;
+	int lo, hi;          // the window
+	int below, above;    // own rows before below or from above on lie in another workgroup's window
 	int failed;
 };
 
@@ -207,6 +209,8 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 	if (t == 0) {
 		sh.lo = r0;
 		sh.hi = r1;
+		sh.below = 0;
+		sh.above = n;
 		sh.failed = 0;
 	}
 	__syncthreads();
@@ -283,6 +287,38 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 
 	uint32_t ep = 0;   // exchanges of a vector so far
 	uint32_t sep = 0;  // all-gathers so far
+	// the rows that other workgroups read: the first all-gather is of the windows
+	bool shared = false;
+	if (G > 1) {
+		sep = 1;
+		u64* const base = V.slots + static_cast<int64_t>(G) * kSlotWords;
+		if (t < 2) {
+			put(base + g * kSlotWords + t, (static_cast<u64>(t == 0 ? lo : lo + nwin) << 32) | sep);
+		}
+		if (t < G && t != g) {
+			u64 a, c;
+			uint32_t spin = 0;
+#pragma unroll 1
+			while (true) {
+				a = get(base + t * kSlotWords);
+				c = get(base + t * kSlotWords + 1);
+				if (static_cast<uint32_t>(a) == sep && static_cast<uint32_t>(c) == sep) {
+					break;
+				}
+				if (++spin >= kSpinLimit) {
+					sh.failed = 1;
+					break;
+				}
+			}
+			if (t < g) {
+				atomicMax(&sh.below, static_cast<int>(c >> 32));
+			} else {
+				atomicMin(&sh.above, static_cast<int>(a >> 32));
+			}
+		}
+		__syncthreads();
+		shared = live && (row < sh.below || row >= sh.above);
+	}
 	// word k (0 .. 3) of node i in the current exchange (byte offsets below
 	// 2^32: a uniform base and one 32-bit register)
 	auto word_at = [&](int k, int i) {
@@ -291,7 +327,7 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 	};
 	auto publish = [&](dbl2 v) {
 		ep++;
-		if (G > 1 && live) {
+		if (shared) {
 			put(word_at(0, row), word_hi(v.x, ep));
 			put(word_at(1, row), word_lo(v.x, ep));
 			put(word_at(2, row), word_hi(v.y, ep));
@@ -420,14 +456,12 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 	auto true_residual = [&]() {
 		publish(x);
 		dbl2 res = {0, 0};
-		if (G == 1) {
-			// through the window's LDS: its directions are kept in registers
-			__syncthreads();
-			if (live) {
-				win[row - lo] = x;
-			}
-			__syncthreads();
+		// the own rows' x through the window, whose directions stay in registers
+		__syncthreads();
+		if (live) {
+			win[row - lo] = x;
 		}
+		__syncthreads();
 		if (live) {
 			dbl2 const bv = ld2(V.b + 2 * static_cast<int64_t>(row));
 			int const end = beg + len * kSlice;
@@ -437,7 +471,7 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 				int const c = V.col[blk];
 				int64_t const o = 4 * static_cast<int64_t>(blk) - 2 * r64;
 				dbl2 const a = ld2(V.val + o), d = ld2(V.val + o + 2 * kSlice);
-				dbl2 const xv = G == 1 ? win[c - lo] : c == row ? x : receive(c);
+				dbl2 const xv = c >= r0 && c < r1 ? win[c - lo] : receive(c);
 				sub_exact(s0, c0, a.x, xv.x);
 				sub_exact(s0, c0, a.y, xv.y);
 				sub_exact(s1, c1, d.x, xv.x);
@@ -445,11 +479,9 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 			}
 			res = dbl2{s0 + c0, s1 + c1};
 		}
-		if (G == 1) {
-			__syncthreads();
-			if (live) {
-				win[row - lo] = pn;
-			}
+		__syncthreads();
+		if (live) {
+			win[row - lo] = pn;
 		}
 		return res;
 	};
@@ -532,7 +564,7 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 		}
 		__syncthreads();
 		// q = A p
-		dbl2 q = {0, 0};
+		dbl2 q = {0, 0}, qodd = {0, 0};
 #pragma unroll
 		for (int k = 0; k < (W + 1) / 2; k++) {
 			asm volatile("" : "+v"(at[k]));   // unpacked in every iteration, not held unpacked
@@ -553,9 +585,13 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 				a = spare[(2 * (k - WR)) * NT + t];
 				c = spare[(2 * (k - WR) + 1) * NT + t];
 			}
-			q.x += static_cast<double>(a.x) * pv.x + static_cast<double>(a.y) * pv.y;
-			q.y += static_cast<double>(c.x) * pv.x + static_cast<double>(c.y) * pv.y;
+			dbl2& s = k & 1 ? qodd : q;
+			s.x = fma(static_cast<double>(a.x), pv.x, s.x);
+			s.x = fma(static_cast<double>(a.y), pv.y, s.x);
+			s.y = fma(static_cast<double>(c.x), pv.x, s.y);
+			s.y = fma(static_cast<double>(c.y), pv.y, s.y);
 		}
+		q += qodd;
 		double v1[1] = {pn.x * q.x + pn.y * q.y};
 		gather(v1, 0, nothing);
 		R.pq = v1[0];
@@ -640,9 +676,36 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 	}
 }
 
-// True when the system's rows and windows fit the clusters above; then *groups
-// workgroups of at most kRows rows and *window nodes at most.
-bool fits(const bfmx_system* s, int* groups, int* window);
+// Most block rows of a workgroup, one per thread.
+constexpr int kRows = 1024;
+
+// The nodes of the widest window when G workgroups share the system's rows (0:
+// they cannot, or a window or row is too long for the kernels above).
+int window_of(const bfmx_system* s, int64_t G);
+
+// ---- batches (resident.hip)
+
+// What a system's run of a batch reports.
+struct Out {
+	int64_t iter;
+	double rr_true;
+	double bb;
+	int32_t status;   // 1 converged, 2 breakdown, 3 stagnated, 0 iteration limit, kFailed
+	int32_t checks;
+};
+
+struct Plan;
+// The clusters for a batch of systems (views[k]: system k's arrays; they must
+// stay). *out is null when no system fits.
+int plan_create(Plan** out, const std::vector<bfmx_system*>& systems, const std::vector<View>& views,
+                hipStream_t st);
+void plan_destroy(Plan* p);
+// Systems the plan does not take, largest first.
+const std::vector<int32_t>& plan_rest(const Plan* p);
+// Queues the runs of the plan's systems; *launched is false when the device
+// refused (the streaming kernel then takes them all). A system whose status is
+// kFailed afterwards was not solved.
+int plan_launch(Plan* p, hipStream_t st, int precond, double rtol2, int64_t max_iter, Out* d_out, bool* launched);
 
 }  // namespace resident
 }  // namespace bfmx

@@ -2,6 +2,7 @@
 // its launches for one system, and the fall-back to the streaming kernels.
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 
 #include "resident.h"
@@ -12,7 +13,6 @@ using namespace resident;
 
 namespace {
 
-constexpr int kRows = 1024;             // block rows of a workgroup, one per thread
 constexpr int64_t kPerLaunch = 8192;    // iterations of one launch at most (some 0.1 s)
 
 // The exchange words of a launch start at number 0 (the vector words' four
@@ -30,7 +30,7 @@ __global__ __launch_bounds__(kBlock) void k_clear(View V, int64_t nw, int64_t ns
 template <typename MT, int W, int PRE, int NT>
 __global__ __launch_bounds__(NT) void k_resident_pcg(View V, int mode, double rtol2, double delta2, int64_t stop,
                                                      Scalars* __restrict__ S) {
-	extern __shared__ double dyn[];
+	extern __shared__ __align__(16) double dyn[];
 	__shared__ Shared sh;
 	Run R;
 	if (mode == 2) {
@@ -98,14 +98,13 @@ int spare(bool mixed, int width, int nt) {
 
 namespace resident {
 
-bool fits(const bfmx_system* s, int* groups, int* window) {
+int window_of(const bfmx_system* s, int64_t G) {
 	int64_t const n = s->n_nodes;
-	int64_t const G = (n + kRows - 1) / kRows;
-	if (n == 0 || G > kMaxGroup) {
-		return false;
+	if (n == 0 || G > kMaxGroup || (n + G - 1) / G > kRows) {
+		return 0;
 	}
 	if (*std::max_element(s->row_len.begin(), s->row_len.end()) > kMaxWidth) {
-		return false;
+		return 0;
 	}
 	int64_t const rows = ((n + G - 1) / G + 63) / 64 * 64;
 	int32_t widest = 0;
@@ -118,9 +117,7 @@ bool fits(const bfmx_system* s, int* groups, int* window) {
 		}
 		widest = std::max(widest, hi - lo + 1);
 	}
-	*groups = static_cast<int>(G);
-	*window = widest;
-	return widest <= kMaxWindow;
+	return widest <= kMaxWindow ? widest : 0;
 }
 
 }  // namespace resident
@@ -133,9 +130,9 @@ int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double d
 		return BFMX_OK;
 	}
 	if (s->res_groups < 0) {
-		int G = 0, win = 0;
-		s->res_groups = fits(s, &G, &win) ? G : 0;
-		s->res_window = win;
+		int64_t const groups = (s->n_nodes + kRows - 1) / kRows;
+		s->res_window = window_of(s, groups);
+		s->res_groups = s->res_window > 0 ? static_cast<int>(groups) : 0;
 		s->res_width = *std::max_element(s->row_len.begin(), s->row_len.end());
 	}
 	int const G = s->res_groups;
@@ -188,5 +185,343 @@ int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double d
 		mode = 2;
 	}
 }
+
+// ------------------------------------------------------------------ batches
+// One launch runs many clusters. The systems are sorted into queues by the
+// size of the cluster they need; a queue's clusters take its systems largest
+// first, one after another. The workgroups (one a CU) are dealt to the queues
+// so that they are expected to end together, and neighbouring cluster sizes
+// share a launch where that ends sooner. A batch is then bound by the sum of
+// its work: in the streaming kernel, one workgroup a system, the largest one's
+// time on one CU is the least a launch can take.
+// Measured, whole launch with the assembly, block Jacobi to 1e-8: 256 panels of
+// 500 to 4,000 nodes 63.2 -> 16.1 ms, 64 panels of 3,000 to 30,000 nodes 835 ->
+// 85 ms, 512 of 500 to 30,000 1,911 -> 518 ms.
+
+namespace resident {
+namespace {
+
+struct Queue {
+	int32_t begin, end;   // in the order of the plan
+	int32_t next;
+	int32_t pad;
+};
+struct Member {
+	int32_t queue, cluster, g, G;
+};
+
+constexpr double kLaunchUs = 20;   // of one launch of clusters
+constexpr int kClearParts = 8;   // workgroups clearing one system's words
+
+// Clears what the runs of the plan's systems exchange.
+__global__ __launch_bounds__(kBlock) void k_clear_batch(const View* __restrict__ views,
+                                                        const int32_t* __restrict__ order,
+                                                        const int32_t* __restrict__ groups,
+                                                        Queue* __restrict__ queues, int nq, u64* __restrict__ post,
+                                                        int npost) {
+	int const k = blockIdx.x / kClearParts, part = blockIdx.x % kClearParts;
+	int const gid = part * kBlock + threadIdx.x, step = kClearParts * kBlock;
+	if (k == 0) {
+		for (int i = gid; i < nq; i += step) {
+			queues[i].next = queues[i].begin;
+		}
+		for (int i = gid; i < npost; i += step) {
+			post[i] = 0;
+		}
+	}
+	int const G = groups[k];
+	if (G == 1) {
+		return;
+	}
+	View const V = views[order[k]];
+	for (int64_t i = gid; i < 2 * V.n; i += step) {
+		V.w[0][i] = V.w[1][i] = V.w[2][i] = V.w[3][i] = 0;
+	}
+	for (int i = gid; i < 2 * G * kSlotWords; i += step) {
+		V.slots[i] = 0;
+	}
+}
+
+template <int W, int PRE>
+__global__ __launch_bounds__(kRows) void k_resident_batch(const View* __restrict__ views,
+                                                          const int32_t* __restrict__ order,
+                                                          const Member* __restrict__ members,
+                                                          Queue* __restrict__ queues, u64* __restrict__ post,
+                                                          double rtol2, int64_t max_iter, Out* __restrict__ out) {
+	extern __shared__ __align__(16) double dyn[];
+	__shared__ Shared sh;
+	__shared__ int job;
+	Member const M = members[blockIdx.x];
+	for (uint32_t round = 1;; round++) {
+		if (threadIdx.x == 0) {
+			// the cluster's first workgroup takes the next system and posts it
+			int k = -1;
+			u64* const at = post + M.cluster;
+			if (M.g == 0) {
+				k = atomicAdd(&queues[M.queue].next, 1);
+				k = k < queues[M.queue].end ? order[k] : -1;
+				if (M.G > 1) {
+					put(at, (static_cast<u64>(static_cast<uint32_t>(k)) << 32) | round);
+				}
+			} else {
+				for (uint32_t spin = 0; spin < kSpinLimit; spin++) {
+					u64 const v = get(at);
+					if (static_cast<uint32_t>(v) == round) {
+						k = static_cast<int>(v >> 32);
+						break;
+					}
+				}
+			}
+			job = k;
+		}
+		__syncthreads();
+		int const k = __builtin_amdgcn_readfirstlane(job);
+		if (k < 0) {
+			break;
+		}
+		View const V = views[k];
+		Run R;
+		run_pcg<double, W, PRE, kRows>(V, M.g, M.G, 0, rtol2, 0.0, max_iter, true, sh,
+		                               reinterpret_cast<resident::dbl2*>(dyn), R);
+		if (M.g == 0 && threadIdx.x == 0) {
+			out[k].iter = R.iter;
+			out[k].rr_true = R.rr_true;
+			out[k].bb = R.bb;
+			out[k].status = R.status;
+			out[k].checks = R.checks;
+		}
+		if (R.status == kFailed) {
+			break;
+		}
+		__syncthreads();
+	}
+}
+
+// Sizes of a cluster: the smallest that holds a system's rows is taken.
+constexpr int kGroups[] = {1,  2,  3,  4,  5,  6,  7,  8,  10, 12,  14,  16,  18,  20,
+                           24, 28, 32, 40, 48, 56, 64, 80, 96, 128, 160, 192, 224, 256};
+
+// Expected microseconds of a system's run: the iterations grow as the square
+// root of the nodes (panels of the batched workload: 20 sqrt(n) for 500 to
+// 30,000 nodes), an iteration with G workgroups takes what resident.h states.
+double run_us(int64_t n, int G) {
+	double const it = G == 1 ? 2.5 : G <= 8 ? 5.2 : G <= 64 ? 5.8 : 10.0;
+	return 20.0 * std::sqrt(static_cast<double>(n)) * it;
+}
+
+// The systems that take clusters of G workgroups.
+struct Class {
+	int G;
+	std::vector<int32_t> members;   // largest first
+	double total = 0, longest = 0;  // expected microseconds
+	int clusters = 0;
+
+	// when the last of them ends, with c clusters taking them largest first
+	double makespan(int c) const {
+		double const mean = total / static_cast<double>(members.size());
+		return std::max(longest, total / c + (c > 1 ? 0.5 * mean : 0.0));
+	}
+};
+
+// Clusters of the classes [c0, c1) in one launch of at most cus workgroups:
+// one each, then one more wherever the launch ends last, while there is room.
+// Returns the launch's expected time (negative: they do not fit).
+double share(std::vector<Class>& classes, size_t c0, size_t c1, int cus) {
+	int used = 0;
+	for (size_t c = c0; c < c1; c++) {
+		classes[c].clusters = 1;
+		used += classes[c].G;
+	}
+	if (used > cus) {
+		return -1;
+	}
+	while (true) {
+		Class* last = nullptr;
+		double worst = 0;
+		for (size_t c = c0; c < c1; c++) {
+			double const t = classes[c].makespan(classes[c].clusters);
+			if (t > worst) {
+				worst = t;
+				last = &classes[c];
+			}
+		}
+		if (used + last->G > cus || last->clusters == static_cast<int>(last->members.size())) {
+			return worst;
+		}
+		last->clusters++;
+		used += last->G;
+	}
+}
+
+}  // namespace
+
+struct Plan {
+	struct Launch {
+		int first, blocks;   // its members
+	};
+	std::vector<Launch> launches;
+	std::vector<int32_t> rest;
+	int taken = 0, queues = 0, clusters = 0, width = 0;
+	size_t lds = 0;
+	View* d_views = nullptr;
+	int32_t* d_order = nullptr;
+	int32_t* d_groups = nullptr;   // cluster size of each system, in that order
+	Member* d_members = nullptr;
+	Queue* d_queues = nullptr;
+	u64* d_post = nullptr;
+};
+
+void plan_destroy(Plan* p) {
+	if (!p) {
+		return;
+	}
+	dfree(p->d_views);
+	dfree(p->d_order);
+	dfree(p->d_groups);
+	dfree(p->d_members);
+	dfree(p->d_queues);
+	dfree(p->d_post);
+	delete p;
+}
+
+const std::vector<int32_t>& plan_rest(const Plan* p) {
+	return p->rest;
+}
+
+int plan_create(Plan** out, const std::vector<bfmx_system*>& systems, const std::vector<View>& views,
+                hipStream_t st) {
+	*out = nullptr;
+	int dev = 0, cus = 0;
+	BFMX_HIP(hipGetDevice(&dev));
+	BFMX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+	std::vector<int32_t> by_size(systems.size());
+	for (size_t k = 0; k < by_size.size(); k++) {
+		by_size[k] = static_cast<int32_t>(k);
+	}
+	std::stable_sort(by_size.begin(), by_size.end(),
+	                 [&](int32_t a, int32_t c) { return systems[a]->n_nodes > systems[c]->n_nodes; });
+	std::vector<Class> classes;
+	auto* p = new Plan();
+	int widest = 0;
+	for (int32_t const k : by_size) {
+		bfmx_system const* s = systems[k];
+		int64_t const need = (s->n_nodes + kRows - 1) / kRows;
+		auto const g = std::find_if(std::begin(kGroups), std::end(kGroups), [&](int x) { return x >= need; });
+		int const win = g != std::end(kGroups) && *g <= cus ? window_of(s, *g) : 0;
+		if (win == 0) {
+			p->rest.push_back(k);
+			continue;
+		}
+		if (classes.empty() || classes.back().G != *g) {
+			classes.push_back(Class{*g, {}});
+		}
+		double const us = run_us(s->n_nodes, *g);
+		classes.back().members.push_back(k);
+		classes.back().total += us;
+		classes.back().longest = std::max(classes.back().longest, us);
+		widest = std::max(widest, win);
+		p->width = std::max(p->width, *std::max_element(s->row_len.begin(), s->row_len.end()));
+		p->taken++;
+	}
+	if (p->taken == 0) {
+		delete p;
+		return BFMX_OK;
+	}
+	p->lds = static_cast<size_t>(widest) * sizeof(resident::dbl2) + static_cast<size_t>(spare(false, p->width, kRows));
+	std::vector<int32_t> order, groups;
+	std::vector<Queue> queues;
+	std::vector<Member> members;
+	// neighbouring classes share a launch where that ends sooner than one
+	// launch after another: best[c] is the least expected time of the classes
+	// from c on, upto[c] the end of their first launch
+	size_t const nc = classes.size();
+	std::vector<double> best(nc + 1, 0);
+	std::vector<size_t> upto(nc + 1, nc);
+	for (size_t c0 = nc; c0-- > 0;) {
+		best[c0] = -1;
+		for (size_t c1 = c0 + 1; c1 <= nc; c1++) {
+			double const t = share(classes, c0, c1, cus);
+			if (t >= 0 && (best[c0] < 0 || t + kLaunchUs + best[c1] < best[c0])) {
+				best[c0] = t + kLaunchUs + best[c1];
+				upto[c0] = c1;
+			}
+		}
+	}
+	for (size_t c0 = 0; c0 < nc; c0 = upto[c0]) {
+		size_t const c1 = upto[c0];
+		share(classes, c0, c1, cus);
+		int const first = static_cast<int>(members.size());
+		for (size_t c = c0; c < c1; c++) {
+			Class& C = classes[c];
+			int const begin = static_cast<int>(order.size());
+			order.insert(order.end(), C.members.begin(), C.members.end());
+			groups.insert(groups.end(), C.members.size(), C.G);
+			for (int k = 0; k < C.clusters; k++) {
+				for (int g = 0; g < C.G; g++) {
+					members.push_back(Member{static_cast<int32_t>(queues.size()), p->clusters, g, C.G});
+				}
+				p->clusters++;
+			}
+			queues.push_back(Queue{begin, static_cast<int32_t>(order.size()), begin, 0});
+		}
+		p->launches.push_back(Plan::Launch{first, static_cast<int>(members.size()) - first});
+	}
+	p->queues = static_cast<int>(queues.size());
+	int const rc = [&]() -> int {
+		BFMX_CHECK(dalloc(&p->d_views, views.size()));
+		BFMX_CHECK(dalloc(&p->d_order, order.size()));
+		BFMX_CHECK(dalloc(&p->d_groups, groups.size()));
+		BFMX_CHECK(dalloc(&p->d_members, members.size()));
+		BFMX_CHECK(dalloc(&p->d_queues, queues.size()));
+		BFMX_CHECK(dalloc(&p->d_post, static_cast<size_t>(p->clusters)));
+		BFMX_HIP(hipMemcpyAsync(p->d_views, views.data(), views.size() * sizeof(View), hipMemcpyHostToDevice, st));
+		BFMX_HIP(hipMemcpyAsync(p->d_order, order.data(), order.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
+		BFMX_HIP(hipMemcpyAsync(p->d_groups, groups.data(), groups.size() * sizeof(int32_t), hipMemcpyHostToDevice,
+		                        st));
+		BFMX_HIP(hipMemcpyAsync(p->d_members, members.data(), members.size() * sizeof(Member), hipMemcpyHostToDevice,
+		                        st));
+		BFMX_HIP(hipMemcpyAsync(p->d_queues, queues.data(), queues.size() * sizeof(Queue), hipMemcpyHostToDevice,
+		                        st));
+		BFMX_HIP(hipStreamSynchronize(st));
+		return BFMX_OK;
+	}();
+	if (rc != BFMX_OK) {
+		plan_destroy(p);
+		return rc;
+	}
+	*out = p;
+	return BFMX_OK;
+}
+
+int plan_launch(Plan* p, hipStream_t st, int precond, double rtol2, int64_t max_iter, Out* d_out, bool* launched) {
+	*launched = false;
+	bool const point = precond == BFMX_PRECOND_JACOBI;
+	auto const kernel = p->width <= 7
+	                        ? (point ? k_resident_batch<7, BFMX_PRECOND_JACOBI> : k_resident_batch<7, BFMX_PRECOND_BLOCK_JACOBI>)
+	                        : (point ? k_resident_batch<9, BFMX_PRECOND_JACOBI> : k_resident_batch<9, BFMX_PRECOND_BLOCK_JACOBI>);
+	BFMX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+	                             static_cast<int>(p->lds)));
+	k_clear_batch<<<p->taken * kClearParts, kBlock, 0, st>>>(p->d_views, p->d_order, p->d_groups, p->d_queues, p->queues,
+	                                                   p->d_post, p->clusters);
+	BFMX_HIP(hipGetLastError());
+	for (auto const& L : p->launches) {
+		const View* views = p->d_views;
+		const int32_t* order = p->d_order;
+		const Member* members = p->d_members + L.first;
+		Queue* queues = p->d_queues;
+		u64* post = p->d_post;
+		void* args[] = {&views, &order, &members, &queues, &post, &rtol2, &max_iter, &d_out};
+		hipError_t const err = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kernel), dim3(L.blocks),
+		                                                  dim3(kRows), args, static_cast<unsigned>(p->lds), st);
+		if (err != hipSuccess) {
+			(void) hipGetLastError();
+			return BFMX_OK;
+		}
+	}
+	*launched = true;
+	return BFMX_OK;
+}
+
+}  // namespace resident
 
 }  // namespace bfmx

@@ -292,7 +292,9 @@ int bfmx_system_apply_model(bfmx_system_t* s, const double* r, double* z);
  * < 2048, < 8192, >= 8192 nodes), the launches captured in one HIP graph.
  * A batch holds either existing assembled systems (bfmx_batch_create) or
  * meshes that every launch assembles before solving
- * (bfmx_batch_create_planar). A configuration is a workgroup size x rows-per-thread pair:
+ * (bfmx_batch_create_planar). Systems of at most 262,144 nodes and nine blocks
+ * a row are solved by clusters of workgroups that hold the matrix in registers,
+ * whatever the configuration; configurations apply to the others. A configuration is a workgroup size x rows-per-thread pair:
  * 0 = 256 x 1, 1 = 256 x 2, 2 = 512 x 1, 3 = 512 x 2, 4 = 1024 x 1. A
  * system's solution does not depend on the rest of the batch (bitwise, for
  * the same configuration). The systems must outlive the batch and stay
@@ -313,8 +315,8 @@ int bfmx_batch_autotune(bfmx_batch_t* b, int precond, int sample, int iters, int
  * the default configurations, max_iter 0 = 20 x the largest DOF count.
  * stats (may be NULL) receives one entry per system, total_ms the launch's
  * device time. Returns BFMX_OK when every system converged.
- * precond BFMX_PRECOND_JACOBI / BFMX_PRECOND_BLOCK_JACOBI: the persistent
- * launch above.
+ * precond BFMX_PRECOND_JACOBI / BFMX_PRECOND_BLOCK_JACOBI: the launches
+ * above.
  * precond BFMX_PRECOND_AMG (multigrid mode): the batch is solved as one
  * block-diagonal system (the systems' rows one after another, a second copy
  * of their matrices) by flexible CG with the FP32 multigrid V-cycle, one

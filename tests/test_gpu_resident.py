@@ -22,7 +22,7 @@ RTOL = 1e-9
 
 def strip(n, kind, het, seed=5):
     """A beam of exactly n nodes: a grid h nodes high, cut off along its last column."""
-    h = 4 if n < 256 else 16 if n < 1000 else 32
+    h = 4 if n < 256 else 16 if n < 1000 else 32 if n < 4000 else 96
     nx = -(-n // h)
     m = meshgen.beam(nx, h - 1, kind=kind, length=nx / h, height=1.0, jitter=0.2, seed=seed)
     # nodes column by column, so that the first n of them are a prefix of the grid
@@ -142,3 +142,34 @@ def test_clusters_on_several_threads():
     for t in threads:
         t.join()
     assert all(np.array_equal(a, g) for a, g in zip(alone, got))
+
+
+@pytest.mark.parametrize("pre", [D.PRECOND_JACOBI, D.PRECOND_BLOCK_JACOBI])
+def test_batches_of_clusters(monkeypatch, pre):
+    """Clusters of many sizes in one batch, Q1 and P1, with a system that does not fit (it takes the streaming
+    kernel in the same call); each against the streaming kernel and, bitwise, a batch of its own."""
+    systems = [D.beam_system(strip(n, 3 + k % 2, het=False, seed=k))
+               for k, n in enumerate((64, 1024, 1026, 2050, 3200, 5000, 7000, 9000, 12500, 20600, 2048, 30002))]
+    wide = meshgen.beam(120, 50, kind=4, jitter=0.2, seed=4)
+    p = np.random.default_rng(1).permutation(wide.n_nodes)
+    q = np.empty_like(p)
+    q[p] = np.arange(p.size)
+    wide.coords, wide.elems = wide.coords[p], q[wide.elems.astype(np.int64)].astype(np.uint64)
+    wide.edges = q[wide.edges.astype(np.int64)]
+    wide.node_sets = {name: v[p] for name, v in wide.node_sets.items()}
+    systems.insert(5, D.beam_system(wide, renumber=False))
+    b = D.Batch(systems)
+    monkeypatch.setenv("BFMX_RESIDENT", "0")
+    st_ref, _ = b.solve(precond=pre, rtol=1e-8)
+    ref = [b.get_u(k) for k in range(len(systems))]
+    monkeypatch.delenv("BFMX_RESIDENT")
+    st, _ = b.solve(precond=pre, rtol=1e-8)
+    for k, s in enumerate(systems):
+        assert st[k]["status"] == 0 and st[k]["rel_residual"] <= 1e-8, k
+        u = b.get_u(k)
+        assert rel_err(u, ref[k]) <= 1e-6, k
+        A, f = s.get_csr_scipy(), s.get_rhs()
+        assert np.linalg.norm(f - A @ u) <= 1.1e-8 * np.linalg.norm(f), k
+        one = D.Batch([s])
+        one.solve(precond=pre, rtol=1e-8)
+        assert np.array_equal(one.get_u(0), u), k

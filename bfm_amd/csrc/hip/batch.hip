@@ -197,45 +197,72 @@ __device__ __forceinline__ void for_rows(int64_t n, F f) {
 	}
 }
 
-// Assembly of one system by one workgroup, in the order of the streaming
-// kernels: zeroed values and load, the element colours one after another
-// (no two elements of a colour share a node), the conditions in call order,
-// then the symmetric elimination.
-template <int BS, int KIND>
-__device__ void assemble_elements(const BatchInst& S) {
-	for (int c = 0; c < S.n_colors; c++) {
-		int32_t const e1 = S.color_ptr[c + 1];
-		for (int64_t e = S.color_ptr[c] + threadIdx.x; e < e1; e += BS) {
-			dev::assemble_any<KIND>(
-			    e, S.elem, S.coords, S.M,
-			    [&](int j, int k, const int* nd) { return dev::find_slot(S.slice_ptr, S.row_len, S.col, nd[j], nd[k]); },
-			    S.val, S.b);
-		}
-		__syncthreads();
+// Assembly of every system of a batch built from meshes, in the order of the
+// streaming kernels: zeroed values and load, the element colours one after
+// another (no two elements of a colour share a node), the conditions in call
+// order, then the symmetric elimination. One launch clears, one a colour adds
+// the elements of that colour, each with `parts` workgroups a system, and one
+// workgroup a system applies the conditions (short node lists). One workgroup
+// a system for all of it left most of the GPU idle and ended with the largest
+// system: 4.8 ms for 64 panels of 3,000 to 30,000 nodes and 0.76 ms for 256 of
+// 500 to 4,000; here 1.3 ms for the 64. (Within the solve kernel the element
+// arithmetic's ~200 registers would cut its occupancy.)
+constexpr int kAsmBlock = 256;
+constexpr int kAsmParts = 64;   // workgroups of one system at most
+
+__global__ __launch_bounds__(kAsmBlock) void k_batch_zero(const BatchInst* __restrict__ insts,
+                                                          const int32_t* __restrict__ order, int parts) {
+	BatchInst const& S = insts[order[blockIdx.x / parts]];
+	int64_t const t = (blockIdx.x % parts) * kAsmBlock + threadIdx.x, step = static_cast<int64_t>(parts) * kAsmBlock;
+	double* const val = S.val;
+	int64_t const nv = 2 * S.nnzb_pad, n = S.n;
+	for (int64_t k = t; k < nv; k += step) {
+		st2(val + 2 * k, dbl2{0, 0});
+	}
+	double* const b = S.b;
+	double* const vfirst = S.vfirst;
+	uint8_t* const fixed = S.fixed;
+	for (int64_t i = t; i < n; i += step) {
+		st2(b + 2 * i, dbl2{0, 0});
+		st2(vfirst + 2 * i, dbl2{0, 0});
+		fixed[2 * i] = 0;
+		fixed[2 * i + 1] = 0;
 	}
 }
 
-template <int BS>
-__device__ void assemble_system(const BatchInst& S) {
-	int64_t const n = S.n;
-	for (int64_t k = threadIdx.x; k < 2 * S.nnzb_pad; k += BS) {
-		st2(S.val + 2 * k, dbl2{0, 0});
+template <int KIND>
+__device__ __forceinline__ void assemble_elements(const BatchInst& S, int64_t e0, int64_t e1, int64_t step) {
+	for (int64_t e = e0; e < e1; e += step) {
+		dev::assemble_any<KIND>(
+		    e, S.elem, S.coords, S.M,
+		    [&](int j, int k, const int* nd) { return dev::find_slot(S.slice_ptr, S.row_len, S.col, nd[j], nd[k]); },
+		    S.val, S.b);
 	}
-	for (int64_t i = threadIdx.x; i < n; i += BS) {
-		st2(S.b + 2 * i, dbl2{0, 0});
-		st2(S.vfirst + 2 * i, dbl2{0, 0});
-		S.fixed[2 * i] = 0;
-		S.fixed[2 * i + 1] = 0;
+}
+
+__global__ __launch_bounds__(kAsmBlock) void k_batch_elements(const BatchInst* __restrict__ insts,
+                                                              const int32_t* __restrict__ order, int parts,
+                                                              int color) {
+	BatchInst const S = insts[order[blockIdx.x / parts]];
+	if (color >= S.n_colors) {
+		return;
 	}
-	__syncthreads();
+	int64_t const e0 = S.color_ptr[color] + (blockIdx.x % parts) * kAsmBlock + threadIdx.x;
+	int64_t const e1 = S.color_ptr[color + 1];
+	int64_t const step = static_cast<int64_t>(parts) * kAsmBlock;
 	if (S.kind == 3) {
-		assemble_elements<BS, 3>(S);
+		assemble_elements<3>(S, e0, e1, step);
 	} else {
-		assemble_elements<BS, 4>(S);
+		assemble_elements<4>(S, e0, e1, step);
 	}
+}
+
+__global__ __launch_bounds__(kAsmBlock) void k_batch_conditions(const BatchInst* __restrict__ insts,
+                                                                const int32_t* __restrict__ order) {
+	BatchInst const S = insts[order[blockIdx.x]];
 	for (int q = 0; q < S.n_cond; q++) {
 		CondRec const C = S.conds[q];
-		for (int t = threadIdx.x; t < C.count; t += BS) {
+		for (int t = threadIdx.x; t < C.count; t += kAsmBlock) {
 			int32_t const i = S.lists[C.list_off + t];
 			if (C.kind == BFMX_DIRICHLET_X || C.kind == BFMX_DIRICHLET_Y) {
 				dev::dirichlet_xy(i, C.kind, C.value, S.fixed, S.vfirst, S.b);
@@ -250,22 +277,9 @@ __device__ void assemble_system(const BatchInst& S) {
 		}
 		__syncthreads();
 	}
-	for (int t = threadIdx.x; t < S.n_elim; t += BS) {
+	for (int t = threadIdx.x; t < S.n_elim; t += kAsmBlock) {
 		dev::eliminate_row(S.elim[t], S.slice_ptr, S.row_len, S.col, S.fixed, S.vfirst, S.val, S.b);
 	}
-	__syncthreads();
-}
-
-// Assembly of every system of a batch built from meshes, one workgroup per
-// system. A launch of its own: the element arithmetic holds the Gauss-point
-// gradients in registers (about 200 VGPRs for Q1), which inside the solve
-// kernel would cut its occupancy from 6-8 waves per SIMD to 2.
-constexpr int kAsmBlock = 256;
-
-__global__ __launch_bounds__(kAsmBlock) void k_batch_assemble(const BatchInst* __restrict__ insts,
-                                                              const int32_t* __restrict__ order) {
-	BatchInst const S = insts[order[blockIdx.x]];
-	assemble_system<kAsmBlock>(S);
 }
 
 template <int BS, int RPT, int PRE>
@@ -435,18 +449,52 @@ void launch(int pre, int cfg, int nblocks, hipStream_t st, const BatchInst* inst
 // true residual, so the run ends when each meets rtol.
 constexpr int kUniBlock = 256;
 
-// Per instance: b . b (fixed summation order).
+// Sums over an instance's rows are formed in kUniParts shares, one workgroup
+// each, and combined in order: one workgroup an instance waited for the largest
+// (64 panels of 3,000 to 30,000 nodes: residuals 570 us, load norms 83 us; here
+// 71 and 12 us).
+constexpr int kUniParts = 32;
+
+// This share's rows of an instance.
+__device__ __forceinline__ void share_of(int64_t n, int part, int64_t& r0, int64_t& r1) {
+	int64_t const rows = (n + kUniParts - 1) / kUniParts;
+	r0 = min(part * rows, n);
+	r1 = min(r0 + rows, n);
+}
+
+// Per instance and share: b . b (fixed summation order).
 __global__ __launch_bounds__(kUniBlock) void k_batch_bnorm(const BatchInst* __restrict__ insts,
-                                                           double* __restrict__ bb) {
+                                                           double* __restrict__ part) {
 	__shared__ double lds[1][kUniBlock / 64];
-	BatchInst const S = insts[blockIdx.x];
+	BatchInst const& S = insts[blockIdx.x / kUniParts];
+	const double* const b = S.b;
+	int64_t r0, r1;
+	share_of(S.n, blockIdx.x % kUniParts, r0, r1);
 	double v[1] = {0};
-	for (int64_t i = threadIdx.x; i < 2 * S.n; i += kUniBlock) {
-		v[0] += S.b[i] * S.b[i];
+	for (int64_t i = 2 * r0 + threadIdx.x; i < 2 * r1; i += kUniBlock) {
+		v[0] += b[i] * b[i];
 	}
 	wg_sum<kUniBlock, 1>(v, lds);
 	if (threadIdx.x == 0) {
-		bb[blockIdx.x] = v[0];
+		part[blockIdx.x] = v[0];
+	}
+}
+
+// The sum of an instance's shares, in order.
+__device__ __forceinline__ double sum_shares(const double* __restrict__ part) {
+	double v = 0;
+#pragma unroll 8
+	for (int k = 0; k < kUniParts; k++) {
+		v += part[k];
+	}
+	return v;
+}
+
+__global__ __launch_bounds__(kUniBlock) void k_batch_bnorm_sum(int m, const double* __restrict__ part,
+                                                               double* __restrict__ bb) {
+	int const k = blockIdx.x * kUniBlock + threadIdx.x;
+	if (k < m) {
+		bb[k] = sum_shares(part + static_cast<int64_t>(k) * kUniParts);
 	}
 }
 
@@ -507,26 +555,37 @@ __global__ __launch_bounds__(kBlock) void k_union_scatter(int64_t n, int m, cons
 	st2(insts[k].x + 2 * i, sqrt(bb[k]) * ld2(ux + 2 * R));
 }
 
-// Per instance: the true residual ||b - A x||^2 of its own system, and the
-// report of the union's solve.
+// Per instance and share: the true residual ||b - A x||^2 of its own system.
 __global__ __launch_bounds__(kUniBlock) void k_batch_resid(const BatchInst* __restrict__ insts,
-                                                           const double* __restrict__ bb, int64_t iters,
-                                                           double rtol2, BatchOut* __restrict__ out) {
+                                                           double* __restrict__ part) {
 	__shared__ double lds[1][kUniBlock / 64];
-	BatchInst const S = insts[blockIdx.x];
+	BatchInst const S = insts[blockIdx.x / kUniParts];
+	int64_t r0, r1;
+	share_of(S.n, blockIdx.x % kUniParts, r0, r1);
 	double v[1] = {0};
-	for (int64_t i = threadIdx.x; i < S.n; i += kUniBlock) {
+	for (int64_t i = r0 + threadIdx.x; i < r1; i += kUniBlock) {
 		dbl2 const ax = row_mul(S, i, [&](int32_t c) { return ld2(S.x + 2 * static_cast<int64_t>(c)); });
 		dbl2 const rv = ld2(S.b + 2 * i) - ax;
 		v[0] += rv.x * rv.x + rv.y * rv.y;
 	}
 	wg_sum<kUniBlock, 1>(v, lds);
 	if (threadIdx.x == 0) {
-		BatchOut& o = out[blockIdx.x];
+		part[blockIdx.x] = v[0];
+	}
+}
+
+// The report of the union's solve.
+__global__ __launch_bounds__(kUniBlock) void k_batch_report(int m, const double* __restrict__ part,
+                                                            const double* __restrict__ bb, int64_t iters,
+                                                            double rtol2, BatchOut* __restrict__ out) {
+	int const k = blockIdx.x * kUniBlock + threadIdx.x;
+	if (k < m) {
+		double const rr = sum_shares(part + static_cast<int64_t>(k) * kUniParts);
+		BatchOut& o = out[k];
 		o.iter = iters;
-		o.rr_true = v[0];
-		o.bb = bb[blockIdx.x];
-		o.status = v[0] <= rtol2 * bb[blockIdx.x] ? 1 : 0;
+		o.rr_true = rr;
+		o.bb = bb[k];
+		o.status = rr <= rtol2 * bb[k] ? 1 : 0;
 		o.checks = 0;
 	}
 }
@@ -575,6 +634,7 @@ struct bfmx_batch {
 	bfmx_system* uni = nullptr;
 	int64_t* d_uoff = nullptr;     // first union row of each instance (m + 1)
 	double* d_ubb = nullptr;       // b . b of each instance
+	double* d_upart = nullptr;     // sums of each instance's shares of rows
 };
 
 namespace bfmx {
@@ -626,6 +686,7 @@ void union_release(bfmx_batch* b) {
 	b->uni = nullptr;
 	dfree(b->d_uoff);
 	dfree(b->d_ubb);
+	dfree(b->d_upart);
 }
 
 void batch_destroy(bfmx_batch* b) {
@@ -777,8 +838,24 @@ void launch_assemble(bfmx_batch* b) {
 		for (auto* s : b->systems) {
 			s->val_gen++;
 		}
-		k_batch_assemble<<<static_cast<int>(b->systems.size()), kAsmBlock, 0, b->stream>>>(b->d_inst,
-		                                                                                   b->d_order_all);
+		int64_t const m = static_cast<int64_t>(b->systems.size());
+		int64_t most = 1;
+		int colors = 0;
+		for (auto const* s : b->systems) {
+			most = std::max(most, s->n_elems);
+			colors = std::max(colors, s->n_colors);
+		}
+		// enough workgroups for a colour (an eighth) of the largest system, as
+		// long as the launch's total stays moderate
+		int64_t const want = (most / 8 + kAsmBlock - 1) / kAsmBlock;
+		int const parts = static_cast<int>(
+		    std::max<int64_t>(1, std::min({want, static_cast<int64_t>(kAsmParts), 65536 / std::max<int64_t>(m, 1)})));
+		int const blocks = static_cast<int>(m) * parts;
+		k_batch_zero<<<blocks, kAsmBlock, 0, b->stream>>>(b->d_inst, b->d_order_all, parts);
+		for (int c = 0; c < colors; c++) {
+			k_batch_elements<<<blocks, kAsmBlock, 0, b->stream>>>(b->d_inst, b->d_order_all, parts, c);
+		}
+		k_batch_conditions<<<static_cast<int>(m), kAsmBlock, 0, b->stream>>>(b->d_inst, b->d_order_all);
 	}
 }
 
@@ -918,6 +995,7 @@ int union_build_parts(bfmx_batch* b) {
 	BFMX_CHECK(dalloc(&U->d_fixed, 2 * n));
 	BFMX_CHECK(dalloc(&b->d_uoff, m + 1));
 	BFMX_CHECK(dalloc(&b->d_ubb, m));
+	BFMX_CHECK(dalloc(&b->d_upart, m * kUniParts));
 	BFMX_CHECK(dalloc(&U->d_conv_part, 2 * m));
 	U->n_conv_seg = static_cast<int>(m);   // every instance meets the tolerance on its own
 	U->d_conv_seg = b->d_uoff;
@@ -946,7 +1024,9 @@ int batch_solve_amg(bfmx_batch* b, double rtol, int64_t max_iter, bfmx_stats_t* 
 	int64_t const n = U->n_nodes;
 	BFMX_HIP(hipEventRecord(b->ev[0], st));
 	launch_assemble(b);
-	k_batch_bnorm<<<m, kUniBlock, 0, st>>>(b->d_inst, b->d_ubb);
+	int const sums = (m + kUniBlock - 1) / kUniBlock;
+	k_batch_bnorm<<<m * kUniParts, kUniBlock, 0, st>>>(b->d_inst, b->d_upart);
+	k_batch_bnorm_sum<<<sums, kUniBlock, 0, st>>>(m, b->d_upart, b->d_ubb);
 	U->val_gen++;
 	k_union_gather<<<blocks_of(n), kBlock, 0, st>>>(n, m, b->d_uoff, b->d_inst, b->d_ubb, U->d_slice_ptr, U->d_val,
 	                                                U->d_b, U->d_fixed);
@@ -969,7 +1049,8 @@ int batch_solve_amg(bfmx_batch* b, double rtol, int64_t max_iter, bfmx_stats_t* 
 		BFMX_HIP(hipMemsetAsync(U->d_x, 0, 2 * n * sizeof(double), st));
 	}
 	k_union_scatter<<<blocks_of(n), kBlock, 0, st>>>(n, m, b->d_uoff, b->d_inst, b->d_ubb, U->d_x);
-	k_batch_resid<<<m, kUniBlock, 0, st>>>(b->d_inst, b->d_ubb, us.iterations, rtol * rtol, b->d_out);
+	k_batch_resid<<<m * kUniParts, kUniBlock, 0, st>>>(b->d_inst, b->d_upart);
+	k_batch_report<<<sums, kUniBlock, 0, st>>>(m, b->d_upart, b->d_ubb, us.iterations, rtol * rtol, b->d_out);
 	BFMX_HIP(hipGetLastError());
 	BFMX_HIP(hipEventRecord(b->ev[1], st));
 	BFMX_HIP(hipMemcpyAsync(b->h_out.data(), b->d_out, b->h_out.size() * sizeof(BatchOut), hipMemcpyDeviceToHost,

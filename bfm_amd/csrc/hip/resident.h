@@ -68,7 +68,7 @@ constexpr uint32_t kSpinLimit = 1u << 22;   // polls of one wait (seconds)
 constexpr int kSlotWords = 16;              // a 128-byte line for each workgroup's contribution to an all-gather
                                             // (several in a line cost 0.4 us more at 32 workgroups)
 constexpr int kMaxGroup = 256;              // workgroups of a cluster
-constexpr int kMaxWindow = 3900;            // nodes of a window (62 KB of the CU's 160 KB of LDS, beside 96 KB of row blocks)
+constexpr int kMaxWindow = 2900;            // nodes of a window (46 KB of the CU's 160 KB of LDS, beside 112 KB)
 constexpr int kMaxWidth = 9;                // blocks of a row held in registers
 constexpr int kCheckEvery = 16;             // iterations between true-residual checks once one has failed
 constexpr int kStall = 8;                   // such checks without halving before the run counts as stalled
@@ -174,7 +174,10 @@ struct Shared {
 
 // Blocks of a row held in registers, by threads of the workgroup: six FP64
 // blocks (48 registers) fit beside the vectors in the 128 registers a thread
-// of 1024 has (with seven the compiler spills); the others go to LDS.
+// of 1024 has; the others go to LDS. The loads of the product are kept in order
+// (multiply()) and the solution in LDS, or the compiler spills parts of the
+// matrix: a spilled register is reloaded through memory in every iteration,
+// behind the stores of the exchange (9 us an iteration instead of 4.8).
 template <typename MT, int W, int NT>
 constexpr int register_blocks() {
 	return sizeof(MT) == 8 && NT > 512 && W > 6 ? 6 : W;
@@ -183,113 +186,114 @@ template <typename MT, int W, int NT>
 constexpr int spare_bytes() {
 	return (W - register_blocks<MT, W, NT>()) * 4 * static_cast<int>(sizeof(MT)) * NT;
 }
+// Whether a thread's part of the solution lives in LDS as well (16 bytes each,
+// after the spare blocks).
+template <typename MT, int NT>
+constexpr bool lds_solution() {
+	return sizeof(MT) == 8 && NT > 512;
+}
+template <typename MT, int W, int NT>
+constexpr int fixed_bytes() {
+	return spare_bytes<MT, W, NT>() + (lds_solution<MT, NT>() ? 16 * NT : 0);
+}
 
-// One cluster's run, called by all NT threads of its workgroup g of G. On
-// return R holds the run's scalars (in every thread) and V.x the solution of
-// the workgroup's rows. win: LDS for the window's directions. mode 0 starts
-// from x = 0, 1 from the x in V.x, 2 continues a run cut at its limit (R as it
-// was left, r and p in V.save). Runs until R.iter >= stop.
-template <typename MT, int W, int PRE, int NT>
-__device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, double delta2, int64_t stop,
-                        bool final_check, Shared& sh, dbl2* lds, Run& R) {
-	constexpr int NW = NT / 64;
-	constexpr int kAhead = 1;
-	constexpr int WR = register_blocks<MT, W, NT>();
-	// the row's last W - WR blocks, two 16-byte halves each, then the window
+// The registers, LDS and exchanges of one workgroup (g of G) of a cluster. MT:
+// stored type of the matrix, W: blocks of a row at most, NT: threads.
+template <typename MT, int W, int NT>
+struct Cluster {
+	static constexpr int NW = NT / 64;
+	static constexpr int WR = register_blocks<MT, W, NT>();
 	typedef MT mt2 __attribute__((ext_vector_type(2)));
-	mt2* const spare = reinterpret_cast<mt2*>(lds);
-	dbl2* const win = lds + spare_bytes<MT, W, NT>() / sizeof(dbl2);
-	int t = threadIdx.x;
-	int const lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
-	int const n = static_cast<int>(V.n);
-	int const rows = ((n + G - 1) / G + 63) / 64 * 64;   // per workgroup (at most NT)
-	int const r0 = min(g * rows, n), r1 = min(r0 + rows, n);
-	int row = r0 + t;
-	bool const live = row < r1;
-	if (t == 0) {
-		sh.lo = r0;
-		sh.hi = r1;
-		sh.below = 0;
-		sh.above = n;
-		sh.failed = 0;
-	}
-	__syncthreads();
-	// the row's blocks into registers, columns as offsets into the window
-	MT m[WR][4];
-	uint32_t at[(W + 1) / 2];
-	int cols[W];
-	dbl2 dinv0 = {0, 0}, dinv1 = {0, 0};
-	int clo = r0, chi = r0;
-#pragma unroll
-	for (int k = 0; k < W; k++) {
-		cols[k] = r0;
-	}
-	int const s = row >> 6, r64 = row & 63;
-	int beg = 0, len = 0;
-	if (live) {
-		beg = V.slice_ptr[s] + r64;
-		len = (V.slice_ptr[s + 1] - beg + 63) >> 6;
-		clo = chi = row;
-	}
-#pragma unroll
-	for (int k = 0; k < W; k++) {
-		mt2 a = {0, 0}, c = {0, 0};
+
+	View const& V;
+	Shared& sh;
+	int const g, G, n;
+	int t, lane, wave;
+	int r0, r1, row;           // own rows, this thread's
+	bool live, shared = false; // it has a row; other workgroups read it
+	int lo, nwin, left, own, halo;   // the window: its first node, nodes, nodes before the own rows, own rows, others
+	mt2* spare;                // the row's last W - WR blocks, two halves each
+	dbl2* win;                 // the vector the matrix is applied to, over the window
+	MT m[WR][4];               // the row's first blocks
+	uint32_t at[(W + 1) / 2];  // its columns, as places in the window, two a word
+	uint32_t ep = 0, sep = 0;  // exchanges of a vector and all-gathers so far
+
+	__device__ __forceinline__ Cluster(View const& v, Shared& s, int wg, int groups, dbl2* lds)
+	    : V(v), sh(s), g(wg), G(groups), n(static_cast<int>(v.n)) {
+		spare = reinterpret_cast<mt2*>(lds);
+		win = lds + fixed_bytes<MT, W, NT>() / sizeof(dbl2);
+		t = threadIdx.x;
+		lane = t & 63;
+		wave = __builtin_amdgcn_readfirstlane(t >> 6);
+		int const rows = ((n + G - 1) / G + 63) / 64 * 64;   // per workgroup (at most NT)
+		r0 = min(g * rows, n);
+		r1 = min(r0 + rows, n);
+		row = r0 + t;
+		live = row < r1;
+		if (t == 0) {
+			sh.lo = r0;
+			sh.hi = r1;
+			sh.below = 0;
+			sh.above = n;
+			sh.failed = 0;
+		}
+		__syncthreads();
+		int clo = r0, chi = r0;
+		int const r64 = row & 63;
+		int beg = 0, len = 0;   // the row's first block, and blocks (padding included)
 		if (live) {
-			cols[k] = row;
+			beg = V.slice_ptr[row >> 6] + r64;
+			len = (V.slice_ptr[(row >> 6) + 1] - beg + 63) >> 6;
+			clo = chi = row;
+		}
+#pragma unroll
+		for (int k = 0; k < W; k++) {
+			mt2 a = {0, 0}, c = {0, 0};
 			if (k < len) {
 				int64_t const blk = beg + k * kSlice;
-				int64_t const o = 4 * blk - 2 * r64;
-				const MT* const from = matrix<MT>(V) + o;
-				cols[k] = V.col[blk];
+				int const col = V.col[blk];
+				const MT* const from = matrix<MT>(V) + 4 * blk - 2 * r64;
 				a = *reinterpret_cast<const mt2*>(from);
 				c = *reinterpret_cast<const mt2*>(from + 2 * kSlice);
-				clo = min(clo, cols[k]);
-				chi = max(chi, cols[k]);
+				clo = min(clo, col);
+				chi = max(chi, col);
 			}
+			if (k < WR) {
+				m[k < WR ? k : 0][0] = a.x;
+				m[k < WR ? k : 0][1] = a.y;
+				m[k < WR ? k : 0][2] = c.x;
+				m[k < WR ? k : 0][3] = c.y;
+			} else {
+				spare[(2 * (k - WR)) * NT + t] = a;
+				spare[(2 * (k - WR) + 1) * NT + t] = c;
+			}
+			__builtin_amdgcn_sched_barrier(0);   // one block at a time: few registers
 		}
-		if (k < WR) {
-			m[k < WR ? k : 0][0] = a.x;
-			m[k < WR ? k : 0][1] = a.y;
-			m[k < WR ? k : 0][2] = c.x;
-			m[k < WR ? k : 0][3] = c.y;
-		} else {
-			spare[(2 * (k - WR)) * NT + t] = a;
-			spare[(2 * (k - WR) + 1) * NT + t] = c;
+		if (live) {
+			atomicMin(&sh.lo, clo);
+			atomicMax(&sh.hi, chi + 1);
 		}
-	}
-	if (live) {
-		const double* top = V.val + 4 * static_cast<int64_t>(V.diag_blk[row]) - 2 * r64;
-		double const a00 = top[0], a01 = top[1], a10 = top[2 * kSlice], a11 = top[2 * kSlice + 1];
-		if (PRE == BFMX_PRECOND_JACOBI) {
-			dinv0 = dbl2{1.0 / a00, 1.0 / a11};
-		} else {
-			double const det = a00 * a11 - a01 * a10;
-			dinv0 = dbl2{a11 / det, -a01 / det};
-			dinv1 = dbl2{-a10 / det, a00 / det};
-		}
-		atomicMin(&sh.lo, clo);
-		atomicMax(&sh.hi, chi + 1);
-	}
-	__syncthreads();
-	int const lo = __builtin_amdgcn_readfirstlane(sh.lo), nwin = __builtin_amdgcn_readfirstlane(sh.hi) - lo, left = r0 - lo, own = r1 - r0, halo = nwin - own;
+		__syncthreads();
+		lo = __builtin_amdgcn_readfirstlane(sh.lo);
+		nwin = __builtin_amdgcn_readfirstlane(sh.hi) - lo;
+		left = r0 - lo;
+		own = r1 - r0;
+		halo = nwin - own;
+		// a block past the row's end (its values are zero) takes place 0
+		auto place = [&](int k) { return k < len ? static_cast<uint32_t>(V.col[beg + k * kSlice] - lo) : 0u; };
 #pragma unroll
-	for (int k = 0; k < W; k += 2) {
-		uint32_t const a = static_cast<uint32_t>(cols[k] - lo);
-		uint32_t const c = k + 1 < W ? static_cast<uint32_t>(cols[k + 1 < W ? k + 1 : k] - lo) : 0;
-		at[k / 2] = a | (c << 16);
-	}
-	auto precond = [&](dbl2 r) {
-		if (PRE == BFMX_PRECOND_JACOBI) {
-			return dbl2{dinv0.x * r.x, dinv0.y * r.y};
+		for (int k = 0; k < W; k += 2) {
+			at[k / 2] = place(k) | (k + 1 < W ? place(k + 1) << 16 : 0u);
+			__builtin_amdgcn_sched_barrier(0);
 		}
-		return dbl2{dinv0.x * r.x + dinv0.y * r.y, dinv1.x * r.x + dinv1.y * r.y};
-	};
+		if (G > 1) {
+			share_windows();
+		}
+	}
 
-	uint32_t ep = 0;   // exchanges of a vector so far
-	uint32_t sep = 0;  // all-gathers so far
-	// the rows that other workgroups read: the first all-gather is of the windows
-	bool shared = false;
-	if (G > 1) {
+	// The rows that other workgroups read: the first all-gather is of the
+	// windows.
+	__device__ __forceinline__ void share_windows() {
 		sep = 1;
 		u64* const base = V.slots + static_cast<int64_t>(G) * kSlotWords;
 		if (t < 2) {
@@ -319,13 +323,34 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 		__syncthreads();
 		shared = live && (row < sh.below || row >= sh.above);
 	}
-	// word k (0 .. 3) of node i in the current exchange (byte offsets below
-	// 2^32: a uniform base and one 32-bit register)
-	auto word_at = [&](int k, int i) {
+
+	// The diagonal block of the own row.
+	__device__ __forceinline__ void diagonal(double& a00, double& a01, double& a10, double& a11) const {
+		const double* top = V.val + 4 * static_cast<int64_t>(V.diag_blk[row]) - 2 * (row & 63);
+		a00 = top[0];
+		a01 = top[1];
+		a10 = top[2 * kSlice];
+		a11 = top[2 * kSlice + 1];
+	}
+
+	// Addresses are formed anew in every iteration: held in registers they would
+	// push the matrix out.
+	__device__ __forceinline__ void forget_addresses() {
+		asm volatile("" : "+v"(t), "+v"(row));
+	}
+
+	__device__ __forceinline__ bool failed() const {
+		return __builtin_amdgcn_readfirstlane(sh.failed) != 0;
+	}
+
+	// Word k (0 .. 3) of node i in the current exchange (byte offsets below
+	// 2^32: a uniform base and one 32-bit register).
+	__device__ __forceinline__ u64* word_at(int k, int i) const {
 		u64* const base = (ep & 1 ? V.w[2 + k / 2] : V.w[k / 2]) + (k & 1 ? n : 0);
 		return reinterpret_cast<u64*>(reinterpret_cast<char*>(base) + static_cast<uint32_t>(i) * 8u);
-	};
-	auto publish = [&](dbl2 v) {
+	}
+
+	__device__ __forceinline__ void publish(dbl2 v) {
 		ep++;
 		if (shared) {
 			put(word_at(0, row), word_hi(v.x, ep));
@@ -333,9 +358,10 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 			put(word_at(2, row), word_hi(v.y, ep));
 			put(word_at(3, row), word_lo(v.y, ep));
 		}
-	};
-	// the last published vector at node i
-	auto receive = [&](int i) {
+	}
+
+	// The last published vector at node i of another workgroup.
+	__device__ __forceinline__ dbl2 receive(int i) const {
 		u64 q0, q1, q2, q3;
 		uint32_t spin = 0;
 #pragma unroll 1
@@ -354,16 +380,19 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 			}
 		}
 		return dbl2{join(q0, q1), join(q2, q3)};
-	};
-	// halo node k (of the window without the own rows) and its place
-	auto halo_at = [&](int k) { return k < left ? k : k + own; };
+	}
 
-	// Sums v over the cluster (the same value everywhere); meanwhile `work`
-	// runs between the posting of the contribution and the wait for the
-	// others'. set: the LDS arrays used (callers alternate, so that no array is
-	// written while a wave may still read it). NV <= 3.
-	auto gather = [&](auto& v, int set, auto&& work) {
-		constexpr int NV = sizeof(v) / sizeof(double);
+	// Place in the window of its node k without the own rows.
+	__device__ __forceinline__ int halo_at(int k) const {
+		return k < left ? k : k + own;
+	}
+
+	// Sums v over the cluster (the same value everywhere); meanwhile `work` runs
+	// between the posting of the contribution and the wait for the others'.
+	// set: the LDS arrays used (callers alternate, so that no array is written
+	// while a wave may still read it). NV <= 3.
+	template <int NV, typename Work>
+	__device__ __forceinline__ void gather(double (&v)[NV], int set, Work&& work) {
 #pragma unroll
 		for (int k = 0; k < NV; k++) {
 			double const s = wave_total(v[k]);
@@ -446,124 +475,14 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 			}
 			v[k] = uniform(s);
 		}
-	};
-	auto nothing = [] {};
-	auto failed = [&] { return __builtin_amdgcn_readfirstlane(sh.failed) != 0; };
+	}
+	template <int NV>
+	__device__ __forceinline__ void gather(double (&v)[NV], int set) {
+		gather(v, set, [] {});
+	}
 
-	// b - A x of the own row with the FP64 matrix, compensated (row_residual in
-	// pcg.hip); x is published for it
-	dbl2 x = {0, 0}, r = {0, 0}, z = {0, 0}, pn = {0, 0};
-	auto true_residual = [&]() {
-		publish(x);
-		dbl2 res = {0, 0};
-		// the own rows' x through the window, whose directions stay in registers
-		__syncthreads();
-		if (live) {
-			win[row - lo] = x;
-		}
-		__syncthreads();
-		if (live) {
-			dbl2 const bv = ld2(V.b + 2 * static_cast<int64_t>(row));
-			int const end = beg + len * kSlice;
-			double s0 = bv.x, s1 = bv.y, c0 = 0, c1 = 0;
-#pragma unroll 1
-			for (int blk = beg; blk < end; blk += kSlice) {
-				int const c = V.col[blk];
-				int64_t const o = 4 * static_cast<int64_t>(blk) - 2 * r64;
-				dbl2 const a = ld2(V.val + o), d = ld2(V.val + o + 2 * kSlice);
-				dbl2 const xv = c >= r0 && c < r1 ? win[c - lo] : receive(c);
-				sub_exact(s0, c0, a.x, xv.x);
-				sub_exact(s0, c0, a.y, xv.y);
-				sub_exact(s1, c1, d.x, xv.x);
-				sub_exact(s1, c1, d.y, xv.y);
-			}
-			res = dbl2{s0 + c0, s1 + c1};
-		}
-		__syncthreads();
-		if (live) {
-			win[row - lo] = pn;
-		}
-		return res;
-	};
-
-	double beta = 0;
-	int status = 0;
-	for (int k = t; k < nwin; k += NT) {
-		win[k] = mode == 2 ? ld2(V.save + 2 * (static_cast<int64_t>(n) + lo + k)) : dbl2{0, 0};
-	}
-	if (mode == 2) {
-		if (live) {
-			x = ld2(V.x + 2 * static_cast<int64_t>(row));
-			r = ld2(V.save + 2 * static_cast<int64_t>(row));
-			z = precond(r);
-		}
-		beta = R.beta;
-		__syncthreads();
-	} else {
-		__syncthreads();
-		if (live) {
-			if (mode == 1) {
-				x = ld2(V.x + 2 * static_cast<int64_t>(row));
-			} else {
-				r = ld2(V.b + 2 * static_cast<int64_t>(row));
-			}
-		}
-		if (mode == 1) {
-			r = true_residual();
-		}
-		z = precond(r);
-		dbl2 const bv = live ? ld2(V.b + 2 * static_cast<int64_t>(row)) : dbl2{0, 0};
-		double v[3] = {r.x * z.x + r.y * z.y, r.x * r.x + r.y * r.y, bv.x * bv.x + bv.y * bv.y};
-		gather(v, 2, nothing);
-		R.rz = v[0];
-		R.rr = R.rr_true = R.rr_ref = v[1];
-		R.bb = v[2];
-		R.tol2 = uniform(rtol2 * v[2]);
-		R.rr_best = R.pq = 0;
-		R.iter = 0;
-		R.stall = R.checking = R.checks = 0;
-		R.updates = 1;
-		status = failed() ? kFailed : R.rr <= R.tol2 ? 1 : 0;
-	}
-	if (status == 0 && R.iter < stop) {
-		publish(z);
-	}
-	dbl2 hz[kAhead];   // z of this thread's first halo nodes
-	auto halo_first = [&] {
-#pragma unroll
-		for (int u = 0; u < kAhead; u++) {
-			int const k = t + u * NT;
-			if (k < halo) {
-				hz[u] = receive(lo + halo_at(k));
-			}
-		}
-	};
-	if (status == 0 && R.iter < stop) {
-		halo_first();
-	}
-	while (status == 0 && R.iter < stop) {
-		// addresses are formed anew in every iteration: held in registers they
-		// would push the matrix out
-		asm volatile("" : "+v"(t), "+v"(row));
-		// p = z + beta p over the window
-		if (live) {
-			pn = z + beta * win[row - lo];
-			win[row - lo] = pn;
-		}
-#pragma unroll
-		for (int u = 0; u < kAhead; u++) {
-			int const k = t + u * NT;
-			if (k < halo) {
-				int const a = halo_at(k);
-				win[a] = hz[u] + beta * win[a];
-			}
-		}
-		for (int k = t + kAhead * NT; k < halo; k += NT) {
-			int const a = halo_at(k);
-			win[a] = receive(lo + a) + beta * win[a];
-		}
-		__syncthreads();
-		// q = A p
+	// The matrix times the window, own row (two accumulators a component).
+	__device__ __forceinline__ dbl2 multiply() {
 		dbl2 q = {0, 0}, qodd = {0, 0};
 #pragma unroll
 		for (int k = 0; k < (W + 1) / 2; k++) {
@@ -590,12 +509,177 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 			s.x = fma(static_cast<double>(a.y), pv.y, s.x);
 			s.y = fma(static_cast<double>(c.x), pv.x, s.y);
 			s.y = fma(static_cast<double>(c.y), pv.y, s.y);
+			if (NT > 512 && k % 2 == 1) {
+				// the next loads wait for these products: the registers hold the matrix
+				asm volatile("" : "+v"(q.x), "+v"(q.y), "+v"(qodd.x), "+v"(qodd.y)::"memory");
+			}
 		}
-		q += qodd;
+		return q + qodd;
+	}
+
+	// b - A x of the own row with the FP64 matrix, compensated (row_residual in
+	// pcg.hip). x is published for it; the own rows of the window are left
+	// holding keep.
+	__device__ __forceinline__ dbl2 true_residual(dbl2 x, dbl2 keep) {
+		publish(x);
+		dbl2 res = {0, 0};
+		__syncthreads();
+		if (live) {
+			win[row - lo] = x;
+		}
+		__syncthreads();
+		if (live) {
+			dbl2 const bv = ld2(V.b + 2 * static_cast<int64_t>(row));
+			int const r64 = row & 63, beg = V.slice_ptr[row >> 6] + r64, end = V.slice_ptr[(row >> 6) + 1];
+			double s0 = bv.x, s1 = bv.y, c0 = 0, c1 = 0;
+#pragma unroll 1
+			for (int blk = beg; blk < end; blk += kSlice) {
+				int const c = V.col[blk];
+				int64_t const o = 4 * static_cast<int64_t>(blk) - 2 * r64;
+				dbl2 const a = ld2(V.val + o), d = ld2(V.val + o + 2 * kSlice);
+				dbl2 const xv = c >= r0 && c < r1 ? win[c - lo] : receive(c);
+				sub_exact(s0, c0, a.x, xv.x);
+				sub_exact(s0, c0, a.y, xv.y);
+				sub_exact(s1, c1, d.x, xv.x);
+				sub_exact(s1, c1, d.y, xv.y);
+			}
+			res = dbl2{s0 + c0, s1 + c1};
+		}
+		__syncthreads();
+		if (live) {
+			win[row - lo] = keep;
+		}
+		return res;
+	}
+};
+
+// One PCG run, called by all NT threads of workgroup g of G. On return R holds
+// the run's scalars (in every thread) and V.x the solution of the workgroup's
+// rows. lds: the spare blocks and the window. mode 0 starts from x = 0, 1 from
+// the x in V.x, 2 continues a run cut at its limit (R as it was left, r and p in
+// V.save). Runs until R.iter >= stop.
+template <typename MT, int W, int PRE, int NT>
+__device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, double delta2, int64_t stop,
+                        bool final_check, Shared& sh, dbl2* lds, Run& R) {
+	constexpr int kAhead = 1;   // halo nodes a thread reads while it waits for the sums
+	Cluster<MT, W, NT> C(V, sh, g, G, lds);
+	dbl2 dinv0 = {0, 0}, dinv1 = {0, 0};
+	if (C.live) {
+		double a00, a01, a10, a11;
+		C.diagonal(a00, a01, a10, a11);
+		if (PRE == BFMX_PRECOND_JACOBI) {
+			dinv0 = dbl2{1.0 / a00, 1.0 / a11};
+		} else {
+			double const det = a00 * a11 - a01 * a10;
+			dinv0 = dbl2{a11 / det, -a01 / det};
+			dinv1 = dbl2{-a10 / det, a00 / det};
+		}
+	}
+	auto precond = [&](dbl2 r) {
+		if (PRE == BFMX_PRECOND_JACOBI) {
+			return dbl2{dinv0.x * r.x, dinv0.y * r.y};
+		}
+		return dbl2{dinv0.x * r.x + dinv0.y * r.y, dinv1.x * r.x + dinv1.y * r.y};
+	};
+	dbl2 r = {0, 0}, z = {0, 0}, pn = {0, 0};
+	// the own x: in a register, or in this thread's own place in LDS
+	dbl2 xr = {0, 0};
+	dbl2* const xs = lds + spare_bytes<MT, W, NT>() / sizeof(dbl2);
+	auto x_get = [&]() {
+		if constexpr (lds_solution<MT, NT>()) {
+			return xs[C.t];
+		} else {
+			return xr;
+		}
+	};
+	auto x_set = [&](dbl2 v) {
+		if constexpr (lds_solution<MT, NT>()) {
+			xs[C.t] = v;
+		} else {
+			xr = v;
+		}
+	};
+	x_set(dbl2{0, 0});
+	double beta = 0;
+	int status = 0;
+	for (int k = C.t; k < C.nwin; k += NT) {
+		C.win[k] = mode == 2 ? ld2(V.save + 2 * (static_cast<int64_t>(C.n) + C.lo + k)) : dbl2{0, 0};
+	}
+	if (mode == 2) {
+		if (C.live) {
+			x_set(ld2(V.x + 2 * static_cast<int64_t>(C.row)));
+			r = ld2(V.save + 2 * static_cast<int64_t>(C.row));
+			z = precond(r);
+		}
+		beta = R.beta;
+		__syncthreads();
+	} else {
+		__syncthreads();
+		if (C.live) {
+			if (mode == 1) {
+				x_set(ld2(V.x + 2 * static_cast<int64_t>(C.row)));
+			} else {
+				r = ld2(V.b + 2 * static_cast<int64_t>(C.row));
+			}
+		}
+		if (mode == 1) {
+			r = C.true_residual(x_get(), pn);
+		}
+		z = precond(r);
+		dbl2 const bv = C.live ? ld2(V.b + 2 * static_cast<int64_t>(C.row)) : dbl2{0, 0};
+		double v[3] = {r.x * z.x + r.y * z.y, r.x * r.x + r.y * r.y, bv.x * bv.x + bv.y * bv.y};
+		C.gather(v, 2);
+		R.rz = v[0];
+		R.rr = R.rr_true = R.rr_ref = v[1];
+		R.bb = v[2];
+		R.tol2 = uniform(rtol2 * v[2]);
+		R.rr_best = R.pq = 0;
+		R.iter = 0;
+		R.stall = R.checking = R.checks = 0;
+		R.updates = 1;
+		status = C.failed() ? kFailed : R.rr <= R.tol2 ? 1 : 0;
+	}
+	if (status == 0 && R.iter < stop) {
+		C.publish(z);
+	}
+	dbl2 hz[kAhead];   // z of this thread's first halo nodes
+	auto halo_first = [&] {
+#pragma unroll
+		for (int u = 0; u < kAhead; u++) {
+			int const k = C.t + u * NT;
+			if (k < C.halo) {
+				hz[u] = C.receive(C.lo + C.halo_at(k));
+			}
+		}
+	};
+	if (status == 0 && R.iter < stop) {
+		halo_first();
+	}
+	while (status == 0 && R.iter < stop) {
+		C.forget_addresses();
+		// p = z + beta p over the window
+		if (C.live) {
+			pn = z + beta * C.win[C.row - C.lo];
+			C.win[C.row - C.lo] = pn;
+		}
+#pragma unroll
+		for (int u = 0; u < kAhead; u++) {
+			int const k = C.t + u * NT;
+			if (k < C.halo) {
+				int const a = C.halo_at(k);
+				C.win[a] = hz[u] + beta * C.win[a];
+			}
+		}
+		for (int k = C.t + kAhead * NT; k < C.halo; k += NT) {
+			int const a = C.halo_at(k);
+			C.win[a] = C.receive(C.lo + a) + beta * C.win[a];
+		}
+		__syncthreads();
+		dbl2 const q = C.multiply();
 		double v1[1] = {pn.x * q.x + pn.y * q.y};
-		gather(v1, 0, nothing);
+		C.gather(v1, 0);
 		R.pq = v1[0];
-		if (failed()) {
+		if (C.failed()) {
 			status = kFailed;
 			break;
 		}
@@ -604,13 +688,13 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 			break;
 		}
 		double const alpha = uniform(R.rz / v1[0]);
-		x += alpha * pn;
+		x_set(x_get() + alpha * pn);
 		r -= alpha * q;
 		z = precond(r);
-		publish(z);
+		C.publish(z);
 		double v2[2] = {r.x * z.x + r.y * z.y, r.x * r.x + r.y * r.y};
-		gather(v2, 1, halo_first);
-		if (failed()) {
+		C.gather(v2, 1, halo_first);
+		if (C.failed()) {
 			status = kFailed;
 			break;
 		}
@@ -624,11 +708,11 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 		if ((at_tol && !R.checking) || (every && (R.checking || R.rr <= delta2 * R.rr_ref))) {
 			// the true residual replaces the recursive one (the directions are
 			// kept) and decides about the end
-			r = true_residual();
+			r = C.true_residual(x_get(), pn);
 			z = precond(r);
 			double v3[2] = {r.x * z.x + r.y * z.y, r.x * r.x + r.y * r.y};
-			gather(v3, 2, nothing);
-			if (failed()) {
+			C.gather(v3, 2);
+			if (C.failed()) {
 				status = kFailed;
 				break;
 			}
@@ -650,7 +734,7 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 					}
 				}
 				if (status == 0) {
-					publish(z);
+					C.publish(z);
 					halo_first();
 				}
 			}
@@ -658,20 +742,20 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 	}
 	R.beta = beta;
 	if (status == 0 && final_check && R.checks == 0) {
-		dbl2 const rt = true_residual();
+		dbl2 const rt = C.true_residual(x_get(), pn);
 		double v[1] = {rt.x * rt.x + rt.y * rt.y};
-		gather(v, 2, nothing);
+		C.gather(v, 2);
 		R.rr_true = v[0];
-		if (failed()) {
+		if (C.failed()) {
 			status = kFailed;
 		}
 	}
 	R.status = status;
-	if (live) {
-		st2(V.x + 2 * static_cast<int64_t>(row), x);
+	if (C.live) {
+		st2(V.x + 2 * static_cast<int64_t>(C.row), x_get());
 		if (status == 0) {
-			st2(V.save + 2 * static_cast<int64_t>(row), r);
-			st2(V.save + 2 * (static_cast<int64_t>(n) + row), pn);
+			st2(V.save + 2 * static_cast<int64_t>(C.row), r);
+			st2(V.save + 2 * (static_cast<int64_t>(C.n) + C.row), pn);
 		}
 	}
 }

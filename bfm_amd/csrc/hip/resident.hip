@@ -89,9 +89,9 @@ PcgKernel pick(bool mixed, int width, int pre, int nt) {
 	return width <= 7 ? pick_precond<double, 7>(pre, nt) : pick_precond<double, 9>(pre, nt);
 }
 
-// LDS bytes of the row blocks that do not fit the registers.
-int spare(bool mixed, int width, int nt) {
-	return mixed || nt <= 512 ? 0 : width <= 7 ? spare_bytes<double, 7, 1024>() : spare_bytes<double, 9, 1024>();
+// LDS bytes beside the window.
+int fixed(bool mixed, int width, int nt) {
+	return mixed || nt <= 512 ? 0 : width <= 7 ? fixed_bytes<double, 7, 1024>() : fixed_bytes<double, 9, 1024>();
 }
 
 }  // namespace
@@ -146,7 +146,7 @@ int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double d
 	       {words(s->d_r), words(s->d_z), words(s->d_q), words(s->d_p[0])}, words(s->d_p[1]), s->d_dinv, n};
 	int const nt = n <= 512 ? 512 : 1024;
 	PcgKernel const kernel = pick(mixed, s->res_width, precond, nt);
-	size_t const lds = static_cast<size_t>(s->res_window) * sizeof(resident::dbl2) + spare(mixed, s->res_width, nt);
+	size_t const lds = static_cast<size_t>(s->res_window) * sizeof(resident::dbl2) + fixed(mixed, s->res_width, nt);
 	if (lds > 48 * 1024) {
 		BFMX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
 		                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
@@ -195,8 +195,8 @@ int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double d
 // its work: in the streaming kernel, one workgroup a system, the largest one's
 // time on one CU is the least a launch can take.
 // Measured, whole launch with the assembly, block Jacobi to 1e-8: 256 panels of
-// 500 to 4,000 nodes 63.2 -> 16.1 ms, 64 panels of 3,000 to 30,000 nodes 835 ->
-// 85 ms, 512 of 500 to 30,000 1,911 -> 518 ms.
+// 500 to 4,000 nodes 63.2 -> 14.8 ms, 64 panels of 3,000 to 30,000 nodes 835 ->
+// 73 ms, 512 of 500 to 30,000 1,911 -> 466 ms.
 
 namespace resident {
 namespace {
@@ -427,7 +427,7 @@ int plan_create(Plan** out, const std::vector<bfmx_system*>& systems, const std:
 		delete p;
 		return BFMX_OK;
 	}
-	p->lds = static_cast<size_t>(widest) * sizeof(resident::dbl2) + static_cast<size_t>(spare(false, p->width, kRows));
+	p->lds = static_cast<size_t>(widest) * sizeof(resident::dbl2) + static_cast<size_t>(fixed(false, p->width, kRows));
 	std::vector<int32_t> order, groups;
 	std::vector<Queue> queues;
 	std::vector<Member> members;

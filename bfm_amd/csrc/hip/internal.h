@@ -568,6 +568,15 @@ int pcg_in_buffers(bfmx_system* s, PcgBuffers const& w, int precond, double rtol
 // does not fit or the device could not run it. *out: the final scalars.
 int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double delta2, int64_t cap, bool warm,
                  Scalars* out, bool* ran);
+// MINRES of s->d_bsolve the same way (status 0: iteration limit, 1: converged,
+// 2: breakdown, 3: exhausted above rtol).
+struct MinresResult {
+	int status;
+	int64_t iter;
+	double rr, bb;
+	int checks;
+};
+int resident_minres(bfmx_system* s, double rtol, int64_t cap, MinresResult* out, bool* ran);
 // noalloc.hip: bfmx_system_solve_noalloc, and the largest system (nodes) its
 // fixed scratch array holds.
 int solve_noalloc(bfmx_system* s, const double* b_in, double* u_out, int precond, double rtol, size_t max_iter,

@@ -1138,7 +1138,9 @@ namespace {
 // iteration: one SpMV pass (v = y / beta, y' = A v - (beta / beta_old) r1,
 // partial v . y'), one update pass (y' -= (alpha / beta) r2, z = M^-1 y',
 // partial y' . z), the Givens recurrences on the host, and the direction and
-// solution update. The sums are fixed-order per-workgroup partials.
+// solution update. The sums are fixed-order per-workgroup partials. Systems of
+// up to 131,072 nodes that fit the registers run in one launch (run_minres in
+// resident.h) with the recurrences on the device; these kernels take the rest.
 
 __global__ __launch_bounds__(kBlock) void k_mr_diag(int nb, const int32_t* __restrict__ diag_blk,
                                                     const double* __restrict__ val, double* __restrict__ dinv) {
@@ -1301,14 +1303,7 @@ int mr_sums(hipStream_t st, int nwg, const double* partial, double* d_out, doubl
 	return BFMX_OK;
 }
 
-struct MrResult {
-	int status;
-	int64_t iter;
-	double rr, bb;
-	int checks;
-};
-
-int solve_minres(bfmx_system* s, double rtol, int64_t cap, MrResult* res) {
+int solve_minres(bfmx_system* s, double rtol, int64_t cap, MinresResult* res) {
 	int64_t const n = s->n_nodes;
 	int const nb = static_cast<int>(n);
 	int const g = grid(n);
@@ -1518,8 +1513,12 @@ int solve(bfmx_system* s, const double* b_in, int precond, int precision, double
 
 	auto const t0 = std::chrono::steady_clock::now();
 	if (precond == BFMX_PRECOND_MINRES) {
-		MrResult mr{};
-		BFMX_CHECK(solve_minres(s, rtol, cap, &mr));
+		MinresResult mr{};
+		bool ran = false;
+		BFMX_CHECK(resident_minres(s, rtol, cap, &mr, &ran));
+		if (!ran) {
+			BFMX_CHECK(solve_minres(s, rtol, cap, &mr));
+		}
 		auto const t1 = std::chrono::steady_clock::now();
 		int32_t const status = mr.status == 1   ? BFMX_OK
 		                       : mr.status == 2 ? BFMX_E_BREAKDOWN

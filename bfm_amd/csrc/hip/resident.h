@@ -760,12 +760,164 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 	}
 }
 
+// Scalars of a MINRES run, the same in every workgroup (solve_minres in pcg.hip
+// names them).
+struct MinresRun {
+	double oldb, beta, dbar, epsln, phibar, cs, sn, beta1, bb, rr;
+	int64_t iter, next_check;
+	int32_t status;    // 0 running (limit reached), 1 converged, 2 breakdown, 3 exhausted above rtol, kFailed
+	int32_t checks;
+};
+
+// MINRES with the matrix in registers, preconditioned by 1 / |diagonal|: the
+// recurrences of solve_minres (pcg.hip) on the device, in every thread; two
+// all-gathers an iteration where the streaming form has two synchronous
+// read-backs. fresh starts from x = 0; else the run goes on from V.x and the
+// vectors r1, r2, w, w2 in V.save and more (2 n doubles each). Runs until
+// R.iter >= stop; the residual is checked at iteration cap whatever its estimate.
+template <int W, int NT>
+__device__ void run_minres(View const& V, int g, int G, bool fresh, double rtol, int64_t stop, int64_t cap,
+                           double* more, Shared& sh, dbl2* lds, MinresRun& R) {
+	Cluster<double, W, NT> C(V, sh, g, G, lds);
+	int64_t const n2 = 2 * static_cast<int64_t>(C.n);
+	dbl2 dinv = {0, 0};
+	dbl2 x = {0, 0}, r1 = {0, 0}, r2 = {0, 0}, y = {0, 0}, w = {0, 0}, w2 = {0, 0};
+	if (C.live) {
+		double a00, a01, a10, a11;
+		C.diagonal(a00, a01, a10, a11);
+		dinv = dbl2{a00 != 0 ? 1.0 / fabs(a00) : 1.0, a11 != 0 ? 1.0 / fabs(a11) : 1.0};
+		int64_t const i = 2 * static_cast<int64_t>(C.row);
+		if (fresh) {
+			r1 = r2 = ld2(V.b + i);
+		} else {
+			x = ld2(V.x + i);
+			r1 = ld2(V.save + i);
+			r2 = ld2(V.save + n2 + i);
+			w = ld2(more + i);
+			w2 = ld2(more + n2 + i);
+		}
+		y = dinv * r2;
+	}
+	if (fresh) {
+		double v[2] = {r2.x * y.x + r2.y * y.y, r2.x * r2.x + r2.y * r2.y};
+		C.gather(v, 2);
+		R = MinresRun{};
+		R.bb = R.rr = v[1];
+		R.cs = -1;
+		R.beta1 = R.beta = R.phibar = uniform(sqrt(v[0]));
+		if (C.failed()) {
+			R.status = kFailed;
+		} else if (!(v[0] > 0)) {
+			R.status = v[1] == 0 ? 1 : 2;   // b = 0: x = 0; else M is not positive
+		}
+	}
+	double const tol2 = uniform(rtol * rtol * R.bb);
+	dbl2 hy = {0, 0};   // y of this thread's first halo node
+	auto halo_first = [&] {
+		if (C.t < C.halo) {
+			hy = C.receive(C.lo + C.halo_at(C.t));
+		}
+	};
+	bool const runs = R.status == 0 && R.iter < stop;
+	if (runs) {
+		C.publish(y);
+		halo_first();
+	}
+	while (R.status == 0 && R.iter < stop) {
+		C.forget_addresses();
+		if (C.live) {
+			C.win[C.row - C.lo] = y;
+		}
+		if (C.t < C.halo) {
+			C.win[C.halo_at(C.t)] = hy;
+		}
+		for (int k = C.t + NT; k < C.halo; k += NT) {
+			int const a = C.halo_at(k);
+			C.win[a] = C.receive(C.lo + a);
+		}
+		__syncthreads();
+		int64_t const it = R.iter + 1;
+		double const sy = uniform(1.0 / R.beta), sr = it >= 2 ? uniform(R.beta / R.oldb) : 0.0;
+		dbl2 const v = sy * y;
+		dbl2 yn = sy * C.multiply() - sr * r1;
+		double d[1] = {v.x * yn.x + v.y * yn.y};
+		C.gather(d, 0);
+		double const alfa = d[0];
+		yn -= uniform(alfa / R.beta) * r2;
+		y = dinv * yn;
+		C.publish(y);
+		d[0] = yn.x * y.x + yn.y * y.y;
+		C.gather(d, 1, halo_first);
+		if (C.failed()) {
+			R.status = kFailed;
+			break;
+		}
+		R.iter = it;
+		if (!(d[0] >= 0) || !isfinite(alfa)) {
+			R.status = 2;   // the preconditioner is not positive definite, or overflow
+			break;
+		}
+		r1 = r2;
+		r2 = yn;
+		R.oldb = R.beta;
+		R.beta = uniform(sqrt(d[0]));
+		double const oldeps = R.epsln;
+		double const delta = uniform(R.cs * R.dbar + R.sn * alfa);
+		double const gbar = uniform(R.sn * R.dbar - R.cs * alfa);
+		R.epsln = uniform(R.sn * R.beta);
+		R.dbar = uniform(-R.cs * R.beta);
+		double const gamma = uniform(fmax(hypot(gbar, R.beta), 1e-300));
+		R.cs = uniform(gbar / gamma);
+		R.sn = uniform(R.beta / gamma);
+		double const phi = uniform(R.cs * R.phibar);
+		R.phibar = uniform(R.sn * R.phibar);
+		// w_new = (v - oldeps w2 - delta w) / gamma; (w2, w) <- (w, w_new)
+		double const rgamma = uniform(1.0 / gamma);
+		dbl2 const wn = (v - oldeps * w2 - delta * w) * rgamma;
+		w2 = w;
+		w = wn;
+		x += phi * wn;
+		// the M^-1-norm estimate phibar triggers a true residual check
+		if ((R.phibar <= rtol * R.beta1 && it >= R.next_check) || R.beta == 0 || it == cap) {
+			dbl2 const res = C.true_residual(x, y);
+			d[0] = res.x * res.x + res.y * res.y;
+			C.gather(d, 2);
+			if (C.failed()) {
+				R.status = kFailed;
+				break;
+			}
+			R.rr = d[0];
+			R.checks++;
+			R.next_check = it + 10;
+			if (d[0] <= tol2) {
+				R.status = 1;
+			} else if (R.beta == 0) {
+				R.status = 3;   // the Krylov space is exhausted above rtol
+			} else {
+				C.publish(y);
+				halo_first();
+			}
+		}
+	}
+	if (C.live) {
+		int64_t const i = 2 * static_cast<int64_t>(C.row);
+		st2(V.x + i, x);
+		if (R.status == 0) {
+			st2(V.save + i, r1);
+			st2(V.save + n2 + i, r2);
+			st2(more + i, w);
+			st2(more + n2 + i, w2);
+		}
+	}
+}
+
 // Most block rows of a workgroup, one per thread.
 constexpr int kRows = 1024;
 
-// The nodes of the widest window when G workgroups share the system's rows (0:
-// they cannot, or a window or row is too long for the kernels above).
-int window_of(const bfmx_system* s, int64_t G);
+// The nodes of the widest window when G workgroups of at most `threads` rows
+// share the system's (0: they cannot, or a window or row is too long for the
+// kernels above).
+int window_of(const bfmx_system* s, int64_t G, int threads = kRows);
 
 // ---- batches (resident.hip)
 

@@ -173,3 +173,32 @@ def test_batches_of_clusters(monkeypatch, pre):
         one = D.Batch([s])
         one.solve(precond=pre, rtol=1e-8)
         assert np.array_equal(one.get_u(0), u), k
+
+
+@pytest.mark.parametrize("nx,ny,kind", [(3, 2, 3), (16, 5, 4), (40, 10, 4), (42, 11, 3), (51, 9, 4), (60, 14, 4)])
+def test_minres(monkeypatch, nx, ny, kind):
+    """Axisymmetric rings of 12 to 915 nodes (one workgroup of 512, and two) against the recurrences on the host;
+    a run cut into launches is the same run. K is indefinite with a condition number of about 1e5 here: two
+    solutions whose residuals meet 1e-8 agree to 1e-3; seen 1e-9."""
+    m = meshgen.beam(nx, ny, kind=kind, length=4.0, height=1.0, jitter=0.2, seed=12)
+    m.coords = m.coords + np.array([1.0, 0.0])
+    s = D.System.from_mesh(m)
+    s.assemble(D.AXISYMMETRIC, 2.0e11, 0.3, 7850.0, g=(0.0, -9.81))
+    sets = m.node_sets
+    s.apply_conditions([1, 0, 3], [0.0, 0.0, -1e6], [sets["bottom"], sets["left"], sets["top"]])
+    kw = dict(precond=D.PRECOND_MINRES, rtol=1e-8)
+    ref, st_ref, u, st = both(monkeypatch, s, **kw)
+    print(f"{m.n_nodes} nodes: {st_ref['iterations']} / {st['iterations']} iterations, difference {rel_err(u, ref):.1e}")
+    assert abs(st["iterations"] - st_ref["iterations"]) <= 0.1 * st_ref["iterations"] + 10
+    A, b = s.get_csr_scipy(), s.get_rhs()
+    assert st["status"] == 0 and np.linalg.norm(b - A @ u) <= 1.1e-8 * np.linalg.norm(b)
+    assert rel_err(u, ref) <= 1e-3
+    monkeypatch.setenv("BFMX_RESIDENT_ITERS", "7")
+    u2, st2 = s.solve(**kw)
+    assert st2["iterations"] == st["iterations"] and np.array_equal(u, u2)
+    monkeypatch.delenv("BFMX_RESIDENT_ITERS")
+    u0, st0 = s.solve(b=np.zeros(2 * s.n_nodes), **kw)
+    assert st0["iterations"] == 0 and not u0.any()
+    with pytest.raises(D.BfmxError) as e:
+        s.solve(precond=D.PRECOND_MINRES, rtol=1e-8, max_iter=5)
+    assert e.value.code == -5 and "5 iterations" in str(e.value)

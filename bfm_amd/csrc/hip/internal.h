@@ -188,6 +188,7 @@ struct AmgLevel {
 	int n_seg = 1;
 	double* d_dense = nullptr;
 	int64_t n_dense = 0;              // its entries
+	int dense_max = 0;                // rows of the largest inverse
 	int32_t* d_seg_ptr = nullptr;     // n_seg + 1 row offsets
 	int32_t* d_seg_row = nullptr;     // segment of each row
 	int64_t* d_seg_off = nullptr;     // first entry of each segment's inverse

@@ -345,16 +345,8 @@ int bfmx_system_get_u(bfmx_system_t* s, double* u) {
 		set_error(!u ? "null output" : "no solution available");
 		return BFMX_E_ARG;
 	}
-	return guarded([&]() -> int {
-		int64_t const n = s->n_nodes;
-		std::vector<double> v(2 * n);
-		BFMX_HIP(hipMemcpy(v.data(), s->d_x, v.size() * sizeof(double), hipMemcpyDeviceToHost));
-		for (int64_t i = 0; i < n; i++) {
-			u[2 * i] = v[2 * s->perm[i]];
-			u[2 * i + 1] = v[2 * s->perm[i] + 1];
-		}
-		return BFMX_OK;
-	});
+	// d_q holds nothing between solves
+	return guarded([&] { return vector_out(s, s->d_x, s->stream, s->d_q, u); });
 }
 
 int bfmx_system_get_entry(bfmx_system_t* s, size_t i, size_t j, double* out) {

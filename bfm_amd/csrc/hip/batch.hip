@@ -604,6 +604,7 @@ struct bfmx_batch {
 	int32_t* d_order_all = nullptr;         // all systems largest first (one launch for equal picks)
 	double* d_work = nullptr;
 	std::vector<bfmx::BatchOut> h_out;
+	std::vector<double*> h_x, h_q;          // each system's solution and scratch on the device
 	struct Exec {
 		hipGraphExec_t exec;
 		int pre;
@@ -755,6 +756,10 @@ int finish_create(bfmx_batch* b, const std::vector<BatchInst>& h) {
 	std::vector<int32_t> order_all(n);
 	std::iota(order_all.begin(), order_all.end(), 0);
 	std::stable_sort(order_all.begin(), order_all.end(), [&](int32_t a, int32_t c) { return h[a].n > h[c].n; });
+	for (auto const& I : h) {
+		b->h_x.push_back(I.x);
+		b->h_q.push_back(I.q);
+	}
 	BFMX_CHECK(dalloc(&b->d_inst, n));
 	BFMX_CHECK(dalloc(&b->d_out, n));
 	BFMX_CHECK(dalloc(&b->d_order, n));
@@ -1657,17 +1662,9 @@ int batch_get_u(bfmx_batch* b, size_t k, double* u) {
 		set_error("no system %zu in the batch", k);
 		return BFMX_E_ARG;
 	}
-	bfmx_system* s = b->systems[k];
-	int64_t const n = s->n_nodes;
-	std::vector<BatchInst> h(1);
-	BFMX_HIP(hipMemcpy(h.data(), b->d_inst + k, sizeof(BatchInst), hipMemcpyDeviceToHost));
-	std::vector<double> v(2 * n);
-	BFMX_HIP(hipMemcpy(v.data(), h[0].x, v.size() * sizeof(double), hipMemcpyDeviceToHost));
-	for (int64_t i = 0; i < n; i++) {
-		u[2 * i] = v[2 * s->perm[i]];
-		u[2 * i + 1] = v[2 * s->perm[i] + 1];
-	}
-	return BFMX_OK;
+	BFMX_HIP(hipSetDevice(b->device));
+	// q is scratch between launches
+	return vector_out(b->systems[k], b->h_x[k], b->stream, b->h_q[k], u);
 }
 
 }  // namespace bfmx

@@ -348,6 +348,7 @@ struct bfmx_system {
 	double* d_dinv = nullptr;        // 4 per node (block inverse) or 2 per node (point)
 	double* d_partial = nullptr;     // per-workgroup partial sums
 	int64_t partial_cap = 0;         // their number
+	int32_t* d_perm = nullptr;       // perm on the device (large systems, on demand)
 	bfmx::Scalars* d_scal = nullptr;
 	bfmx::Scalars* h_scal = nullptr; // pinned host mirror ring (4 entries)
 	hipEvent_t ev[6] = {};
@@ -563,6 +564,20 @@ struct PcgBuffers {
 // graph capture); *out receives the final scalars, the solution stays in
 // w.x (internal node order). The system's own solver buffers are untouched.
 int pcg_in_buffers(bfmx_system* s, PcgBuffers const& w, int precond, double rtol, int64_t cap, Scalars* out);
+// Vectors between the callers' DOF order and the internal node order. From
+// kDevicePerm nodes on the reordering runs on the device and the copy goes
+// straight from or to the caller's memory: at 1,002,501 nodes a load in took 1.9
+// ms and a solution out 3.0 ms through a reordered host copy, 0.6 and 1.2 ms on
+// the device; below, the host's loop over a pinned copy takes less than the launch
+// (5,124 nodes: 0.06 ms).
+constexpr int64_t kDevicePerm = 16384;
+void launch_to_internal(hipStream_t st, int64_t n, const int32_t* perm, const double* original, double* internal);
+void launch_to_original(hipStream_t st, int64_t n, const int32_t* perm, const double* internal, double* original);
+int ensure_perm(bfmx_system* s, hipStream_t st);   // s->d_perm, complete on return
+// d_v (internal order) to out (the caller's), on stream st; d_stage: 2 n
+// doubles of device memory whose contents are not needed (null: the host
+// reorders).
+int vector_out(bfmx_system* s, const double* d_v, hipStream_t st, double* d_stage, double* out);
 // resident.hip: point or block Jacobi PCG of s->d_bsolve in the solver's
 // buffers, with the matrix held in registers, from x = 0 or (warm) from
 // s->d_x; *ran is false (and nothing but the buffers changed) when the system
@@ -622,8 +637,10 @@ void pool_free_bytes(void* p);
 // A pinned (device-visible) host buffer of at least `bytes`, one per host
 // thread and slot (0 .. kStagingSlots - 1), grown as needed and kept until
 // the process ends; valid until the thread's next call for the same slot.
-// Slots of the multigrid build: 0 a level's graph, 1 counts read back.
-constexpr int kStagingSlots = 2;
+// Slots: 0 a level's graph and 1 counts read back (the multigrid build), 2 a
+// small system's load or solution.
+constexpr int kStagingSlots = 3;
+constexpr int kVectorSlot = 2;
 int pinned_staging(void** p, size_t bytes, int slot = 0);
 
 // Small pinned host blocks from a process-wide cache (pool.hip); a block goes

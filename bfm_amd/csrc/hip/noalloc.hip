@@ -79,28 +79,6 @@ struct Layout {
 	}
 };
 
-// bsolve[2 perm[i] + c] = stage[2 i + c] (perm[old] = new).
-__global__ __launch_bounds__(kBlock) void k_perm_in(int64_t n, const int32_t* __restrict__ perm,
-                                                    const double* __restrict__ stage, double* __restrict__ bsolve) {
-	int64_t const i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-	if (i < n) {
-		int64_t const k = perm[i];
-		bsolve[2 * k] = stage[2 * i];
-		bsolve[2 * k + 1] = stage[2 * i + 1];
-	}
-}
-
-// stage[2 i + c] = x[2 perm[i] + c].
-__global__ __launch_bounds__(kBlock) void k_perm_out(int64_t n, const int32_t* __restrict__ perm,
-                                                     const double* __restrict__ x, double* __restrict__ stage) {
-	int64_t const i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-	if (i < n) {
-		int64_t const k = perm[i];
-		stage[2 * i] = x[2 * k];
-		stage[2 * i + 1] = x[2 * k + 1];
-	}
-}
-
 }  // namespace
 
 int64_t noalloc_max_nodes() {
@@ -139,11 +117,10 @@ int solve_noalloc(bfmx_system* s, const double* b_in, double* u_out, int precond
 	int32_t* perm = reinterpret_cast<int32_t*>(base + L.perm);
 	double* stage = at(L.stage);
 	hipStream_t const st = s->stream;
-	int const g = static_cast<int>((n + kBlock - 1) / kBlock);
 	BFMX_HIP(hipMemcpyAsync(perm, s->perm.data(), n * sizeof(int32_t), hipMemcpyHostToDevice, st));
 	if (b_in) {
 		BFMX_HIP(hipMemcpyAsync(stage, b_in, 2 * n * sizeof(double), hipMemcpyHostToDevice, st));
-		k_perm_in<<<g, kBlock, 0, st>>>(n, perm, stage, w.bsolve);
+		launch_to_internal(st, n, perm, stage, w.bsolve);
 	} else {
 		BFMX_HIP(hipMemcpyAsync(w.bsolve, s->d_b, 2 * n * sizeof(double), hipMemcpyDeviceToDevice, st));
 	}
@@ -156,7 +133,7 @@ int solve_noalloc(bfmx_system* s, const double* b_in, double* u_out, int precond
 	                       : last.done == 3 ? BFMX_E_STAGNATION
 	                                        : BFMX_E_MAXITER;
 	if (u_out && (status == BFMX_OK || status == BFMX_E_MAXITER)) {
-		k_perm_out<<<g, kBlock, 0, st>>>(n, perm, w.x, stage);
+		launch_to_original(st, n, perm, w.x, stage);
 		BFMX_HIP(hipGetLastError());
 		BFMX_HIP(hipMemcpyAsync(u_out, stage, 2 * n * sizeof(double), hipMemcpyDeviceToHost, st));
 		BFMX_HIP(hipStreamSynchronize(st));

@@ -48,6 +48,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstdlib>
+#include <mutex>
 
 #include "resident.h"
 
@@ -741,6 +742,26 @@ int grid(int64_t n) {
 	return static_cast<int>((n + kBlock - 1) / kBlock);
 }
 
+// internal[2 perm[i] + c] = original[2 i + c] (perm[old] = new).
+__global__ __launch_bounds__(kBlock) void k_to_internal(int64_t n, const int32_t* __restrict__ perm,
+                                                        const double* __restrict__ original,
+                                                        double* __restrict__ internal) {
+	int64_t const i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+	if (i < n) {
+		st2(internal + 2 * static_cast<int64_t>(perm[i]), ld2(original + 2 * i));
+	}
+}
+
+// original[2 i + c] = internal[2 perm[i] + c].
+__global__ __launch_bounds__(kBlock) void k_to_original(int64_t n, const int32_t* __restrict__ perm,
+                                                        const double* __restrict__ internal,
+                                                        double* __restrict__ original) {
+	int64_t const i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+	if (i < n) {
+		st2(original + 2 * i, ld2(internal + 2 * static_cast<int64_t>(perm[i])));
+	}
+}
+
 int ensure_workspace(bfmx_system* s) {
 	int64_t const n = s->n_nodes;
 	if (s->d_x) {
@@ -1082,6 +1103,57 @@ int run_chunks(bfmx_system* s, int precond, bool mixed, double rtol2, int64_t ca
 
 }  // namespace
 
+void launch_to_internal(hipStream_t st, int64_t n, const int32_t* perm, const double* original, double* internal) {
+	k_to_internal<<<grid(n), kBlock, 0, st>>>(n, perm, original, internal);
+}
+
+void launch_to_original(hipStream_t st, int64_t n, const int32_t* perm, const double* internal, double* original) {
+	k_to_original<<<grid(n), kBlock, 0, st>>>(n, perm, internal, original);
+}
+
+int ensure_perm(bfmx_system* s, hipStream_t st) {
+	// batches on several threads may hold the same system
+	static std::mutex m;
+	std::lock_guard<std::mutex> lock(m);
+	if (!s->d_perm) {
+		int32_t* d = nullptr;
+		BFMX_CHECK(palloc(&d, static_cast<size_t>(s->n_nodes)));
+		BFMX_HIP(hipMemcpyAsync(d, s->perm.data(), s->perm.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
+		BFMX_HIP(hipStreamSynchronize(st));   // complete for every stream that reads it
+		s->d_perm = d;
+	}
+	return BFMX_OK;
+}
+
+int vector_out(bfmx_system* s, const double* d_v, hipStream_t st, double* d_stage, double* out) {
+	int64_t const n = s->n_nodes;
+	if (n >= kDevicePerm && d_stage) {
+		BFMX_CHECK(ensure_perm(s, st));
+		launch_to_original(st, n, s->d_perm, d_v, d_stage);
+		BFMX_HIP(hipGetLastError());
+		BFMX_HIP(hipMemcpyAsync(out, d_stage, 2 * n * sizeof(double), hipMemcpyDeviceToHost, st));
+		BFMX_HIP(hipStreamSynchronize(st));
+		return BFMX_OK;
+	}
+	void* pinned = nullptr;
+	std::vector<double> pageable;
+	double* v = nullptr;
+	if (n < kDevicePerm) {
+		BFMX_CHECK(pinned_staging(&pinned, 2 * n * sizeof(double), kVectorSlot));
+		v = static_cast<double*>(pinned);
+	} else {
+		pageable.resize(2 * n);
+		v = pageable.data();
+	}
+	BFMX_HIP(hipMemcpyAsync(v, d_v, 2 * n * sizeof(double), hipMemcpyDeviceToHost, st));
+	BFMX_HIP(hipStreamSynchronize(st));
+	for (int64_t i = 0; i < n; i++) {
+		out[2 * i] = v[2 * s->perm[i]];
+		out[2 * i + 1] = v[2 * s->perm[i] + 1];
+	}
+	return BFMX_OK;
+}
+
 void drop_graphs(bfmx_system* s, int precond) {
 	(void) hipStreamSynchronize(s->stream);
 	auto keep = s->graphs.begin();
@@ -1119,6 +1191,7 @@ void release_solver(bfmx_system* s) {
 	pfree(s->d_dinv);
 	pfree(s->d_partial);
 	pfree(s->d_scal);
+	pfree(s->d_perm);
 	pfree(s->d_val32);
 	pinned_small_free(s->h_scal, 4 * sizeof(Scalars));
 	s->h_scal = nullptr;
@@ -1498,13 +1571,21 @@ int solve(bfmx_system* s, const double* b_in, int precond, int precision, double
 	if (learned) {
 		BFMX_CHECK(mpnn_prepare(s));
 	}
-	if (b_in) {
-		std::vector<double> bp(2 * n);
+	if (b_in && n >= kDevicePerm) {
+		BFMX_CHECK(ensure_perm(s, st));
+		BFMX_HIP(hipMemcpyAsync(s->d_q, b_in, 2 * n * sizeof(double), hipMemcpyHostToDevice, st));
+		launch_to_internal(st, n, s->d_perm, s->d_q, s->d_bsolve);
+		BFMX_HIP(hipGetLastError());
+		BFMX_HIP(hipStreamSynchronize(st));   // the caller's array is read by here on every way out
+	} else if (b_in) {
+		void* pinned = nullptr;
+		BFMX_CHECK(pinned_staging(&pinned, 2 * n * sizeof(double), kVectorSlot));
+		double* const bp = static_cast<double*>(pinned);
 		for (int64_t i = 0; i < n; i++) {
 			bp[2 * s->perm[i]] = b_in[2 * i];
 			bp[2 * s->perm[i] + 1] = b_in[2 * i + 1];
 		}
-		BFMX_HIP(hipMemcpyAsync(s->d_bsolve, bp.data(), 2 * n * sizeof(double), hipMemcpyHostToDevice, st));
+		BFMX_HIP(hipMemcpyAsync(s->d_bsolve, bp, 2 * n * sizeof(double), hipMemcpyHostToDevice, st));
 		BFMX_HIP(hipStreamSynchronize(st));
 	} else {
 		BFMX_HIP(hipMemcpyAsync(s->d_bsolve, s->d_b, 2 * n * sizeof(double), hipMemcpyDeviceToDevice, st));

@@ -1143,11 +1143,8 @@ int solve_resident(bfmx_batch* b, int pre, double rtol2, int64_t max_iter, const
 	}
 	BFMX_HIP(hipEventRecord(b->ev[0], b->stream));
 	launch_assemble(b);
-	bool launched = false;
-	BFMX_CHECK(resident::plan_launch(b->plan, b->stream, pre, rtol2, max_iter, b->d_out, &launched));
-	if (!launched) {
-		return BFMX_OK;
-	}
+	resident::ClusterLock const lock(b->device);
+	BFMX_CHECK(resident::plan_launch(b->plan, b->stream, pre, rtol2, max_iter, b->d_out));
 	const int32_t* at = b->d_rest;
 	for (int c = kClasses - 1; c >= 0; c--) {
 		if (b->rest_count[c] > 0) {

@@ -30,11 +30,17 @@
 // Every workgroup forms the same sums in the same order, so all of them take
 // the same branches; the result does not depend on scheduling.
 //
-// The workgroups of a cluster must be resident together: launches are
-// cooperative, and every wait is bounded (kSpinLimit polls), so that each
-// workgroup ends whatever happens; the caller then solves with the streaming
-// kernels.
+// The workgroups of a cluster must be resident together. A launch has at most
+// one workgroup a CU, kernels on other streams end and leave their CUs to it,
+// and clusters that could wait for each other's CUs do not run at once: a host
+// thread holds the device's ClusterLock from their launch to their end (an
+// ordinary launch under the lock costs 11 us with its synchronization, a
+// cooperative one 20 us). Between processes nothing prevents that, so every
+// wait is bounded (kSpinLimit polls): each workgroup ends whatever happens, and
+// the caller then solves with the streaming kernels.
 #pragma once
+
+#include <mutex>
 
 #include "internal.h"
 
@@ -914,6 +920,19 @@ __device__ void run_minres(View const& V, int g, int G, bool fresh, double rtol,
 // Most block rows of a workgroup, one per thread.
 constexpr int kRows = 1024;
 
+// Compute units of a device: the most workgroups of a launch of clusters.
+int compute_units(int device);
+
+// One thread at a time launches clusters of several workgroups on a device; it
+// holds this until they have ended (its stream drained).
+class ClusterLock {
+public:
+	explicit ClusterLock(int device);
+
+private:
+	std::unique_lock<std::mutex> m_lock;
+};
+
 // The nodes of the widest window when G workgroups of at most `threads` rows
 // share the system's (0: they cannot, or a window or row is too long for the
 // kernels above).
@@ -938,10 +957,9 @@ int plan_create(Plan** out, const std::vector<bfmx_system*>& systems, const std:
 void plan_destroy(Plan* p);
 // Systems the plan does not take, largest first.
 const std::vector<int32_t>& plan_rest(const Plan* p);
-// Queues the runs of the plan's systems; *launched is false when the device
-// refused (the streaming kernel then takes them all). A system whose status is
-// kFailed afterwards was not solved.
-int plan_launch(Plan* p, hipStream_t st, int precond, double rtol2, int64_t max_iter, Out* d_out, bool* launched);
+// Queues the runs of the plan's systems (the caller holds a ClusterLock until
+// st is drained). A system whose status is kFailed afterwards was not solved.
+int plan_launch(Plan* p, hipStream_t st, int precond, double rtol2, int64_t max_iter, Out* d_out);
 
 }  // namespace resident
 }  // namespace bfmx

@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <optional>
 
 #include "resident.h"
 
@@ -98,6 +99,16 @@ int fixed(bool mixed, int width, int nt) {
 
 namespace resident {
 
+int compute_units(int device) {
+	int cus = 0;
+	return hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess ? cus : 0;
+}
+
+ClusterLock::ClusterLock(int device) {
+	static std::mutex m[64];   // of the devices; two that share one only wait for each other
+	m_lock = std::unique_lock<std::mutex>(m[device & 63]);
+}
+
 int window_of(const bfmx_system* s, int64_t G, int threads) {
 	int64_t const n = s->n_nodes;
 	if (n == 0 || G > kMaxGroup || (n + G - 1) / G > threads) {
@@ -131,9 +142,12 @@ int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double d
 	}
 	if (s->res_groups < 0) {
 		int64_t const groups = (s->n_nodes + kRows - 1) / kRows;
-		s->res_window = window_of(s, groups);
-		s->res_groups = s->res_window > 0 ? static_cast<int>(groups) : 0;
-		s->res_width = *std::max_element(s->row_len.begin(), s->row_len.end());
+		s->res_window = groups <= compute_units(s->device) ? window_of(s, groups) : 0;
+		s->res_groups = 0;
+		if (s->res_window > 0) {
+			s->res_groups = static_cast<int>(groups);
+			s->res_width = *std::max_element(s->row_len.begin(), s->row_len.end());
+		}
 	}
 	int const G = s->res_groups;
 	if (G == 0) {
@@ -158,20 +172,13 @@ int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double d
 	int mode = warm ? 1 : 0;
 	cap = (cap + kCheckEvery - 1) / kCheckEvery * kCheckEvery;
 	while (true) {
-		int64_t stop = std::min(cap, (mode == 2 ? out->iter : 0) + per_launch);
+		int64_t const stop = std::min(cap, (mode == 2 ? out->iter : 0) + per_launch);
+		std::optional<ClusterLock> lock;
 		if (G > 1) {
+			lock.emplace(s->device);
 			k_clear<<<static_cast<int>((2 * n + kBlock - 1) / kBlock), kBlock, 0, st>>>(V, 2 * n, nslots);
-			Scalars* S = s->d_scal;
-			void* args[] = {&V, &mode, &rtol2, &delta2, &stop, &S};
-			hipError_t const err = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kernel), dim3(G), dim3(nt),
-			                                                  args, static_cast<unsigned>(lds), st);
-			if (err != hipSuccess) {
-				(void) hipGetLastError();
-				return BFMX_OK;   // the device cannot hold the cluster: the streaming kernels
-			}
-		} else {
-			kernel<<<1, nt, lds, st>>>(V, mode, rtol2, delta2, stop, s->d_scal);
 		}
+		kernel<<<G, nt, lds, st>>>(V, mode, rtol2, delta2, stop, s->d_scal);
 		BFMX_HIP(hipGetLastError());
 		BFMX_HIP(hipMemcpyAsync(out, s->d_scal, sizeof(Scalars), hipMemcpyDeviceToHost, st));
 		BFMX_HIP(hipStreamSynchronize(st));
@@ -221,7 +228,7 @@ int resident_minres(bfmx_system* s, double rtol, int64_t cap, MinresResult* out,
 	*ran = false;
 	const char* e = std::getenv("BFMX_RESIDENT");
 	int64_t const n = s->n_nodes, G = (n + kMinresThreads - 1) / kMinresThreads;
-	int const win = e && e[0] == '0' ? 0 : window_of(s, G, kMinresThreads);
+	int const win = (e && e[0] == '0') || G > compute_units(s->device) ? 0 : window_of(s, G, kMinresThreads);
 	if (win == 0) {
 		return BFMX_OK;
 	}
@@ -245,22 +252,14 @@ int resident_minres(bfmx_system* s, double rtol, int64_t cap, MinresResult* out,
 		const char* cut = std::getenv("BFMX_RESIDENT_ITERS");
 		int64_t const per_launch = cut && std::atoll(cut) > 0 ? std::atoll(cut) : kPerLaunch;
 		for (int fresh = 1; R.status == 0 && (fresh || R.iter < cap); fresh = 0) {
-			int64_t stop = std::min(cap, R.iter + per_launch);
+			int64_t const stop = std::min(cap, R.iter + per_launch);
+			std::optional<ClusterLock> lock;
 			if (G > 1) {
+				lock.emplace(s->device);
 				k_clear<<<static_cast<int>((2 * n + kBlock - 1) / kBlock), kBlock, 0, st>>>(V, 2 * n,
 				                                                                         2 * G * kSlotWords);
-				void* args[] = {&V, &fresh, &rtol, &stop, &cap, &more, &d_run};
-				hipError_t const err = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kernel),
-				                                                  dim3(static_cast<unsigned>(G)), dim3(kMinresThreads),
-				                                                  args, static_cast<unsigned>(lds), st);
-				if (err != hipSuccess) {
-					(void) hipGetLastError();
-					R.status = kFailed;
-					return BFMX_OK;
-				}
-			} else {
-				kernel<<<1, kMinresThreads, lds, st>>>(V, fresh, rtol, stop, cap, more, d_run);
 			}
+			kernel<<<static_cast<unsigned>(G), kMinresThreads, lds, st>>>(V, fresh, rtol, stop, cap, more, d_run);
 			BFMX_HIP(hipGetLastError());
 			BFMX_HIP(hipMemcpyAsync(&R, d_run, sizeof R, hipMemcpyDeviceToHost, st));
 			BFMX_HIP(hipStreamSynchronize(st));
@@ -481,9 +480,9 @@ const std::vector<int32_t>& plan_rest(const Plan* p) {
 int plan_create(Plan** out, const std::vector<bfmx_system*>& systems, const std::vector<View>& views,
                 hipStream_t st) {
 	*out = nullptr;
-	int dev = 0, cus = 0;
+	int dev = 0;
 	BFMX_HIP(hipGetDevice(&dev));
-	BFMX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+	int const cus = compute_units(dev);
 	std::vector<int32_t> by_size(systems.size());
 	for (size_t k = 0; k < by_size.size(); k++) {
 		by_size[k] = static_cast<int32_t>(k);
@@ -583,8 +582,7 @@ int plan_create(Plan** out, const std::vector<bfmx_system*>& systems, const std:
 	return BFMX_OK;
 }
 
-int plan_launch(Plan* p, hipStream_t st, int precond, double rtol2, int64_t max_iter, Out* d_out, bool* launched) {
-	*launched = false;
+int plan_launch(Plan* p, hipStream_t st, int precond, double rtol2, int64_t max_iter, Out* d_out) {
 	bool const point = precond == BFMX_PRECOND_JACOBI;
 	auto const kernel = p->width <= 7
 	                        ? (point ? k_resident_batch<7, BFMX_PRECOND_JACOBI> : k_resident_batch<7, BFMX_PRECOND_BLOCK_JACOBI>)
@@ -595,20 +593,10 @@ int plan_launch(Plan* p, hipStream_t st, int precond, double rtol2, int64_t max_
 	                                                   p->d_post, p->clusters);
 	BFMX_HIP(hipGetLastError());
 	for (auto const& L : p->launches) {
-		const View* views = p->d_views;
-		const int32_t* order = p->d_order;
-		const Member* members = p->d_members + L.first;
-		Queue* queues = p->d_queues;
-		u64* post = p->d_post;
-		void* args[] = {&views, &order, &members, &queues, &post, &rtol2, &max_iter, &d_out};
-		hipError_t const err = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kernel), dim3(L.blocks),
-		                                                  dim3(kRows), args, static_cast<unsigned>(p->lds), st);
-		if (err != hipSuccess) {
-			(void) hipGetLastError();
-			return BFMX_OK;
-		}
+		kernel<<<L.blocks, kRows, p->lds, st>>>(p->d_views, p->d_order, p->d_members + L.first, p->d_queues, p->d_post,
+		                                        rtol2, max_iter, d_out);
+		BFMX_HIP(hipGetLastError());
 	}
-	*launched = true;
 	return BFMX_OK;
 }
 

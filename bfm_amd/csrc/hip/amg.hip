@@ -1919,24 +1919,50 @@ __device__ __forceinline__ double dense_row(int row, int lane, const int32_t* __
 }
 
 // x = A^-1 b with the dense inverses of the coarsest's segments, one
-// wavefront per row.
+// wavefront per row. With one segment (ONE) the row's place follows from the
+// arguments: its first loads need no lookup and are in flight with the done
+// flag (251,251 nodes, 132 rows at the end: 12.7 us in one workgroup, 4.4 here).
 constexpr int kDenseRowsPerBlock = kBlock / 64;
 
-template <int BS, typename BT>
+template <int BS, typename BT, bool ONE>
 __global__ __launch_bounds__(kBlock) void k_dense_solve(int n, const int32_t* __restrict__ seg_ptr,
                                                         const int32_t* __restrict__ seg_row,
                                                         const int64_t* __restrict__ seg_off,
                                                         const double* __restrict__ Ainv, const BT* __restrict__ b,
                                                         float* __restrict__ x, const Scalars* __restrict__ S) {
-	if (S->done) {
-		return;
-	}
 	int const row = blockIdx.x * kDenseRowsPerBlock + (threadIdx.x >> 6);
 	int const lane = threadIdx.x & 63;
-	if (row >= n) {
-		return;   // whole wavefronts leave together
+	if (!ONE) {
+		if (S->done || row >= n) {
+			return;   // whole wavefronts leave together
+		}
+		double const acc = dense_row<BS, BT>(row, lane, seg_ptr, seg_row, seg_off, Ainv, b);
+		if (lane == 0) {
+			x[row] = static_cast<float>(acc);
+		}
+		return;
 	}
-	double const acc = dense_row<BS, BT>(row, lane, seg_ptr, seg_row, seg_off, Ainv, b);
+	constexpr int kEach = 3;   // 192 rows: what coarsening ends at
+	const double* const Ar = Ainv + static_cast<int64_t>(min(row, n - 1)) * n;
+	double a[kEach], v[kEach];
+#pragma unroll
+	for (int u = 0; u < kEach; u++) {
+		int const j = lane + 64 * u, jc = min(j, n - 1);
+		a[u] = Ar[jc];
+		v[u] = j < n ? static_cast<double>(b[jc]) : 0.0;
+	}
+	if (done_after(S, a[0], a[1], a[2]) || row >= n) {
+		return;
+	}
+	double acc = 0;
+#pragma unroll
+	for (int u = 0; u < kEach; u++) {
+		acc += a[u] * v[u];
+	}
+	for (int j = lane + 64 * kEach; j < n; j += 64) {
+		acc += Ar[j] * static_cast<double>(b[j]);
+	}
+	acc = wave_sum(acc);
 	if (lane == 0) {
 		x[row] = static_cast<float>(acc);
 	}
@@ -2070,6 +2096,304 @@ __global__ __launch_bounds__(kWg) void k_coarse_cycle(const AmgLevelDesc* __rest
 #pragma unroll
 	for (int j = 0; j < kPfPerThread; j++) {
 		asm volatile("" ::"v"(touched[j]));
+	}
+}
+
+// The cycle of one small level above a dense coarsest, the usual end of a
+// hierarchy (a level's rows are an eighth or ninth of the level's above it, and
+// coarsening ends at 64 rows). What bounds such a cycle is its chain of
+// dependent loads, so all of it is loaded once at the start, in parallel: a
+// row's blocks in the registers of its quad (lane q of the four takes blocks q,
+// q + 4, ...; kKeepBlocks of them, the rest of a longer row is read each time),
+// its entries of P and R as well. The vectors live in LDS and registers, and
+// each pass costs LDS latency and a barrier. The dense product splits a column
+// over as many threads as there are. The same operations as the passes above,
+// summed by quads. Measured, 132 and 16 rows (1,105 nodes): 16.5 us in
+// k_coarse_cycle, 11.5 here; 165 and 20 rows (1,002,501 nodes): 23.7 and 12.6.
+struct CoarseTwo {
+	int nb, nc, deg, n_seg;
+	const int32_t* slice_ptr;
+	const int32_t* col;
+	const float* val32;
+	const float* dinv;
+	const double* scal;
+	const float* b;
+	float* x;              // the correction
+	const int32_t* rptr;
+	const int32_t* rrow;
+	const float* R;
+	const int32_t* pptr;
+	const int32_t* pcol;
+	const float* P;
+	const double* inv;
+	const int32_t* seg_ptr;
+	const int32_t* seg_row;
+	const int64_t* seg_off;
+	int64_t n_dense;
+};
+
+constexpr int kKeepBlocks = 3;    // a lane's, so rows of up to 12 blocks
+constexpr int kKeepR = 2;         // entries of a coarse row's column a lane keeps
+constexpr int kTouch = 3;         // lines of the inverse each thread brings into L2
+static_assert(4 * kWgRows <= kWg, "a quad a row");
+
+__device__ __forceinline__ float quad_sum(float v) {
+	v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));
+	v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));
+	return v;
+}
+
+__global__ __launch_bounds__(kWg) void k_coarse_two(CoarseTwo L, const Scalars* __restrict__ S) {
+	__shared__ float xs[2][3 * kWgRows], rs[3 * kWgRows], bc[3 * kWgRows], xc[3 * kWgRows];
+	__shared__ float coef[2 * kMaxDeg + 1];
+	__shared__ double part[kWg];
+	int const t = threadIdx.x, q = t & 3, i = min(t >> 2, L.nb - 1), r = i & 63;
+	bool const live = (t >> 2) < L.nb;
+	int const lane = t % kRestrictLanes, J0 = t / kRestrictLanes, Jc = min(J0, L.nc - 1);
+	int32_t const beg = L.slice_ptr[i >> 6], end = L.slice_ptr[(i >> 6) + 1];
+	int32_t const e0 = L.pptr[i], e1 = L.pptr[i + 1], t0 = L.rptr[Jc], t1 = L.rptr[Jc + 1];
+	float b[3];
+#pragma unroll
+	for (int a = 0; a < 3; a++) {
+		b[a] = L.b[3 * i + a];
+	}
+	if (done_after(S, beg, end, e0, e1, t0, t1, b[0])) {
+		return;
+	}
+	// everything the cycle reads, in flight together
+	float A[kKeepBlocks][3][3], Dinv[9], Pe[9], Re[kKeepR][9];
+	int32_t at[kKeepBlocks], pj = 0, ri[kKeepR] = {};
+#pragma unroll
+	for (int u = 0; u < kKeepBlocks; u++) {
+		int32_t const blk = beg + r + kSlice * (q + 4 * u);
+		bool const in = blk < end;
+		at[u] = in ? L.col[blk] : i;
+		if (in) {
+			ld_block<3>(L.val32, blk, r, A[u]);
+		} else {
+#pragma unroll
+			for (int a = 0; a < 9; a++) {
+				A[u][a / 3][a % 3] = 0;
+			}
+		}
+	}
+#pragma unroll
+	for (int a = 0; a < 9; a++) {
+		Dinv[a] = L.dinv[9 * i + a];
+		Pe[a] = 0;
+	}
+	if (e0 + q < e1) {
+		pj = L.pcol[e0 + q];
+#pragma unroll
+		for (int a = 0; a < 9; a++) {
+			Pe[a] = L.P[9 * static_cast<int64_t>(e0 + q) + a];
+		}
+	}
+#pragma unroll
+	for (int u = 0; u < kKeepR; u++) {
+		int32_t const e = t0 + lane + kRestrictLanes * u;
+		bool const in = J0 < L.nc && e < t1;
+		ri[u] = in ? L.rrow[e] : 0;
+#pragma unroll
+		for (int a = 0; a < 9; a++) {
+			Re[u][a] = in ? L.R[9 * static_cast<int64_t>(e) + a] : 0;
+		}
+	}
+	uint32_t touched[kTouch];
+#pragma unroll
+	for (int u = 0; u < kTouch; u++) {
+		int64_t const at8 = static_cast<int64_t>(t + kWg * u) * (kPfLine / 8);
+		touched[u] = at8 < L.n_dense ? *reinterpret_cast<const uint32_t*>(L.inv + at8) : 0;
+	}
+	if (t <= 2 * kMaxDeg) {
+		coef[t] = static_cast<float>(L.scal[t]);
+	}
+	float const first = static_cast<float>(L.scal[2]);
+
+	// sum of the row's blocks times x, in every lane of the quad
+	auto multiply = [&](const float* x, float (&acc)[3]) {
+#pragma unroll
+		for (int a = 0; a < 3; a++) {
+			acc[a] = 0;
+		}
+#pragma unroll
+		for (int u = 0; u < kKeepBlocks; u++) {
+#pragma unroll
+			for (int k = 0; k < 3; k++) {
+				float const xv = x[3 * at[u] + k];
+#pragma unroll
+				for (int a = 0; a < 3; a++) {
+					acc[a] += A[u][a][k] * xv;
+				}
+			}
+		}
+		for (int32_t blk = beg + r + kSlice * (q + 4 * kKeepBlocks); blk < end; blk += 4 * kSlice) {
+			int32_t const c = L.col[blk];
+			float M[3][3];
+			ld_block<3>(L.val32, blk, r, M);
+#pragma unroll
+			for (int k = 0; k < 3; k++) {
+				float const xv = x[3 * c + k];
+#pragma unroll
+				for (int a = 0; a < 3; a++) {
+					acc[a] += M[a][k] * xv;
+				}
+			}
+		}
+#pragma unroll
+		for (int a = 0; a < 3; a++) {
+			acc[a] = quad_sum(acc[a]);
+		}
+	};
+	float x[3], d[3];
+	// d = c1 d + c2 D^-1 (b - A x), x += d; c1 is not used at a first step
+	auto step = [&](const float (&res)[3], bool begin, float c1, float c2) {
+#pragma unroll
+		for (int a = 0; a < 3; a++) {
+			float z = 0;
+#pragma unroll
+			for (int k = 0; k < 3; k++) {
+				z += Dinv[3 * a + k] * res[k];
+			}
+			d[a] = begin ? c2 * z : c1 * d[a] + c2 * z;
+			x[a] += d[a];
+		}
+	};
+	auto put = [&](float* to) {
+		if (live && q < 3) {
+			to[3 * i + q] = q == 0 ? x[0] : q == 1 ? x[1] : x[2];
+		}
+	};
+	x[0] = x[1] = x[2] = 0;
+	step(b, true, 0, first);
+	int cur = 0;
+	put(xs[cur]);
+	__syncthreads();
+	float acc[3], res[3];
+	for (int k = 1; k < L.deg; k++) {
+		multiply(xs[cur], acc);
+#pragma unroll
+		for (int a = 0; a < 3; a++) {
+			res[a] = b[a] - acc[a];
+		}
+		step(res, false, coef[1 + 2 * k], coef[2 + 2 * k]);
+		cur ^= 1;
+		put(xs[cur]);
+		__syncthreads();
+	}
+	multiply(xs[cur], acc);
+	if (live && q < 3) {
+		rs[3 * i + q] = q == 0 ? b[0] - acc[0] : q == 1 ? b[1] - acc[1] : b[2] - acc[2];
+	}
+	__syncthreads();
+	// restriction: kRestrictLanes lanes a coarse row
+	for (int J = J0; J - J0 < L.nc; J += kWg / kRestrictLanes) {
+		bool const kept = J == J0, in = J < L.nc;
+		float s3[3] = {0, 0, 0};
+		auto add = [&](int32_t row, const float (&p)[9]) {
+#pragma unroll
+			for (int k = 0; k < 3; k++) {
+#pragma unroll
+				for (int c = 0; c < 3; c++) {
+					s3[c] += p[3 * k + c] * rs[3 * row + k];
+				}
+			}
+		};
+		if (kept) {
+#pragma unroll
+			for (int u = 0; u < kKeepR; u++) {
+				add(ri[u], Re[u]);
+			}
+		}
+		int32_t const u0 = kept ? t0 : in ? L.rptr[J] : 0, u1 = !in ? 0 : kept ? t1 : L.rptr[J + 1];
+		for (int32_t e = u0 + lane + (kept ? kKeepR * kRestrictLanes : 0); e < u1; e += kRestrictLanes) {
+			float p[9];
+#pragma unroll
+			for (int a = 0; a < 9; a++) {
+				p[a] = L.R[9 * static_cast<int64_t>(e) + a];
+			}
+			add(L.rrow[e], p);
+		}
+#pragma unroll
+		for (int c = 0; c < 3; c++) {
+#pragma unroll
+			for (int off = kRestrictLanes / 2; off > 0; off >>= 1) {
+				s3[c] += __shfl_xor(s3[c], off, 64);
+			}
+		}
+		if (in && lane < 3) {
+			bc[3 * J + lane] = lane == 0 ? s3[0] : lane == 1 ? s3[1] : s3[2];
+		}
+	}
+	__syncthreads();
+	// the touched values themselves are not needed: this keeps their loads
+#pragma unroll
+	for (int u = 0; u < kTouch; u++) {
+		asm volatile("" ::"v"(touched[u]));
+	}
+	// the dense inverses: thread (g, row) sums every parts-th column
+	int const n = 3 * L.nc, parts = kWg / n, row = t % n, g = t / n;
+	if (g < parts) {
+		int base = 0, len = n;
+		int64_t off = 0;
+		if (L.n_seg > 1) {
+			int const sg = L.seg_row[row / 3];
+			base = 3 * L.seg_ptr[sg];
+			len = 3 * L.seg_ptr[sg + 1] - base;
+			off = L.seg_off[sg];
+		}
+		// the inverse is symmetric: read across its columns, coalesced
+		const double* const col = L.inv + off + (row - base);
+		double sum = 0;
+#pragma unroll 4
+		for (int j = g; j < len; j += parts) {
+			sum += col[static_cast<int64_t>(j) * len] * static_cast<double>(bc[base + j]);
+		}
+		part[t] = sum;
+	}
+	__syncthreads();
+	if (t < n) {
+		double sum = 0;
+		for (int k = 0; k < parts; k++) {
+			sum += part[k * n + t];
+		}
+		xc[t] = static_cast<float>(sum);
+	}
+	__syncthreads();
+	// x += P x_c
+	float px[3];
+#pragma unroll
+	for (int k = 0; k < 3; k++) {
+		px[k] = Pe[3 * k] * xc[3 * pj] + Pe[3 * k + 1] * xc[3 * pj + 1] + Pe[3 * k + 2] * xc[3 * pj + 2];
+	}
+	for (int32_t e = e0 + q + 4; e < e1; e += 4) {
+		int32_t const J = L.pcol[e];
+		const float* const p = L.P + 9 * static_cast<int64_t>(e);
+#pragma unroll
+		for (int k = 0; k < 3; k++) {
+			px[k] += p[3 * k] * xc[3 * J] + p[3 * k + 1] * xc[3 * J + 1] + p[3 * k + 2] * xc[3 * J + 2];
+		}
+	}
+#pragma unroll
+	for (int k = 0; k < 3; k++) {
+		x[k] += quad_sum(px[k]);
+	}
+	put(xs[cur]);
+	__syncthreads();
+	for (int k = 0; k < L.deg; k++) {
+		multiply(xs[cur], acc);
+#pragma unroll
+		for (int a = 0; a < 3; a++) {
+			res[a] = b[a] - acc[a];
+		}
+		step(res, k == 0, coef[1 + 2 * k], coef[2 + 2 * k]);
+		cur ^= 1;
+		if (k + 1 == L.deg) {
+			put(L.x);
+		} else {
+			put(xs[cur]);
+			__syncthreads();
+		}
 	}
 }
 
@@ -3472,7 +3796,9 @@ int amg_build_impl(bfmx_system* s, bool device) {
 			std::fprintf(stderr, "multigrid coarsest: %d segments, largest %d rows, %s\n", Lc.n_seg, seg_largest(fseg),
 			             Lc.d_dense ? "dense inverses" : "Chebyshev iteration");
 		}
-		// the small coarse levels run in one workgroup
+		// the small coarse levels run in one workgroup: k_coarse_two where
+		// there is one above a dense coarsest; a dense coarsest alone is spread
+		// over the grid; k_coarse_cycle takes the other ends
 		s->amg_wg = -1;
 		for (size_t l = 1; l < lv.size(); l++) {
 			if (lv[l].nb <= kWgRows) {
@@ -3480,7 +3806,11 @@ int amg_build_impl(bfmx_system* s, bool device) {
 				break;
 			}
 		}
-		if (s->amg_wg > 0) {
+		size_t const small = s->amg_wg > 0 ? lv.size() - s->amg_wg : 0;
+		if (small == 1 && lv.back().d_dense) {
+			s->amg_wg = -1;
+		}
+		if (s->amg_wg > 0 && !(small == 2 && lv.back().d_dense)) {
 			std::vector<AmgLevelDesc> desc;
 			for (size_t l = s->amg_wg; l < lv.size(); l++) {
 				AmgLevel const& L = lv[l];
@@ -3761,14 +4091,22 @@ float* vcycle(bfmx_system* s, size_t l, const BT* b, const double* q, double* pa
 		// b is this level's own d_b (restricted into it); the workgroup cycle
 		// runs every level from here down
 		int const nl = static_cast<int>(s->amg.size() - l);
+		if (!s->d_amg_desc) {
+			AmgLevel const& C = s->amg[l + 1];
+			CoarseTwo const two{L.nb, C.nb, level_deg(s->amg_par, l), C.n_seg, L.d_slice_ptr, L.d_col, L.d_val32,
+			                    L.d_dinv, L.d_scal, L.d_b, L.d_x[1], L.d_rptr, L.d_rrow, L.d_R, L.d_pptr, L.d_pcol,
+			                    L.d_P, C.d_dense, C.d_seg_ptr, C.d_seg_row, C.d_seg_off, C.n_dense};
+			k_coarse_two<<<1, kWg, 0, st>>>(two, S);
+			return L.d_x[1];
+		}
 		k_coarse_cycle<<<1, kWg, 0, st>>>(s->d_amg_desc, nl, s->d_amg_pf, s->amg_npf, S);
 		return nl == 1 && L.d_dense ? L.d_x[0] : L.d_x[1];
 	}
 	if (coarsest && L.d_dense) {
 		int const n = BS * L.nb;
 		int const g = (n + kDenseRowsPerBlock - 1) / kDenseRowsPerBlock;
-		k_dense_solve<BS, BT><<<g, kBlock, 0, st>>>(n, L.d_seg_ptr, L.d_seg_row, L.d_seg_off, L.d_dense, b, L.d_x[0],
-		                                            S);
+		(L.n_seg == 1 ? k_dense_solve<BS, BT, true> : k_dense_solve<BS, BT, false>)<<<g, kBlock, 0, st>>>(
+		    n, L.d_seg_ptr, L.d_seg_row, L.d_seg_off, L.d_dense, b, L.d_x[0], S);
 		if (q) {
 			k_dot_partials<<<grid(n), kBlock, 0, st>>>(n, L.d_x[0], q, partial, S);
 		}

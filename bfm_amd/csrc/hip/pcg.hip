@@ -49,6 +49,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <mutex>
+#include <type_traits>
 
 #include "resident.h"
 
@@ -234,6 +235,44 @@ __device__ __forceinline__ bool reduce_live(const double* __restrict__ partial, 
 	return true;
 }
 
+// The sums of at most kFoldMax workgroups' partials, in every thread of each
+// workgroup of the kernel that needs them: a reduction kernel less (4 us and a
+// launch's gap), for some 1.5 us at the start of its consumer. Every workgroup
+// sums in the same order, so all have the same bits. The line is where each
+// workgroup's share of the partials still is four loads a thread; together they
+// read 8 MB from L2 there, 16 times that at 1,002,501 nodes.
+// Measured, microseconds an iteration of flexible CG: 1,105 nodes with the
+// multigrid 44.7 -> 41.5, 40,501 with the network as well 234 -> 226, 251,251
+// with the multigrid 233 -> 229.
+constexpr int kFoldMax = 4 * kBlock;
+
+template <int NV>
+__device__ __forceinline__ void fold_partials(const double* __restrict__ partial, int n, double (&tot)[NV]) {
+	__shared__ double lds[NV][kBlock / 64];
+	double v[NV][kFoldMax / kBlock];
+#pragma unroll
+	for (int k = 0; k < NV; k++) {
+#pragma unroll
+		for (int u = 0; u < kFoldMax / kBlock; u++) {
+			int const i = threadIdx.x + u * kBlock;
+			v[k][u] = i < n ? partial[k * n + i] : 0.0;
+		}
+	}
+#pragma unroll
+	for (int k = 0; k < NV; k++) {
+		double const sum = wave_sum((v[k][0] + v[k][1]) + (v[k][2] + v[k][3]));
+		if ((threadIdx.x & 63) == 0) {
+			lds[k][threadIdx.x >> 6] = sum;
+		}
+	}
+	__syncthreads();
+#pragma unroll
+	for (int k = 0; k < NV; k++) {
+		tot[k] = (lds[k][0] + lds[k][1]) + (lds[k][2] + lds[k][3]);
+	}
+}
+static_assert(kBlock == 256 && kFoldMax == 4 * kBlock, "fold_partials sums four by four");
+
 // z = M^-1 r for one node.
 template <int PRE>
 __device__ __forceinline__ dbl2 apply_precond(const double* __restrict__ dinv, int i, dbl2 r) {
@@ -398,22 +437,28 @@ __global__ __launch_bounds__(kRed) void k_red_fcg_beta(int nwg, const double* __
 // V-cycle, FP64 from the learned preconditioner), q = A p_new with the FP64
 // matrix, partials p_new . q and p_new . r.
 // SEG: a segmented flexible CG (beta of the row's segment, partial sums kept
-// apart per segment).
+// apart per segment). FOLD: beta from the nz partials of z . q at `dots`
+// (fold_partials) instead of S->beta.
 #ifdef BFMX_FCG_WAVES
 #define BFMX_FCG_ATTR __attribute__((amdgpu_waves_per_eu(BFMX_FCG_WAVES, BFMX_FCG_WAVES)))
 #else
 #define BFMX_FCG_ATTR
 #endif
-template <typename ZT, bool SEG = false>
+template <typename ZT, bool SEG = false, bool FOLD = false>
 __global__ __launch_bounds__(kBlock) BFMX_FCG_ATTR void k_fcg_spmv(int nb, const int32_t* __restrict__ slice_ptr,
                                                      const int32_t* __restrict__ col,
                                                      const double* __restrict__ val, const ZT* __restrict__ z,
                                                      double* __restrict__ p0, double* __restrict__ p1,
                                                      double* __restrict__ q, const double* __restrict__ r,
                                                      double* __restrict__ partial, const Scalars* __restrict__ S,
-                                                     SegView sv = SegView{}, const double* __restrict__ seg_scal = nullptr) {
+                                                     SegView sv = SegView{}, const double* __restrict__ seg_scal = nullptr,
+                                                     const double* __restrict__ dots = nullptr, int nz = 0) {
 	if (S->done) {
 		return;
+	}
+	double zq[1] = {0};
+	if (FOLD) {
+		fold_partials<1>(dots, nz, zq);
 	}
 	// the two direction buffers alternate with the count of iterations run
 	// (the iterations a hold skips do not switch them)
@@ -422,7 +467,9 @@ __global__ __launch_bounds__(kBlock) BFMX_FCG_ATTR void k_fcg_spmv(int nb, const
 	double* __restrict__ pnew = odd ? p0 : p1;
 	int const blk = xcd_remap(blockIdx.x, gridDim.x);
 	bool const second = SEG && static_cast<int>(threadIdx.x) >= sv.split[blk];
-	double const beta = SEG ? seg_scal[3 * sv.seg[2 * blk + second] + 1] : S->beta;
+	double const beta = SEG    ? seg_scal[3 * sv.seg[2 * blk + second] + 1]
+	                    : FOLD ? (S->pq > 0 ? -zq[0] / S->pq : 0.0)
+	                           : S->beta;
 	int const row = blk * kBlock + threadIdx.x;
 	auto ldz = [&](int c) {
 		if constexpr (sizeof(ZT) == 4) {
@@ -512,20 +559,39 @@ __global__ __launch_bounds__(kRed) void k_red_fcg_alpha(int nwg, const double* _
 	}
 }
 
-// x += alpha p, r -= alpha q, partials r . r.
-template <bool SEG = false>
+// x += alpha p, r -= alpha q, partials r . r. FOLD: what k_red_fcg_alpha does,
+// in every workgroup from the partials of k_fcg_spmv at `dots` (the first one
+// keeps p . q and a breakdown in *S, which the others do not need).
+template <bool SEG = false, bool FOLD = false>
 __global__ __launch_bounds__(kBlock) void k_fcg_update(int nb, const double* __restrict__ p0,
                                                        const double* __restrict__ p1, const double* __restrict__ q,
                                                        double* __restrict__ x, double* __restrict__ r,
-                                                       double* __restrict__ partial, const Scalars* __restrict__ S,
+                                                       double* __restrict__ partial, Scalars* __restrict__ S,
                                                        SegView sv = SegView{},
-                                                       const double* __restrict__ seg_scal = nullptr) {
+                                                       const double* __restrict__ seg_scal = nullptr,
+                                                       const double* __restrict__ dots = nullptr) {
 	if (S->done) {
 		return;
 	}
+	double folded = 0;
+	if (FOLD) {
+		double tot[2];
+		fold_partials<2>(dots, gridDim.x, tot);
+		bool const ok = tot[0] > 0 && isfinite(tot[0]);
+		if (blockIdx.x == 0 && threadIdx.x == 0) {
+			S->pq = tot[0];
+			if (!ok) {
+				S->done = 2;
+			}
+		}
+		if (!ok) {
+			return;
+		}
+		folded = tot[1] / tot[0];
+	}
 	const double* __restrict__ p = (S->iter & 1) ? p0 : p1;   // the direction k_fcg_spmv wrote
 	bool const second = SEG && static_cast<int>(threadIdx.x) >= sv.split[blockIdx.x];
-	double const alpha = SEG ? seg_scal[3 * sv.seg[2 * blockIdx.x + second]] : S->alpha;
+	double const alpha = SEG ? seg_scal[3 * sv.seg[2 * blockIdx.x + second]] : FOLD ? folded : S->alpha;
 	int const i = blockIdx.x * kBlock + threadIdx.x;
 	double v[1] = {0};
 	if (i < nb) {
@@ -777,8 +843,9 @@ int ensure_workspace(bfmx_system* s) {
 	BFMX_CHECK(palloc(&s->d_p[1], 2 * n));
 	BFMX_CHECK(palloc(&s->d_dinv, 4 * n));
 	// per-workgroup partial sums: three per 256-row workgroup (the residual
-	// kernel), one per 64-row workgroup (the learned preconditioner's decoder)
-	s->partial_cap = std::max<int64_t>(3 * static_cast<int64_t>(grid(n)), (n + 63) / 64);
+	// kernel), one per 64-row workgroup (the learned preconditioner's decoder);
+	// three of each workgroup where flexible CG folds them (launch_fcg_iteration)
+	s->partial_cap = std::max<int64_t>({3 * static_cast<int64_t>(grid(n)), (n + 63) / 64, 3 * kFoldMax});
 	BFMX_CHECK(palloc(&s->d_partial, static_cast<size_t>(s->partial_cap)));
 	BFMX_CHECK(palloc(&s->d_scal, 1));
 	BFMX_CHECK(pinned_small_alloc(reinterpret_cast<void**>(&s->h_scal), 4 * sizeof(Scalars)));
@@ -878,11 +945,27 @@ void launch_fcg_iteration(bfmx_system* s, int pre) {
 		k_red_fcg_rr<<<1, kRed, 0, s->stream>>>(g, s->d_partial, s->d_scal);
 		return;
 	}
-	if (pre == BFMX_PRECOND_AMG) {
-		float* z = amg_vcycle(s, s->d_r, s->d_q, s->d_partial, s->d_scal, &nwz);
+	// p . q and p . r go behind the partials of z . q where both are folded
+	double* const dots = s->d_partial + kFoldMax;
+	auto direction = [&](auto* z) {
+		typedef std::remove_pointer_t<decltype(z)> ZT;
+		if (nwz <= kFoldMax && g <= kFoldMax) {
+			k_fcg_spmv<ZT, false, true><<<g, kBlock, 0, s->stream>>>(
+			    nb, s->d_slice_ptr, s->d_col, s->d_val, z, s->d_p[0], s->d_p[1], s->d_q, s->d_r, dots, s->d_scal,
+			    SegView{}, nullptr, s->d_partial, nwz);
+			k_fcg_update<false, true><<<g, kBlock, 0, s->stream>>>(nb, s->d_p[0], s->d_p[1], s->d_q, s->d_x, s->d_r,
+			                                                       s->d_partial, s->d_scal, SegView{}, nullptr, dots);
+			return;
+		}
 		k_red_fcg_beta<<<1, kRed, 0, s->stream>>>(nwz, s->d_partial, s->d_scal);
-		k_fcg_spmv<float><<<g, kBlock, 0, s->stream>>>(nb, s->d_slice_ptr, s->d_col, s->d_val, z, s->d_p[0],
-		                                               s->d_p[1], s->d_q, s->d_r, s->d_partial, s->d_scal);
+		k_fcg_spmv<ZT><<<g, kBlock, 0, s->stream>>>(nb, s->d_slice_ptr, s->d_col, s->d_val, z, s->d_p[0], s->d_p[1],
+		                                            s->d_q, s->d_r, s->d_partial, s->d_scal);
+		k_red_fcg_alpha<<<1, kRed, 0, s->stream>>>(g, s->d_partial, s->d_scal);
+		k_fcg_update<false><<<g, kBlock, 0, s->stream>>>(nb, s->d_p[0], s->d_p[1], s->d_q, s->d_x, s->d_r,
+		                                                 s->d_partial, s->d_scal);
+	};
+	if (pre == BFMX_PRECOND_AMG) {
+		direction(amg_vcycle(s, s->d_r, s->d_q, s->d_partial, s->d_scal, &nwz));
 	} else {
 		// the learned network's correction added to block Jacobi, or to the
 		// multigrid V-cycle (its dot partials are not needed: z . q comes
@@ -891,14 +974,8 @@ void launch_fcg_iteration(bfmx_system* s, int pre) {
 		const float* base = pre == BFMX_PRECOND_AMG_LEARNED
 		                        ? amg_vcycle(s, s->d_r, nullptr, nullptr, s->d_scal, &nwv)
 		                        : nullptr;
-		double* z = mpnn_apply(s, s->d_r, s->d_q, s->d_partial, s->d_scal, &nwz, base);
-		k_red_fcg_beta<<<1, kRed, 0, s->stream>>>(nwz, s->d_partial, s->d_scal);
-		k_fcg_spmv<double><<<g, kBlock, 0, s->stream>>>(nb, s->d_slice_ptr, s->d_col, s->d_val, z, s->d_p[0],
-		                                                s->d_p[1], s->d_q, s->d_r, s->d_partial, s->d_scal);
+		direction(mpnn_apply(s, s->d_r, s->d_q, s->d_partial, s->d_scal, &nwz, base));
 	}
-	k_red_fcg_alpha<<<1, kRed, 0, s->stream>>>(g, s->d_partial, s->d_scal);
-	k_fcg_update<false><<<g, kBlock, 0, s->stream>>>(nb, s->d_p[0], s->d_p[1], s->d_q, s->d_x, s->d_r, s->d_partial,
-	                                                 s->d_scal);
 	k_red_fcg_rr<<<1, kRed, 0, s->stream>>>(g, s->d_partial, s->d_scal);
 }
 

@@ -175,17 +175,35 @@ __device__ __forceinline__ void gather16(int64_t i, int64_t b, int B, int g, con
 	int32_t const beg = slice_ptr[i >> 6] + r;
 	int const len = row_len[i];
 	// three neighbours' loads in flight together (a learned solve on the
-	// 2M-DOF beam: 141 -> 126 ms; two: 136 ms, four: 134 ms)
-#pragma unroll 3
-	for (int k = 0; k < len; k++) {
-		int64_t const blk = beg + k * kSlice;
-		int64_t const j = col[blk];
-		float const w = val32[blk_at(blk, r, a, bb)] * si * feat[8 * j + 5];
-		float v[16];
-		ld16(T + (j * B + b) * kH + 16 * g, v);
+	// 2M-DOF beam: 141 -> 126 ms; two: 136 ms, four: 134 ms), and with them the
+	// next three's columns, so that a group waits once for memory and not once
+	// for its columns and again for their rows. Past the row's end the own row
+	// is read with weight 0.
+	constexpr int kTogether = 3;
+	int32_t j[kTogether];
 #pragma unroll
-		for (int c = 0; c < 16; c++) {
-			acc[c] += w * v[c];
+	for (int u = 0; u < kTogether; u++) {
+		j[u] = u < len ? col[beg + u * kSlice] : static_cast<int32_t>(i);
+	}
+	for (int k = 0; k < len; k += kTogether) {
+		int32_t next[kTogether];
+		float w[kTogether], v[kTogether][16];
+#pragma unroll
+		for (int u = 0; u < kTogether; u++) {
+			int const kn = k + kTogether + u;
+			next[u] = kn < len ? col[beg + kn * kSlice] : static_cast<int32_t>(i);
+			bool const in = k + u < len;
+			int64_t const blk = beg + (in ? k + u : 0) * kSlice;
+			w[u] = in ? val32[blk_at(blk, r, a, bb)] * si * feat[8 * static_cast<int64_t>(j[u]) + 5] : 0.f;
+			ld16(T + (static_cast<int64_t>(j[u]) * B + b) * kH + 16 * g, v[u]);
+		}
+#pragma unroll
+		for (int u = 0; u < kTogether; u++) {
+#pragma unroll
+			for (int c = 0; c < 16; c++) {
+				acc[c] += w[u] * v[u][c];
+			}
+			j[u] = next[u];
 		}
 	}
 }
@@ -257,7 +275,7 @@ __global__ __launch_bounds__(kWG) void k_encode(int64_t R, int B, const RT* __re
 		W0[k] = params[kOffW0 + k];
 	}
 	__syncthreads();
-	int64_t const rg = static_cast<int64_t>(blockIdx.x) * kWG + threadIdx.x;
+	int64_t const rg = static_cast<int64_t>(xcd_remap(blockIdx.x, gridDim.x)) * kWG + threadIdx.x;
 	if (rg >= R) {
 		return;
 	}
@@ -321,7 +339,7 @@ __global__ __launch_bounds__(kWG) void k_layer(int64_t R, int B, const int32_t* 
 		*reinterpret_cast<u16x8*>(&Ws[n][8 * k8]) = *reinterpret_cast<const u16x8*>(Wt + n * 2 * kH + 8 * k8);
 	}
 	int const t = threadIdx.x, row = t >> 2, g = t & 3;
-	int64_t const rg = static_cast<int64_t>(blockIdx.x) * kT + row;
+	int64_t const tile = static_cast<int64_t>(xcd_remap(blockIdx.x, gridDim.x)) * kT, rg = tile + row;
 	float self[16], acc[16];
 #pragma unroll
 	for (int c = 0; c < 16; c++) {
@@ -367,7 +385,7 @@ __global__ __launch_bounds__(kWG) void k_layer(int64_t R, int B, const int32_t* 
 	if constexpr (kSplit) {
 #pragma unroll
 		for (int q = 0; q < 4; q++) {
-			int64_t const ro = static_cast<int64_t>(blockIdx.x) * kT + 16 * w + 4 * lq + q;
+			int64_t const ro = tile + 16 * w + 4 * lq + q;
 			if (ro < R) {
 #pragma unroll
 				for (int nb = 0; nb < 4; nb++) {
@@ -419,7 +437,7 @@ __global__ __launch_bounds__(kWG) void k_adjoint(int64_t R, int B, const int32_t
 		*reinterpret_cast<u16x8*>(&Ws[n][8 * k8]) = *reinterpret_cast<const u16x8*>(W + n * kH + 8 * k8);
 	}
 	int const t = threadIdx.x, row = t >> 2, g = t & 3;
-	int64_t const rg = static_cast<int64_t>(blockIdx.x) * kT + row;
+	int64_t const tile = static_cast<int64_t>(xcd_remap(blockIdx.x, gridDim.x)) * kT, rg = tile + row;
 	float a[16];
 #pragma unroll
 	for (int c = 0; c < 16; c++) {
@@ -461,7 +479,7 @@ __global__ __launch_bounds__(kWG) void k_adjoint(int64_t R, int B, const int32_t
 	if constexpr (kSplit) {
 #pragma unroll
 		for (int q = 0; q < 4; q++) {
-			int64_t const ro = static_cast<int64_t>(blockIdx.x) * kT + 16 * w + 4 * lq + q;
+			int64_t const ro = tile + 16 * w + 4 * lq + q;
 			if (ro < R) {
 #pragma unroll
 				for (int nb = 0; nb < 8; nb++) {
@@ -520,7 +538,7 @@ __global__ __launch_bounds__(kWG) void k_decode(int64_t R, int B, const RT* __re
 	}
 	__syncthreads();
 	int const t = threadIdx.x, rr = t >> 2, g = t & 3;
-	int64_t const rg = static_cast<int64_t>(blockIdx.x) * kT + rr;
+	int64_t const rg = static_cast<int64_t>(xcd_remap(blockIdx.x, gridDim.x)) * kT + rr;
 	float u0 = 0.f, u1 = 0.f;
 	if (rg < R) {
 		int64_t const i = rg / B;
@@ -583,7 +601,7 @@ __global__ __launch_bounds__(kWG) void k_loss(int64_t R, int B, const int32_t* _
                                               const float* __restrict__ z, const float* __restrict__ e,
                                               int64_t pstride, const float* __restrict__ den, float* __restrict__ gout,
                                               double* __restrict__ partial) {
-	int64_t const rg = static_cast<int64_t>(blockIdx.x) * kWG + threadIdx.x;
+	int64_t const rg = static_cast<int64_t>(xcd_remap(blockIdx.x, gridDim.x)) * kWG + threadIdx.x;
 	double lv = 0;
 	if (rg < R) {
 		int64_t const i = rg / B;
@@ -731,31 +749,15 @@ __global__ __launch_bounds__(kWG) void k_agg_bwd(int64_t R, int B, const int32_t
                                                  const float* __restrict__ feat, const float* __restrict__ dM,
                                                  float* __restrict__ dHin) {
 	int const t = threadIdx.x, row = t >> 2, g = t & 3;
-	int64_t const rg = static_cast<int64_t>(blockIdx.x) * kT + row;
+	int64_t const rg = static_cast<int64_t>(xcd_remap(blockIdx.x, gridDim.x)) * kT + row;
 	if (rg >= R) {
 		return;
 	}
 	int64_t const j = rg / B;
 	int64_t const b = rg - j * B;
-	int const r = static_cast<int>(j & 63), a = g & 1, bb = g >> 1;
-	float const sj = feat[8 * j + 5];
-	int32_t const beg = slice_ptr[j >> 6] + r;
-	int const len = row_len[j];
 	float acc[16];
-#pragma unroll
-	for (int c = 0; c < 16; c++) {
-		acc[c] = dHin[rg * kH + 16 * g + c];
-	}
-	for (int k = 0; k < len; k++) {
-		int64_t const blk = beg + k * kSlice;
-		int64_t const i = col[blk];
-		float const wgt = val32[blk_at(blk, r, a, bb)] * sj * feat[8 * i + 5];
-		const float* dmi = dM + (i * B + b) * kH + 16 * g;
-#pragma unroll
-		for (int c = 0; c < 16; c++) {
-			acc[c] += wgt * dmi[c];
-		}
-	}
+	ld16(dHin + rg * kH + 16 * g, acc);
+	gather16<true>(j, b, B, g, slice_ptr, row_len, col, val32, feat, dM, acc);
 #pragma unroll
 	for (int c = 0; c < 16; c++) {
 		dHin[rg * kH + 16 * g + c] = acc[c];

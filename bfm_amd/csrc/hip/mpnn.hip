@@ -159,26 +159,25 @@ __device__ __forceinline__ void split16(u16* hi, u16* lo, const float (&v)[16]) 
 	*reinterpret_cast<u16x8*>(lo + 8) = l1;
 }
 
-// acc[c] += sum over the neighbours k of node i (row slot order) of
-// w_ik T[(k B + b) H + 16 g + c], w_ik = entry (a, b') of block (i, k) times
-// isd_i isd_k with (a, b') = (g / 2, g % 2), or (g % 2, g / 2) when TR (the
-// adjoint: for the symmetric A, entry (a, b') of block (k, i) is entry
-// (b', a) of block (i, k)).
-template <bool TR, typename AT>
-__device__ __forceinline__ void gather16(int64_t i, int64_t b, int B, int g, const int32_t* __restrict__ slice_ptr,
-                                         const int32_t* __restrict__ row_len, const int32_t* __restrict__ col,
-                                         const float* __restrict__ val32, const float* __restrict__ feat,
-                                         const AT* __restrict__ T, float (&acc)[16]) {
+// add(w_ik, load(k)) for the neighbours k of node i in row slot order; w_ik =
+// entry (a, b') of block (i, k) times isd_i isd_k with (a, b') = (g / 2, g % 2),
+// or (g % 2, g / 2) when TR (the adjoint: for the symmetric A, entry (a, b') of
+// block (k, i) is entry (b', a) of block (i, k)).
+// Three neighbours' loads are in flight together (a learned solve on the
+// 2M-DOF beam: 141 -> 126 ms; two: 136 ms, four: 134 ms), and with them the
+// next three's columns, so that a group waits once for memory and not once
+// for its columns and again for their rows. Past the row's end the own row
+// is read with weight 0.
+template <bool TR, typename Load, typename Add>
+__device__ __forceinline__ void each_neighbour(int64_t i, int g, const int32_t* __restrict__ slice_ptr,
+                                               const int32_t* __restrict__ row_len, const int32_t* __restrict__ col,
+                                               const float* __restrict__ val32, const float* __restrict__ feat,
+                                               Load load, Add add) {
 	int const r = static_cast<int>(i & 63);
 	int const a = TR ? (g & 1) : (g >> 1), bb = TR ? (g >> 1) : (g & 1);
 	float const si = feat[8 * i + 5];
 	int32_t const beg = slice_ptr[i >> 6] + r;
 	int const len = row_len[i];
-	// three neighbours' loads in flight together (a learned solve on the
-	// 2M-DOF beam: 141 -> 126 ms; two: 136 ms, four: 134 ms), and with them the
-	// next three's columns, so that a group waits once for memory and not once
-	// for its columns and again for their rows. Past the row's end the own row
-	// is read with weight 0.
 	constexpr int kTogether = 3;
 	int32_t j[kTogether];
 #pragma unroll
@@ -187,7 +186,8 @@ __device__ __forceinline__ void gather16(int64_t i, int64_t b, int B, int g, con
 	}
 	for (int k = 0; k < len; k += kTogether) {
 		int32_t next[kTogether];
-		float w[kTogether], v[kTogether][16];
+		float w[kTogether];
+		decltype(load(int64_t{0})) v[kTogether];
 #pragma unroll
 		for (int u = 0; u < kTogether; u++) {
 			int const kn = k + kTogether + u;
@@ -195,17 +195,38 @@ __device__ __forceinline__ void gather16(int64_t i, int64_t b, int B, int g, con
 			bool const in = k + u < len;
 			int64_t const blk = beg + (in ? k + u : 0) * kSlice;
 			w[u] = in ? val32[blk_at(blk, r, a, bb)] * si * feat[8 * static_cast<int64_t>(j[u]) + 5] : 0.f;
-			ld16(T + (static_cast<int64_t>(j[u]) * B + b) * kH + 16 * g, v[u]);
+			v[u] = load(static_cast<int64_t>(j[u]));
 		}
 #pragma unroll
 		for (int u = 0; u < kTogether; u++) {
-#pragma unroll
-			for (int c = 0; c < 16; c++) {
-				acc[c] += w[u] * v[u][c];
-			}
+			add(w[u], v[u]);
 			j[u] = next[u];
 		}
 	}
+}
+
+// acc[c] += sum over the neighbours k of node i of w_ik T[(k B + b) H + 16 g + c].
+template <bool TR, typename AT>
+__device__ __forceinline__ void gather16(int64_t i, int64_t b, int B, int g, const int32_t* __restrict__ slice_ptr,
+                                         const int32_t* __restrict__ row_len, const int32_t* __restrict__ col,
+                                         const float* __restrict__ val32, const float* __restrict__ feat,
+                                         const AT* __restrict__ T, float (&acc)[16]) {
+	struct Row {
+		float v[16];
+	};
+	each_neighbour<TR>(
+	    i, g, slice_ptr, row_len, col, val32, feat,
+	    [&](int64_t j) {
+		    Row x;
+		    ld16(T + (j * B + b) * kH + 16 * g, x.v);
+		    return x;
+	    },
+	    [&](float w, Row const& x) {
+#pragma unroll
+		    for (int c = 0; c < 16; c++) {
+			    acc[c] += w * x.v[c];
+		    }
+	    });
 }
 
 // --------------------------------------------------------------- features
@@ -258,18 +279,35 @@ __global__ __launch_bounds__(kWG) void k_feat2(int nb, const int32_t* __restrict
 
 // ------------------------------------------------------------------ forward
 
-// h0 = x W0 (AT: BF16 when training, FP32 in a solve), row rg = node * B + b.
-// RESID: x = Delta^-1/2 P r with r of pair b at r + b * pstride (FP64 in a
-// solve, FP32 when training); otherwise x is given (2 per row, FP32). X (may
+// In a solve (FP32 activations, one row a node) the two ends of the network are
+// two values a node wide, since the aggregation of h0 = x W0 is that of x times
+// W0 and the decoder's of t0 followed by W0^T that of t0 W0^T: the first layer
+// aggregates the two values of x and forms h0 and its message in registers, the
+// last adjoint layer multiplies its result by W0^T before it is written (2 + 8
+// values a row in place of 128), and the decoder aggregates those. What bounds
+// the layers is the gather of 256-byte rows and their writes; these ends do
+// neither. Measured on 40,501 nodes: encoder and first layer 21.8 -> 14.7 us, last
+// adjoint layer 15.5 -> 15.0, decoder 12.9 -> 6.6.
+
+// x = Delta^-1/2 P r of node j.
+struct Pair {
+	float x0, x1;
+};
+__device__ __forceinline__ Pair scaled_residual(int64_t j, const double* __restrict__ r,
+                                                const float* __restrict__ feat) {
+	const float* f = feat + 8 * j;
+	int const fx = static_cast<int>(f[7]);
+	return Pair{(fx & 1) ? 0.f : f[5] * static_cast<float>(r[2 * j]),
+	            (fx & 2) ? 0.f : f[5] * static_cast<float>(r[2 * j + 1])};
+}
+
+// h0 = x W0 in training (BF16), row rg = node * B + b. RESID: x = Delta^-1/2 P r
+// with r of pair b at r + b * pstride; otherwise x is given (2 per row). X (may
 // be null) receives x.
-template <bool RESID, typename RT, typename AT>
-__global__ __launch_bounds__(kWG) void k_encode(int64_t R, int B, const RT* __restrict__ r, int64_t pstride,
+template <bool RESID>
+__global__ __launch_bounds__(kWG) void k_encode(int64_t R, int B, const float* __restrict__ r, int64_t pstride,
                                                 const float* __restrict__ feat, const float* __restrict__ params,
-                                                AT* __restrict__ H0, float* __restrict__ X,
-                                                const Scalars* __restrict__ S) {
-	if (S && S->done) {
-		return;
-	}
+                                                u16* __restrict__ H0, float* __restrict__ X) {
 	__shared__ float W0[2 * kH];
 	for (int k = threadIdx.x; k < 2 * kH; k += kWG) {
 		W0[k] = params[kOffW0 + k];
@@ -285,11 +323,11 @@ __global__ __launch_bounds__(kWG) void k_encode(int64_t R, int B, const RT* __re
 		int64_t const b = rg - i * B;
 		const float* f = feat + 8 * i;
 		int const fx = static_cast<int>(f[7]);
-		x0 = (fx & 1) ? 0.f : f[5] * static_cast<float>(r[b * pstride + 2 * i]);
-		x1 = (fx & 2) ? 0.f : f[5] * static_cast<float>(r[b * pstride + 2 * i + 1]);
+		x0 = (fx & 1) ? 0.f : f[5] * r[b * pstride + 2 * i];
+		x1 = (fx & 2) ? 0.f : f[5] * r[b * pstride + 2 * i + 1];
 	} else {
-		x0 = static_cast<float>(r[2 * rg]);
-		x1 = static_cast<float>(r[2 * rg + 1]);
+		x0 = r[2 * rg];
+		x1 = r[2 * rg + 1];
 	}
 	if (X) {
 		X[2 * rg] = x0;
@@ -303,15 +341,7 @@ __global__ __launch_bounds__(kWG) void k_encode(int64_t R, int B, const RT* __re
 			int const c = 16 * c16 + t;
 			o[t] = x0 * W0[c] + x1 * W0[kH + c];
 		}
-		if constexpr (sizeof(AT) == 2) {
-			st16(H0 + rg * kH + 16 * c16, o);
-		} else {
-#pragma unroll
-			for (int k = 0; k < 4; k++) {
-				*reinterpret_cast<f32x4*>(H0 + rg * kH + 16 * c16 + 4 * k) =
-				    f32x4{o[4 * k], o[4 * k + 1], o[4 * k + 2], o[4 * k + 3]};
-			}
-		}
+		st16(H0 + rg * kH + 16 * c16, o);
 	}
 }
 
@@ -319,15 +349,19 @@ __global__ __launch_bounds__(kWG) void k_encode(int64_t R, int B, const RT* __re
 // features), then h_out = [h_in, m] W on MFMA (Wt: the layer weight
 // transposed, 64 x 128, BF16). AT = u16: BF16 activations (training; Mout,
 // when given, receives m); AT = float: FP32 activations (a solve) and each
-// MFMA input split in two BF16 parts (hi + lo).
-template <typename AT>
+// MFMA input split in two BF16 parts (hi + lo). HEAD: the first layer of a
+// solve, from r instead of Hin.
+template <typename AT, bool HEAD = false>
 __global__ __launch_bounds__(kWG) void k_layer(int64_t R, int B, const int32_t* __restrict__ slice_ptr,
                                                const int32_t* __restrict__ row_len,
                                                const int32_t* __restrict__ col, const float* __restrict__ val32,
                                                const float* __restrict__ feat, const AT* __restrict__ Hin,
                                                AT* __restrict__ Hout, u16* __restrict__ Mout,
-                                               const u16* __restrict__ Wt, const Scalars* __restrict__ S) {
+                                               const u16* __restrict__ Wt, const Scalars* __restrict__ S,
+                                               const double* __restrict__ r = nullptr,
+                                               const float* __restrict__ params = nullptr) {
 	constexpr bool kSplit = sizeof(AT) == 4;
+	static_assert(kSplit || !HEAD, "training keeps h0 for its backward pass");
 	if (S && S->done) {
 		return;
 	}
@@ -346,7 +380,26 @@ __global__ __launch_bounds__(kWG) void k_layer(int64_t R, int B, const int32_t* 
 		self[c] = 0.f;
 		acc[c] = 0.f;
 	}
-	if (rg < R) {
+	if (HEAD) {
+		if (rg < R) {
+			float w0[16], w1[16], s0 = 0.f, s1 = 0.f;
+			ld16(params + kOffW0 + 16 * g, w0);
+			ld16(params + kOffW0 + kH + 16 * g, w1);
+			Pair const x = scaled_residual(rg, r, feat);
+			each_neighbour<false>(
+			    rg, g, slice_ptr, row_len, col, val32, feat,
+			    [&](int64_t j) { return scaled_residual(j, r, feat); },
+			    [&](float w, Pair const& xj) {
+				    s0 += w * xj.x0;
+				    s1 += w * xj.x1;
+			    });
+#pragma unroll
+			for (int c = 0; c < 16; c++) {
+				self[c] = x.x0 * w0[c] + x.x1 * w1[c];
+				acc[c] = s0 * w0[c] + s1 * w1[c];
+			}
+		}
+	} else if (rg < R) {
 		int64_t const i = rg / B;
 		int64_t const b = rg - i * B;
 		ld16(Hin + rg * kH + 16 * g, self);
@@ -411,20 +464,33 @@ __global__ __launch_bounds__(kWG) void k_layer(int64_t R, int B, const int32_t* 
 	}
 }
 
+// The sum of v over the 16 lanes of a row, in each of them.
+__device__ __forceinline__ float row_sum(float v) {
+	v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));    // lanes 1 0 3 2
+	v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));    // lanes 2 3 0 1
+	v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true));   // the other four of eight
+	v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, true));   // the other eight
+	return v;
+}
+
 // One adjoint layer over a 64-row tile: a = Sin (FIRST: the output v of N) or
 // a = Sin + agg^T(Tin), then [Sout, Tout] = a W^T on MFMA (W: the layer
 // weight, 128 x 64, BF16, natural layout). AT = u16: BF16 activations and a
 // rounded to BF16 (training); AT = float: FP32 activations, a split in two
-// BF16 parts (a solve).
-template <bool FIRST, typename AT>
+// BF16 parts (a solve). TAIL: the last layer of a solve, which writes
+// Sout W0^T (2 a row) and, of each quarter g of Tout's channels, its product
+// with that quarter of W0^T (2 at 2 g of the row's 8).
+template <bool FIRST, typename AT, bool TAIL = false>
 __global__ __launch_bounds__(kWG) void k_adjoint(int64_t R, int B, const int32_t* __restrict__ slice_ptr,
                                                  const int32_t* __restrict__ row_len,
                                                  const int32_t* __restrict__ col, const float* __restrict__ val32,
                                                  const float* __restrict__ feat, const AT* __restrict__ Sin,
                                                  const AT* __restrict__ Tin, AT* __restrict__ Sout,
                                                  AT* __restrict__ Tout, const u16* __restrict__ W,
-                                                 const Scalars* __restrict__ S) {
+                                                 const Scalars* __restrict__ S,
+                                                 const float* __restrict__ params = nullptr) {
 	constexpr bool kSplit = sizeof(AT) == 4;
+	static_assert(kSplit || !TAIL, "training keeps the last layer's output");
 	if (S && S->done) {
 		return;
 	}
@@ -476,7 +542,38 @@ __global__ __launch_bounds__(kWG) void k_adjoint(int64_t R, int B, const int32_t
 			}
 		}
 	}
-	if constexpr (kSplit) {
+	if constexpr (TAIL) {
+		float w0[2][4];
+#pragma unroll
+		for (int nb = 0; nb < 4; nb++) {
+			w0[0][nb] = params[kOffW0 + 16 * nb + lr];
+			w0[1][nb] = params[kOffW0 + kH + 16 * nb + lr];
+		}
+#pragma unroll
+		for (int q = 0; q < 4; q++) {
+			// the ten sums over the sixteen lanes of a row; lane k writes the k-th
+			float mine = 0.f;
+#pragma unroll
+			for (int k = 0; k < 10; k++) {
+				int const t2 = k & 1, g2 = k / 2 - 1;
+				float v = 0.f;
+				if (k < 2) {
+#pragma unroll
+					for (int nb = 0; nb < 4; nb++) {
+						v += d[nb][q] * w0[t2][nb];
+					}
+				} else {
+					v = d[4 + g2][q] * w0[t2][g2];
+				}
+				v = row_sum(v);
+				mine = lr == k ? v : mine;
+			}
+			int64_t const ro = tile + 16 * w + 4 * lq + q;
+			if (ro < R && lr < 10) {
+				*(lr < 2 ? Sout + 2 * ro + lr : Tout + 8 * ro + lr - 2) = mine;
+			}
+		}
+	} else if constexpr (kSplit) {
 #pragma unroll
 		for (int q = 0; q < 4; q++) {
 			int64_t const ro = tile + 16 * w + 4 * lq + q;
@@ -513,7 +610,8 @@ __global__ __launch_bounds__(kWG) void k_adjoint(int64_t R, int B, const int32_t
 }
 
 // Decoder (64 rows per workgroup, four threads per row): a0 = S0 + agg^T(T0)
-// (FP32), u = a0 W0^T, z = y + P Delta^-1/2 u. In a solve (!TRAIN) y = D^-1 r
+// (FP32), u = a0 W0^T, z = y + P Delta^-1/2 u. In a solve (!TRAIN) S0 and T0
+// are what the last adjoint layer's TAIL wrote, y = D^-1 r
 // with the solver's FP64 2x2 inverses (dinv64), or y = base when given (the
 // multigrid V-cycle's output), and z is FP64; DOT adds
 // per-workgroup partial sums of z . q. Training: y from the FP32 features,
@@ -540,7 +638,19 @@ __global__ __launch_bounds__(kWG) void k_decode(int64_t R, int B, const RT* __re
 	int const t = threadIdx.x, rr = t >> 2, g = t & 3;
 	int64_t const rg = static_cast<int64_t>(xcd_remap(blockIdx.x, gridDim.x)) * kT + rr;
 	float u0 = 0.f, u1 = 0.f;
-	if (rg < R) {
+	if (!TRAIN && rg < R) {
+		if (g == 0) {
+			u0 = S0[2 * rg];
+			u1 = S0[2 * rg + 1];
+		}
+		each_neighbour<true>(
+		    rg, g, slice_ptr, row_len, col, val32, feat,
+		    [&](int64_t j) { return Pair{static_cast<float>(T0[8 * j + 2 * g]), static_cast<float>(T0[8 * j + 2 * g + 1])}; },
+		    [&](float w, Pair const& y) {
+			    u0 += w * y.x0;
+			    u1 += w * y.x1;
+		    });
+	} else if (rg < R) {
 		int64_t const i = rg / B;
 		int64_t const b = rg - i * B;
 		float a[16];
@@ -939,18 +1049,24 @@ struct Net {
 	const float* feat;
 };
 
-// Forward N over R = n B rows: h[1..3] from h[0] (and the messages when ms).
+// Forward N over R = n B rows: h[1..3] from h[0] (and the messages when ms), or
+// from r with the first layer's HEAD (a solve).
 template <typename AT>
 void net_forward(hipStream_t st, const Net& g, int64_t R, int B, const bfmx_model* m, AT* const* h, u16* const* ms,
-                 const Scalars* S) {
+                 const Scalars* S, const double* r = nullptr) {
 	int const gt = grid_of(R, kT);
-	for (int l = 0; l < 3; l++) {
+	if constexpr (sizeof(AT) == 4) {
+		k_layer<AT, true><<<gt, kWG, 0, st>>>(R, B, g.slice_ptr, g.row_len, g.col, g.val32, g.feat, nullptr, h[1],
+		                                      nullptr, m->d_Wt, S, r, m->d_params);
+	}
+	for (int l = sizeof(AT) == 4 ? 1 : 0; l < 3; l++) {
 		k_layer<AT><<<gt, kWG, 0, st>>>(R, B, g.slice_ptr, g.row_len, g.col, g.val32, g.feat, h[l], h[l + 1],
 		                                ms ? ms[l] : nullptr, m->d_Wt + l * kLayer, S);
 	}
 }
 
-// Adjoint N^T from v through the three layers; leaves (s0, t0) in (sa, ta).
+// Adjoint N^T from v through the three layers; leaves (s0, t0) in (sa, ta), in
+// a solve what the last layer's TAIL makes of them.
 template <typename AT>
 void net_adjoint(hipStream_t st, const Net& g, int64_t R, int B, const bfmx_model* m, const AT* v, AT* sa, AT* ta,
                  AT* sb, AT* tb, const Scalars* S) {
@@ -959,8 +1075,8 @@ void net_adjoint(hipStream_t st, const Net& g, int64_t R, int B, const bfmx_mode
 	                                        m->d_W + 2 * kLayer, S);
 	k_adjoint<false, AT><<<gt, kWG, 0, st>>>(R, B, g.slice_ptr, g.row_len, g.col, g.val32, g.feat, sa, ta, sb, tb,
 	                                         m->d_W + 1 * kLayer, S);
-	k_adjoint<false, AT><<<gt, kWG, 0, st>>>(R, B, g.slice_ptr, g.row_len, g.col, g.val32, g.feat, sb, tb, sa, ta,
-	                                         m->d_W + 0 * kLayer, S);
+	k_adjoint<false, AT, sizeof(AT) == 4><<<gt, kWG, 0, st>>>(R, B, g.slice_ptr, g.row_len, g.col, g.val32, g.feat, sb, tb,
+	                                                          sa, ta, m->d_W + 0 * kLayer, S, m->d_params);
 }
 
 void release_workspace(bfmx_model* m) {
@@ -1160,7 +1276,7 @@ int model_loss_grad(bfmx_model* m, bfmx_trainset* ts, int entry, int p0, int B) 
 	Net const g{s->d_slice_ptr, s->d_row_len, s->d_col, E.d_val32, E.d_feat};
 	int const gr = grid_of(R, kWG), gt = grid_of(R, kT);
 	// u = N^T N x, z = y + P Delta^-1/2 u
-	k_encode<true, float, u16><<<gr, kWG, 0, st>>>(R, B, r, ps, E.d_feat, m->d_params, m->h[0], m->x, nullptr);
+	k_encode<true><<<gr, kWG, 0, st>>>(R, B, r, ps, E.d_feat, m->d_params, m->h[0], m->x);
 	net_forward<u16>(st, g, R, B, m, m->h, m->m, nullptr);
 	net_adjoint<u16>(st, g, R, B, m, m->h[3], m->adj[0], m->adj[1], m->adj[2], m->adj[3], nullptr);
 	k_decode<true, false, float, float, u16><<<gt, kWG, 0, st>>>(R, B, r, ps, g.slice_ptr, g.row_len, g.col, g.val32,
@@ -1171,8 +1287,7 @@ int model_loss_grad(bfmx_model* m, bfmx_trainset* ts, int entry, int p0, int B) 
 	                           m->xg, m->lpart);
 	k_sum_loss<<<1, kWG, 0, st>>>(gr, m->lpart, m->loss);
 	// N g
-	k_encode<false, float, u16><<<gr, kWG, 0, st>>>(R, B, m->xg, 0, E.d_feat, m->d_params, m->hg[0], nullptr,
-	                                                nullptr);
+	k_encode<false><<<gr, kWG, 0, st>>>(R, B, m->xg, 0, E.d_feat, m->d_params, m->hg[0], nullptr);
 	net_forward<u16>(st, g, R, B, m, m->hg, m->mg, nullptr);
 	// d<N g, N x>/d theta + d<N x, N g>/d theta
 	k_bf16_to_f32<<<grid_of(R * kH, kWG), kWG, 0, st>>>(R * kH, m->hg[3], m->up);
@@ -1415,10 +1530,9 @@ double* mpnn_apply(bfmx_system* s, const double* r, const double* q, double* par
 	int64_t const R = s->n_nodes;
 	Net const g{s->d_slice_ptr, s->d_row_len, s->d_col, s->d_val32, s->d_mp_feat};
 	float** h = s->d_mp_h;   // four FP32 buffers of 64 per node
-	int const gr = grid_of(R, kWG), gt = grid_of(R, kT);
-	k_encode<true, double, float><<<gr, kWG, 0, st>>>(R, 1, r, 0, g.feat, m->d_params, h[0], nullptr, S);
+	int const gt = grid_of(R, kT);
 	float* hf[4] = {h[0], h[1], h[0], h[1]};   // ping-pong: h3 lands in h[1]
-	net_forward<float>(st, g, R, 1, m, hf, nullptr, S);
+	net_forward<float>(st, g, R, 1, m, hf, nullptr, S, r);
 	net_adjoint<float>(st, g, R, 1, m, h[1], h[2], h[3], h[0], h[1], S);
 	k_decode<false, true, double, double, float><<<gt, kWG, 0, st>>>(R, 1, r, 0, g.slice_ptr, g.row_len, g.col, g.val32,
 	                                                          g.feat, m->d_params, h[2], h[3], s->d_dinv, base,

@@ -159,63 +159,74 @@ __device__ __forceinline__ void split16(u16* hi, u16* lo, const float (&v)[16]) 
 	*reinterpret_cast<u16x8*>(lo + 8) = l1;
 }
 
+// What a row's gather starts from: its slots and isd_i.
+struct RowHead {
+	int32_t beg, len;
+	float si;
+};
+__device__ __forceinline__ RowHead row_head(int64_t i, const int32_t* __restrict__ slice_ptr,
+                                            const int32_t* __restrict__ row_len, const float* __restrict__ feat) {
+	return RowHead{slice_ptr[i >> 6] + static_cast<int32_t>(i & 63), row_len[i], feat[8 * i + 5]};
+}
+
 // add(w_ik, load(k)) for the neighbours k of node i in row slot order; w_ik =
 // entry (a, b') of block (i, k) times isd_i isd_k with (a, b') = (g / 2, g % 2),
 // or (g % 2, g / 2) when TR (the adjoint: for the symmetric A, entry (a, b') of
 // block (k, i) is entry (b', a) of block (i, k)).
-// Three neighbours' loads are in flight together (a learned solve on the
-// 2M-DOF beam: 141 -> 126 ms; two: 136 ms, four: 134 ms), and with them the
-// next three's columns, so that a group waits once for memory and not once
-// for its columns and again for their rows. Past the row's end the own row
-// is read with weight 0.
-template <bool TR, typename Load, typename Add>
-__device__ __forceinline__ void each_neighbour(int64_t i, int g, const int32_t* __restrict__ slice_ptr,
-                                               const int32_t* __restrict__ row_len, const int32_t* __restrict__ col,
+// TOGETHER neighbours' loads are in flight together, and with them the next
+// group's columns, so that a group waits once for memory and not once for its
+// columns and again for their rows. Past the row's end the own row is read
+// with weight 0. Rows of 64 values: three together (a learned solve on the
+// 2M-DOF beam: 141 -> 126 ms; two: 136 ms, four: 134 ms); rows of two: nine, a
+// whole row of a structured mesh.
+template <bool TR, int TOGETHER, typename Load, typename Add>
+__device__ __forceinline__ void each_neighbour(int64_t i, RowHead const& h, int g, const int32_t* __restrict__ col,
                                                const float* __restrict__ val32, const float* __restrict__ feat,
                                                Load load, Add add) {
 	int const r = static_cast<int>(i & 63);
 	int const a = TR ? (g & 1) : (g >> 1), bb = TR ? (g >> 1) : (g & 1);
-	float const si = feat[8 * i + 5];
-	int32_t const beg = slice_ptr[i >> 6] + r;
-	int const len = row_len[i];
-	constexpr int kTogether = 3;
-	int32_t j[kTogether];
+	int32_t j[TOGETHER];
 #pragma unroll
-	for (int u = 0; u < kTogether; u++) {
-		j[u] = u < len ? col[beg + u * kSlice] : static_cast<int32_t>(i);
+	for (int u = 0; u < TOGETHER; u++) {
+		j[u] = u < h.len ? col[h.beg + u * kSlice] : static_cast<int32_t>(i);
 	}
-	for (int k = 0; k < len; k += kTogether) {
-		int32_t next[kTogether];
-		float w[kTogether];
-		decltype(load(int64_t{0})) v[kTogether];
+	for (int k = 0; k < h.len; k += TOGETHER) {
+		int32_t next[TOGETHER];
+		float w[TOGETHER];
+		decltype(load(int64_t{0})) v[TOGETHER];
 #pragma unroll
-		for (int u = 0; u < kTogether; u++) {
-			int const kn = k + kTogether + u;
-			next[u] = kn < len ? col[beg + kn * kSlice] : static_cast<int32_t>(i);
-			bool const in = k + u < len;
-			int64_t const blk = beg + (in ? k + u : 0) * kSlice;
-			w[u] = in ? val32[blk_at(blk, r, a, bb)] * si * feat[8 * static_cast<int64_t>(j[u]) + 5] : 0.f;
+		for (int u = 0; u < TOGETHER; u++) {
+			int const kn = k + TOGETHER + u;
+			next[u] = kn < h.len ? col[h.beg + kn * kSlice] : static_cast<int32_t>(i);
+			bool const in = k + u < h.len;
+			int64_t const blk = h.beg + (in ? k + u : 0) * kSlice;
+			w[u] = in ? val32[blk_at(blk, r, a, bb)] * h.si * feat[8 * static_cast<int64_t>(j[u]) + 5] : 0.f;
 			v[u] = load(static_cast<int64_t>(j[u]));
 		}
 #pragma unroll
-		for (int u = 0; u < kTogether; u++) {
+		for (int u = 0; u < TOGETHER; u++) {
 			add(w[u], v[u]);
 			j[u] = next[u];
 		}
 	}
 }
 
+// The done flag of a solve (S may be null) read with the loads of v.
+template <typename... T>
+__device__ __forceinline__ int stop_after(const Scalars* __restrict__ S, T const&... v) {
+	return S ? done_after(S, v...) : 0;
+}
+
 // acc[c] += sum over the neighbours k of node i of w_ik T[(k B + b) H + 16 g + c].
 template <bool TR, typename AT>
-__device__ __forceinline__ void gather16(int64_t i, int64_t b, int B, int g, const int32_t* __restrict__ slice_ptr,
-                                         const int32_t* __restrict__ row_len, const int32_t* __restrict__ col,
-                                         const float* __restrict__ val32, const float* __restrict__ feat,
+__device__ __forceinline__ void gather16(int64_t i, RowHead const& h, int64_t b, int B, int g,
+                                         const int32_t* __restrict__ col, const float* __restrict__ val32, const float* __restrict__ feat,
                                          const AT* __restrict__ T, float (&acc)[16]) {
 	struct Row {
 		float v[16];
 	};
-	each_neighbour<TR>(
-	    i, g, slice_ptr, row_len, col, val32, feat,
+	each_neighbour<TR, 3>(
+	    i, h, g, col, val32, feat,
 	    [&](int64_t j) {
 		    Row x;
 		    ld16(T + (j * B + b) * kH + 16 * g, x.v);
@@ -362,18 +373,22 @@ __global__ __launch_bounds__(kWG) void k_layer(int64_t R, int B, const int32_t* 
                                                const float* __restrict__ params = nullptr) {
 	constexpr bool kSplit = sizeof(AT) == 4;
 	static_assert(kSplit || !HEAD, "training keeps h0 for its backward pass");
-	if (S && S->done) {
-		return;
-	}
 	__shared__ u16 X[kT][kP128];
 	__shared__ u16 Xl[kSplit ? kT : 1][kP128];
 	__shared__ u16 Ws[kH][kP128];
-	for (int e = threadIdx.x; e < kH * 16; e += kWG) {
-		int const n = e >> 4, k8 = e & 15;
-		*reinterpret_cast<u16x8*>(&Ws[n][8 * k8]) = *reinterpret_cast<const u16x8*>(Wt + n * 2 * kH + 8 * k8);
-	}
 	int const t = threadIdx.x, row = t >> 2, g = t & 3;
 	int64_t const tile = static_cast<int64_t>(xcd_remap(blockIdx.x, gridDim.x)) * kT, rg = tile + row;
+	int64_t const i = min(rg, R - 1) / B, b = min(rg, R - 1) - i * B;
+	// the weights go to LDS after the gather, their loads are its first wait
+	u16x8 ws[kH * 16 / kWG];
+#pragma unroll
+	for (int u = 0; u < kH * 16 / kWG; u++) {
+		ws[u] = *reinterpret_cast<const u16x8*>(Wt + 8 * (t + u * kWG));
+	}
+	RowHead const h = row_head(i, slice_ptr, row_len, feat);
+	if (stop_after(S, h.beg, h.len, h.si, ws[0], ws[1], ws[2], ws[3])) {
+		return;
+	}
 	float self[16], acc[16];
 #pragma unroll
 	for (int c = 0; c < 16; c++) {
@@ -386,8 +401,8 @@ __global__ __launch_bounds__(kWG) void k_layer(int64_t R, int B, const int32_t* 
 			ld16(params + kOffW0 + 16 * g, w0);
 			ld16(params + kOffW0 + kH + 16 * g, w1);
 			Pair const x = scaled_residual(rg, r, feat);
-			each_neighbour<false>(
-			    rg, g, slice_ptr, row_len, col, val32, feat,
+			each_neighbour<false, 9>(
+			    rg, h, g, col, val32, feat,
 			    [&](int64_t j) { return scaled_residual(j, r, feat); },
 			    [&](float w, Pair const& xj) {
 				    s0 += w * xj.x0;
@@ -400,10 +415,8 @@ __global__ __launch_bounds__(kWG) void k_layer(int64_t R, int B, const int32_t* 
 			}
 		}
 	} else if (rg < R) {
-		int64_t const i = rg / B;
-		int64_t const b = rg - i * B;
 		ld16(Hin + rg * kH + 16 * g, self);
-		gather16<false>(i, b, B, g, slice_ptr, row_len, col, val32, feat, Hin, acc);
+		gather16<false>(i, h, b, B, g, col, val32, feat, Hin, acc);
 	}
 	if constexpr (kSplit) {
 		split16(&X[row][16 * g], &Xl[row][16 * g], self);
@@ -414,6 +427,11 @@ __global__ __launch_bounds__(kWG) void k_layer(int64_t R, int B, const int32_t* 
 		if (Mout && rg < R) {
 			st16(Mout + rg * kH + 16 * g, acc);
 		}
+	}
+#pragma unroll
+	for (int u = 0; u < kH * 16 / kWG; u++) {
+		int const e = t + u * kWG;
+		*reinterpret_cast<u16x8*>(&Ws[e >> 4][8 * (e & 15)]) = ws[u];
 	}
 	__syncthreads();
 	int const w = t >> 6, l = t & 63, lr = l & 15, lq = l >> 4;
@@ -491,19 +509,25 @@ __global__ __launch_bounds__(kWG) void k_adjoint(int64_t R, int B, const int32_t
                                                  const float* __restrict__ params = nullptr) {
 	constexpr bool kSplit = sizeof(AT) == 4;
 	static_assert(kSplit || !TAIL, "training keeps the last layer's output");
-	if (S && S->done) {
-		return;
-	}
 	__shared__ u16 A[kT][kP64];
 	__shared__ u16 Al[kSplit ? kT : 1][kP64];
 	__shared__ u16 Ws[2 * kH][kP64];
 	__shared__ u16 O[kSplit ? 1 : kT][kP128];
-	for (int e = threadIdx.x; e < 2 * kH * 8; e += kWG) {
-		int const n = e >> 3, k8 = e & 7;
-		*reinterpret_cast<u16x8*>(&Ws[n][8 * k8]) = *reinterpret_cast<const u16x8*>(W + n * kH + 8 * k8);
-	}
 	int const t = threadIdx.x, row = t >> 2, g = t & 3;
 	int64_t const tile = static_cast<int64_t>(xcd_remap(blockIdx.x, gridDim.x)) * kT, rg = tile + row;
+	int64_t const i = min(rg, R - 1) / B, b = min(rg, R - 1) - i * B;
+	u16x8 ws[kH * 16 / kWG];   // as in k_layer
+#pragma unroll
+	for (int u = 0; u < kH * 16 / kWG; u++) {
+		ws[u] = *reinterpret_cast<const u16x8*>(W + 8 * (t + u * kWG));
+	}
+	RowHead h{};
+	if (!FIRST) {
+		h = row_head(i, slice_ptr, row_len, feat);
+	}
+	if (stop_after(S, h.beg, h.len, h.si, ws[0], ws[1], ws[2], ws[3])) {
+		return;
+	}
 	float a[16];
 #pragma unroll
 	for (int c = 0; c < 16; c++) {
@@ -512,15 +536,18 @@ __global__ __launch_bounds__(kWG) void k_adjoint(int64_t R, int B, const int32_t
 	if (rg < R) {
 		ld16(Sin + rg * kH + 16 * g, a);
 		if (!FIRST) {
-			int64_t const i = rg / B;
-			int64_t const b = rg - i * B;
-			gather16<true>(i, b, B, g, slice_ptr, row_len, col, val32, feat, Tin, a);
+			gather16<true>(i, h, b, B, g, col, val32, feat, Tin, a);
 		}
 	}
 	if constexpr (kSplit) {
 		split16(&A[row][16 * g], &Al[row][16 * g], a);
 	} else {
 		st16(&A[row][16 * g], a);
+	}
+#pragma unroll
+	for (int u = 0; u < kH * 16 / kWG; u++) {
+		int const e = t + u * kWG;
+		*reinterpret_cast<u16x8*>(&Ws[e >> 3][8 * (e & 7)]) = ws[u];
 	}
 	__syncthreads();
 	int const w = t >> 6, l = t & 63, lr = l & 15, lq = l >> 4;
@@ -626,36 +653,38 @@ __global__ __launch_bounds__(kWG) void k_decode(int64_t R, int B, const RT* __re
                                                 const double* __restrict__ dinv64, const float* __restrict__ base,
                                                 ZT* __restrict__ z, const double* __restrict__ q,
                                                 double* __restrict__ partial, const Scalars* __restrict__ S) {
-	if (S && S->done) {
-		return;
-	}
 	__shared__ float W0[2 * kH];
 	__shared__ float part[kWG][2];
-	for (int k = threadIdx.x; k < 2 * kH; k += kWG) {
-		W0[k] = params[kOffW0 + k];
-	}
-	__syncthreads();
 	int const t = threadIdx.x, rr = t >> 2, g = t & 3;
 	int64_t const rg = static_cast<int64_t>(xcd_remap(blockIdx.x, gridDim.x)) * kT + rr;
+	int64_t const i = min(rg, R - 1) / B, b = min(rg, R - 1) - i * B;
+	RowHead const h = row_head(i, slice_ptr, row_len, feat);
+	if (stop_after(S, h.beg, h.len, h.si)) {
+		return;
+	}
+	if (TRAIN) {
+		for (int k = t; k < 2 * kH; k += kWG) {
+			W0[k] = params[kOffW0 + k];
+		}
+		__syncthreads();
+	}
 	float u0 = 0.f, u1 = 0.f;
 	if (!TRAIN && rg < R) {
 		if (g == 0) {
 			u0 = S0[2 * rg];
 			u1 = S0[2 * rg + 1];
 		}
-		each_neighbour<true>(
-		    rg, g, slice_ptr, row_len, col, val32, feat,
+		each_neighbour<true, 9>(
+		    rg, h, g, col, val32, feat,
 		    [&](int64_t j) { return Pair{static_cast<float>(T0[8 * j + 2 * g]), static_cast<float>(T0[8 * j + 2 * g + 1])}; },
 		    [&](float w, Pair const& y) {
 			    u0 += w * y.x0;
 			    u1 += w * y.x1;
 		    });
 	} else if (rg < R) {
-		int64_t const i = rg / B;
-		int64_t const b = rg - i * B;
 		float a[16];
 		ld16(S0 + rg * kH + 16 * g, a);
-		gather16<true>(i, b, B, g, slice_ptr, row_len, col, val32, feat, T0, a);
+		gather16<true>(i, h, b, B, g, col, val32, feat, T0, a);
 #pragma unroll
 		for (int c = 0; c < 16; c++) {
 			u0 += a[c] * W0[16 * g + c];
@@ -669,8 +698,6 @@ __global__ __launch_bounds__(kWG) void k_decode(int64_t R, int B, const RT* __re
 	if (g == 0 && rg < R) {
 		u0 = part[t][0] + part[t + 1][0] + part[t + 2][0] + part[t + 3][0];
 		u1 = part[t][1] + part[t + 1][1] + part[t + 2][1] + part[t + 3][1];
-		int64_t const i = rg / B;
-		int64_t const b = rg - i * B;
 		const float* f = feat + 8 * i;
 		int const fx = static_cast<int>(f[7]);
 		float const c0 = (fx & 1) ? 0.f : f[5] * u0;
@@ -867,7 +894,7 @@ __global__ __launch_bounds__(kWG) void k_agg_bwd(int64_t R, int B, const int32_t
 	int64_t const b = rg - j * B;
 	float acc[16];
 	ld16(dHin + rg * kH + 16 * g, acc);
-	gather16<true>(j, b, B, g, slice_ptr, row_len, col, val32, feat, dM, acc);
+	gather16<true>(j, row_head(j, slice_ptr, row_len, feat), b, B, g, col, val32, feat, dM, acc);
 #pragma unroll
 	for (int c = 0; c < 16; c++) {
 		dHin[rg * kH + 16 * g + c] = acc[c];

@@ -65,12 +65,23 @@ constexpr int kNParams = kOffL + 3 * kLayer;
 constexpr int kGradParts = 512;              // workgroups of the gradient kernels (partials)
 constexpr float kEncInit = 0.015f;           // initial encoder weights: uniform in +-kEncInit
 
-__device__ __forceinline__ u16 f2bf(float f) {   // round to nearest even
-	uint32_t const u = __float_as_uint(f);
-	if ((u & 0x7fffffffu) > 0x7f800000u) {
-		return 0x7fc0;
+// To BF16, round to nearest even: the conversion instruction, two values at
+// once where there are two. In integer code (six or more instructions a value)
+// the two-part splits of a solve's layers were a tenth of their time: on
+// 40,501 nodes the layers 14.2 -> 12.8 us, the first 13.8 -> 12.0, the adjoint
+// layers 14.9, 14.2 and 7.1 -> 14.2, 13.0 and 6.7 (with the branches between a
+// gather's loads gone as well).
+__device__ __forceinline__ u16 f2bf(float f) {
+	return __builtin_bit_cast(u16, static_cast<__bf16>(f));
+}
+__device__ __forceinline__ u16x8 f2bf(const float* v) {
+	typedef float f32x8 __attribute__((ext_vector_type(8)));
+	f32x8 x;
+#pragma unroll
+	for (int c = 0; c < 8; c++) {
+		x[c] = v[c];
 	}
-	return static_cast<u16>((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+	return __builtin_bit_cast(u16x8, __builtin_convertvector(x, bf16x8));
 }
 __device__ __forceinline__ float bf2f(u16 h) {
 	return __uint_as_float(static_cast<uint32_t>(h) << 16);
@@ -132,31 +143,24 @@ __device__ __forceinline__ void ld16(const float* p, float (&v)[16]) {
 
 // The BF16 rounding of 16 values (8-byte-aligned LDS or global row).
 __device__ __forceinline__ void st16(u16* p, const float (&v)[16]) {
-	u16x8 a, b;
-#pragma unroll
-	for (int c = 0; c < 8; c++) {
-		a[c] = f2bf(v[c]);
-		b[c] = f2bf(v[8 + c]);
-	}
-	*reinterpret_cast<u16x8*>(p) = a;
-	*reinterpret_cast<u16x8*>(p + 8) = b;
+	*reinterpret_cast<u16x8*>(p) = f2bf(v);
+	*reinterpret_cast<u16x8*>(p + 8) = f2bf(v + 8);
 }
 
 // v = hi + lo with hi, lo BF16 (hi the rounding of v, lo of the remainder):
 // two BF16 MFMAs on (hi, lo) give the product to about 16 significant bits.
 __device__ __forceinline__ void split16(u16* hi, u16* lo, const float (&v)[16]) {
-	u16x8 h0, h1, l0, l1;
 #pragma unroll
-	for (int c = 0; c < 8; c++) {
-		h0[c] = f2bf(v[c]);
-		h1[c] = f2bf(v[8 + c]);
-		l0[c] = f2bf(v[c] - bf2f(h0[c]));
-		l1[c] = f2bf(v[8 + c] - bf2f(h1[c]));
+	for (int k = 0; k < 16; k += 8) {
+		u16x8 const h = f2bf(v + k);
+		float rest[8];
+#pragma unroll
+		for (int c = 0; c < 8; c++) {
+			rest[c] = v[k + c] - bf2f(h[c]);
+		}
+		*reinterpret_cast<u16x8*>(hi + k) = h;
+		*reinterpret_cast<u16x8*>(lo + k) = f2bf(rest);
 	}
-	*reinterpret_cast<u16x8*>(hi) = h0;
-	*reinterpret_cast<u16x8*>(hi + 8) = h1;
-	*reinterpret_cast<u16x8*>(lo) = l0;
-	*reinterpret_cast<u16x8*>(lo + 8) = l1;
 }
 
 // What a row's gather starts from: its slots and isd_i.
@@ -175,8 +179,9 @@ __device__ __forceinline__ RowHead row_head(int64_t i, const int32_t* __restrict
 // block (k, i) is entry (b', a) of block (i, k)).
 // TOGETHER neighbours' loads are in flight together, and with them the next
 // group's columns, so that a group waits once for memory and not once for its
-// columns and again for their rows. Past the row's end the own row is read
-// with weight 0. Rows of 64 values: three together (a learned solve on the
+// columns and again for their rows. Past the row's end (every row has its
+// diagonal) the last neighbour is read again, with weight 0: no branches
+// between the loads. Rows of 64 values: three together (a learned solve on the
 // 2M-DOF beam: 141 -> 126 ms; two: 136 ms, four: 134 ms); rows of two: nine, a
 // whole row of a structured mesh.
 template <bool TR, int TOGETHER, typename Load, typename Add>
@@ -185,10 +190,11 @@ __device__ __forceinline__ void each_neighbour(int64_t i, RowHead const& h, int 
                                                Load load, Add add) {
 	int const r = static_cast<int>(i & 63);
 	int const a = TR ? (g & 1) : (g >> 1), bb = TR ? (g >> 1) : (g & 1);
+	int const last = max(h.len - 1, 0);
 	int32_t j[TOGETHER];
 #pragma unroll
 	for (int u = 0; u < TOGETHER; u++) {
-		j[u] = u < h.len ? col[h.beg + u * kSlice] : static_cast<int32_t>(i);
+		j[u] = col[h.beg + min(u, last) * kSlice];
 	}
 	for (int k = 0; k < h.len; k += TOGETHER) {
 		int32_t next[TOGETHER];
@@ -196,11 +202,10 @@ __device__ __forceinline__ void each_neighbour(int64_t i, RowHead const& h, int 
 		decltype(load(int64_t{0})) v[TOGETHER];
 #pragma unroll
 		for (int u = 0; u < TOGETHER; u++) {
-			int const kn = k + TOGETHER + u;
-			next[u] = kn < h.len ? col[h.beg + kn * kSlice] : static_cast<int32_t>(i);
-			bool const in = k + u < h.len;
-			int64_t const blk = h.beg + (in ? k + u : 0) * kSlice;
-			w[u] = in ? val32[blk_at(blk, r, a, bb)] * h.si * feat[8 * static_cast<int64_t>(j[u]) + 5] : 0.f;
+			next[u] = col[h.beg + min(k + TOGETHER + u, last) * kSlice];
+			int64_t const blk = h.beg + min(k + u, last) * kSlice;
+			float const wk = val32[blk_at(blk, r, a, bb)] * h.si * feat[8 * static_cast<int64_t>(j[u]) + 5];
+			w[u] = k + u < h.len ? wk : 0.f;
 			v[u] = load(static_cast<int64_t>(j[u]));
 		}
 #pragma unroll

@@ -1,16 +1,15 @@
 // Batched solves: many independent planar systems of uneven sizes.
 //
 // Systems whose matrix fits the registers of a cluster of workgroups (rows of
-// at most nine blocks, up to 262,144 nodes) are solved by resident.hip: all
-// clusters in one launch, each taking one system after another. The others,
-// and all of them where the device refuses that launch, are solved by the
-// streaming kernel below, one persistent launch per size class (captured in
+// at most nine blocks, up to 262,144 nodes) are solved by resident.hip, each
+// cluster taking one system after another. The others, and all of them where a
+// cluster's bounded wait ran out, are solved by the streaming kernel below, one persistent launch per size class (captured in
 // one HIP graph when it solves the whole batch).
 //
-// In the streaming kernel one workgroup runs the whole Jacobi or block-Jacobi PCG of one system: its
-// passes over the rows (SpMV with the direction update folded into the
-// gathers, the vector updates, the residual recomputation) are separated by
-// workgroup barriers, and its dot products are workgroup reductions in a
+// In the streaming kernel one workgroup runs the whole Jacobi or block-Jacobi
+// PCG of one system: its passes over the rows (SpMV with the direction update
+// folded into the gathers, the vector updates, the residual recomputation) are
+// separated by workgroup barriers, and its dot products are workgroup reductions in a
 // fixed order, so an iteration costs no kernel launch and no device-scope
 // synchronisation. Systems are dealt to workgroups largest first; the
 // hardware dispatcher balances them over the CUs as workgroups finish.
@@ -209,6 +208,11 @@ __device__ __forceinline__ void for_rows(int64_t n, F f) {
 // arithmetic's ~200 registers would cut its occupancy.)
 constexpr int kAsmBlock = 256;
 constexpr int kAsmParts = 64;   // workgroups of one system at most
+// With more systems than this (four a CU, so that the sizes even out) one
+// workgroup runs a system's colours, whose rows it then finds in its caches:
+// 4,096 panels of 500 to 30,000 nodes 90 ms with a launch a colour, 67 here (the
+// multigrid batch 783 and 760 ms); at 64, 1.3 and 4.8 ms.
+constexpr int kAsmMany = 1024;
 
 __global__ __launch_bounds__(kAsmBlock) void k_batch_zero(const BatchInst* __restrict__ insts,
                                                           const int32_t* __restrict__ order, int parts) {
@@ -254,6 +258,22 @@ __global__ __launch_bounds__(kAsmBlock) void k_batch_elements(const BatchInst* _
 		assemble_elements<3>(S, e0, e1, step);
 	} else {
 		assemble_elements<4>(S, e0, e1, step);
+	}
+}
+
+// All colours of a system by one workgroup, for batches of many systems
+// (launch_assemble).
+__global__ __launch_bounds__(kAsmBlock) void k_batch_colors(const BatchInst* __restrict__ insts,
+                                                            const int32_t* __restrict__ order) {
+	BatchInst const S = insts[order[blockIdx.x]];
+	for (int c = 0; c < S.n_colors; c++) {
+		int64_t const e0 = S.color_ptr[c] + threadIdx.x, e1 = S.color_ptr[c + 1];
+		if (S.kind == 3) {
+			assemble_elements<3>(S, e0, e1, kAsmBlock);
+		} else {
+			assemble_elements<4>(S, e0, e1, kAsmBlock);
+		}
+		__syncthreads();
 	}
 }
 
@@ -857,7 +877,10 @@ void launch_assemble(bfmx_batch* b) {
 		    std::max<int64_t>(1, std::min({want, static_cast<int64_t>(kAsmParts), 65536 / std::max<int64_t>(m, 1)})));
 		int const blocks = static_cast<int>(m) * parts;
 		k_batch_zero<<<blocks, kAsmBlock, 0, b->stream>>>(b->d_inst, b->d_order_all, parts);
-		for (int c = 0; c < colors; c++) {
+		if (m > kAsmMany) {
+			k_batch_colors<<<static_cast<int>(m), kAsmBlock, 0, b->stream>>>(b->d_inst, b->d_order_all);
+		}
+		for (int c = 0; c < colors && m <= kAsmMany; c++) {
 			k_batch_elements<<<blocks, kAsmBlock, 0, b->stream>>>(b->d_inst, b->d_order_all, parts, c);
 		}
 		k_batch_conditions<<<static_cast<int>(m), kAsmBlock, 0, b->stream>>>(b->d_inst, b->d_order_all);

@@ -16,9 +16,9 @@ numeric set-up are reused: a new load case) is reported beside it, and
 plain FP64 Jacobi-PCG is timed on the system (the speedups are reported).
 
 Also reported: the batched workload (4096 seeded holed panels of 1k-60k DOFs,
-assembled and solved by block-Jacobi PCG in one graph launch, one workgroup per
-panel: DOF/s and the launch's algorithmic GB/s, and the same batch in the
-multigrid mode); the roofline of the headline solver's largest kernel (the
+assembled and solved by block-Jacobi PCG, each by a cluster of workgroups that
+holds its matrix in registers: DOF/s, and the same batch in the multigrid
+mode); the roofline of the headline solver's largest kernel (the
 flexible-CG FP64 SpMV), of its finest-level post-smoothing step (FP32 SpMV +
 block-Jacobi Chebyshev step) and of the FP64 CG SpMV (algorithmic bytes /
 mean launch time from HIP events on the solver's stream), the end-to-end time (upload + renumbering + assembly + conditions +
@@ -48,9 +48,6 @@ HBM_PEAK_GBS = 8000.0
 # (FETCH_SIZE x 1.9998 + WRITE_SIZE, the factors read off a 256 MiB
 # device-to-device copy in the same runs): profiles/hbm_traffic_q1_2m.md
 TRAFFIC_Q1_2M = {"k_cg_spmv": 389.3e6, "k_fcg_spmv": 397.4e6, "k_cheb": 254.9e6}
-# the same for the 4096-panel persistent launch's k_batch_pcg (one dispatch,
-# picks [4, 4, 4]): profiles/batched_panels_persistent_and_multigrid_kernel_stats.md
-TRAFFIC_BATCH_4096 = 68.47e12
 CPU_SAMPLE = (180, 45)   # Q1 beam cells for the reference CPU path (16,652 DOFs)
 
 
@@ -212,9 +209,10 @@ def copy_calibration(nbytes):
 def batched_leg(D, meshgen, count, rtol):
     """The batched workload: `count` seeded holed panels (1k-60k DOFs, plane
     strain, traction U(1e5, 1e7) N/m on top, bottom corners pinned), built
-    into one batch from their meshes; one timed graph launch assembles every
-    panel (one workgroup each) and solves it by block-Jacobi PCG (one
-    workgroup each, the autotuner's configurations) to rtol."""
+    into one batch from their meshes; one timed launch assembles every panel
+    (a launch per colour over all of them) and solves it by block-Jacobi PCG
+    to rtol (a cluster of workgroups each; the autotuner's configurations are
+    for panels that do not fit one)."""
     t = time.perf_counter()
     inst, sizes, dofs = [], [], 0
     for k in range(count):
@@ -240,11 +238,14 @@ def batched_leg(D, meshgen, count, rtol):
     assert all(x["status"] == 0 and x["rel_residual"] <= rtol for x in st)
     its = np.array([x["iterations"] for x in st])
     nnzb = np.array([b.system(k).info()["nnzb"] for k in range(count)])
-    byt = sum(D.batch_bytes(int(nnzb[k]), sizes[k], int(st[k]["iterations"]), int(st[k]["restarts"]), pre)
-              for k in range(count))
+    # the clusters read each panel's matrix and load once and keep them; what
+    # a streaming solve of the same iterations would move is given beside it
+    byt = sum(D.batch_bytes(int(nnzb[k]), sizes[k], 1, 0, pre) for k in range(count))
+    streamed = sum(D.batch_bytes(int(nnzb[k]), sizes[k], int(st[k]["iterations"]), int(st[k]["restarts"]), pre)
+                   for k in range(count))
     gbs = byt / (ms / 1e3) / 1e9
     log(f"batched: {ms:.1f} ms device ({wall * 1e3:.1f} ms wall), {dofs / (ms / 1e3):.3e} DOF/s, "
-        f"iterations mean {its.mean():.0f} max {its.max()}, {gbs:.0f} GB/s algorithmic")
+        f"iterations mean {its.mean():.0f} max {its.max()}, {streamed / (ms / 1e3) / 1e9:.0f} GB/s if it were streamed")
     # multigrid mode: the same batch solved as one block-diagonal system by
     # flexible CG + the multigrid V-cycle (each load scaled to unit norm, the
     # tolerance checks testing every panel's own residual); the first launch
@@ -265,17 +266,16 @@ def batched_leg(D, meshgen, count, rtol):
         f"persistent launch; first launch (union and hierarchy build) {t_mg_setup:.1f} s")
     return {
         "workload": f"{count} holed panels (seeds 0-{count - 1}), 1k-60k DOFs, plane strain, block-Jacobi PCG "
-                    f"to rtol {rtol:g}, assembled and solved in one graph launch",
+                    f"to rtol {rtol:g}, assembled and solved from one call",
         "n_dof": int(dofs), "ms_per_step": ms, "wall_ms": wall * 1e3, "value": dofs / (ms / 1e3),
         "unit": "DOF/s", "iterations_mean": float(its.mean()), "iterations_max": int(its.max()),
         "picks": picks.tolist(), "autotune_ms": times.tolist(), "setup_s": {"meshes": t_mesh,
                                                                               "batch_create": t_create,
                                                                               "autotune": t_tune},
-        "roofline": {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": gbs / HBM_PEAK_GBS,
-                     "traffic": TRAFFIC_BATCH_4096 if count == 4096 and picks.tolist() == [4, 4, 4] else None,
-                     "kernel": "k_batch_pcg (block Jacobi, autotuned) + k_batch_assemble (whole graph launch)",
-                     "algorithmic_bytes": byt},
+        "roofline": {"bound": "latency of the clusters' exchanges and issue (the matrix stays in registers)",
+                     "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS,
+                     "traffic": None, "kernel": "k_resident_batch (block Jacobi) + k_batch_elements (whole launch)",
+                     "algorithmic_bytes": byt, "streamed_bytes_of_its_iterations": streamed},
         "multigrid": {
             "solver": "the batch as one block-diagonal system: flexible CG (FP64) + FP32 smoothed-aggregation "
                       "V-cycle, one dense coarsest inverse per panel, loads scaled to unit norm, every panel's "

@@ -42,7 +42,8 @@
 // also forms the partials of z . q_prev) and five kernels:
 //   k_red_fcg_beta, k_fcg_spmv (p = z + beta p_old, q = A p, partials of p . q
 //   and p . r), k_red_fcg_alpha, k_fcg_update (x, r and partials of r . r),
-//   k_red_fcg_rr.
+//   k_red_fcg_rr; up to 1,024 workgroups the consumers of beta and alpha fold
+//   the partials themselves (fold_partials), two kernels less.
 
 #include <algorithm>
 #include <chrono>

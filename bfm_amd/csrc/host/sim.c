@@ -263,8 +263,9 @@ static double now_ms(void) {
 }
 
 /* Largest instance (nodes) that the batched path solves with point or block
- * Jacobi: those solves run one workgroup per instance, which suits many small
- * problems, not a few large ones. */
+ * Jacobi: the streaming kernel that takes what fits no cluster of workgroups
+ * runs one workgroup per instance, which suits many small problems, not a few
+ * large ones. */
 #define BATCH_MAX_NODES 32768
 
 /* Whether bfm_sim_run takes the batched path: several instances, the batched

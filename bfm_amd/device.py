@@ -460,7 +460,7 @@ class _BatchSystem(System):
 
 
 class Batch:
-    """Systems solved together by one persistent launch per size class (include/bfmx.h)."""
+    """Systems solved together, by clusters of workgroups or one workgroup each (include/bfmx.h)."""
 
     def __init__(self, systems):
         self.systems = list(systems)   # kept alive with the batch

@@ -287,14 +287,15 @@ int bfmx_system_set_model(bfmx_system_t* s, bfmx_model_t* m);
 int bfmx_system_apply_model(bfmx_system_t* s, const double* r, double* z);
 
 /* ---- batched solves (no reference counterpart) -------------------------
- * Many systems (uneven sizes) solved by Jacobi or block-Jacobi PCG, one
- * workgroup per system, in one persistent launch per size class (systems of
- * < 2048, < 8192, >= 8192 nodes), the launches captured in one HIP graph.
+ * Many systems (uneven sizes) solved by Jacobi or block-Jacobi PCG, each by a
+ * cluster of workgroups or (what does not fit one) by one workgroup, in one
+ * persistent launch per size class (systems of < 2048, < 8192, >= 8192 nodes).
  * A batch holds either existing assembled systems (bfmx_batch_create) or
  * meshes that every launch assembles before solving
  * (bfmx_batch_create_planar). Systems of at most 262,144 nodes and nine blocks
  * a row are solved by clusters of workgroups that hold the matrix in registers,
- * whatever the configuration; configurations apply to the others. A configuration is a workgroup size x rows-per-thread pair:
+ * whatever the configuration; configurations apply to the others. A
+ * configuration is a workgroup size x rows-per-thread pair:
  * 0 = 256 x 1, 1 = 256 x 2, 2 = 512 x 1, 3 = 512 x 2, 4 = 1024 x 1. A
  * system's solution does not depend on the rest of the batch (bitwise, for
  * the same configuration). The systems must outlive the batch and stay
@@ -364,7 +365,7 @@ typedef struct {
  * pattern, element colouring; instances are spread over up to 16 threads)
  * and packs all device arrays into a few allocations. Each bfmx_batch_solve
  * launch then assembles K and the load of every instance, applies its
- * conditions and solves it, one workgroup per instance. The input arrays
+ * conditions and solves it. The input arrays
  * are copied; they need not outlive the call. */
 int bfmx_batch_create_planar(bfmx_batch_t** out, size_t n, const bfmx_instance_t* inst, int renumber);
 

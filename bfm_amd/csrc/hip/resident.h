@@ -285,6 +285,12 @@ struct Cluster {
 		left = r0 - lo;
 		own = r1 - r0;
 		halo = nwin - own;
+		// A workgroup without rows (a cluster may be larger than its system needs)
+		// has no window, yet multiplies its zero blocks by place 0: what was left
+		// there may be a NaN. Read behind the barriers of the caller's first steps.
+		if (nwin == 0 && t == 0) {
+			win[0] = dbl2{0, 0};
+		}
 		// a block past the row's end (its values are zero) takes place 0
 		auto place = [&](int k) { return k < len ? static_cast<uint32_t>(V.col[beg + k * kSlice] - lo) : 0u; };
 #pragma unroll

@@ -175,6 +175,24 @@ def test_batches_of_clusters(monkeypatch, pre):
         assert np.array_equal(one.get_u(0), u), k
 
 
+@pytest.mark.parametrize("pre", [D.PRECOND_JACOBI, D.PRECOND_BLOCK_JACOBI])
+def test_a_system_after_a_broken_one(pre):
+    """A cluster's size is rounded up: 28,700 and 29,000 nodes leave two and one of its 32 workgroups without rows.
+    They follow systems of NaN moduli on the same clusters (eight of 32 workgroups fill the GPU), whose NaNs stay
+    behind in the workgroups' memory; their runs are those of a batch without the broken ones."""
+    wide = strip(32000, 3, het=False)
+    bad = [D.beam_system(wide, material=dict(meshgen.BEAM_MATERIAL, E=float("nan"))) for _ in range(8)]
+    good = [D.beam_system(strip(n, 3, het=False)) for n in (29000, 28700)]
+    alone = D.Batch(good)
+    alone.solve(precond=pre, rtol=1e-6)
+    b = D.Batch(bad + good)
+    st, _ = b.solve(precond=pre, rtol=1e-6, check=False)
+    assert all(x["status"] == -4 for x in st[:8])
+    for k in range(2):
+        assert st[8 + k]["status"] == 0
+        assert np.array_equal(b.get_u(8 + k), alone.get_u(k))
+
+
 @pytest.mark.parametrize("nx,ny,kind", [(3, 2, 3), (16, 5, 4), (40, 10, 4), (42, 11, 3), (51, 9, 4), (60, 14, 4)])
 def test_minres(monkeypatch, nx, ny, kind):
     """Axisymmetric rings of 12 to 915 nodes (one workgroup of 512, and two) against the recurrences on the host;

@@ -1134,7 +1134,8 @@ int make_plan(bfmx_batch* b) {
 	auto words = [](double* p) { return reinterpret_cast<resident::u64*>(p); };
 	for (auto const& I : h) {
 		views.push_back(resident::View{I.slice_ptr, I.col, I.diag_blk, I.val, nullptr, I.b, I.x,
-		                               {words(I.r), words(I.z), words(I.q), words(I.p0)}, words(I.p1), I.dinv, I.n});
+		                               {words(I.r), words(I.z), words(I.q), words(I.p0)}, words(I.p1), I.dinv,
+		                               &b->d_out[views.size()].gave_up, I.n});
 	}
 	BFMX_CHECK(resident::plan_create(&b->plan, b->systems, views, b->stream));
 	if (b->plan && !resident::plan_rest(b->plan).empty()) {
@@ -1167,7 +1168,8 @@ int solve_resident(bfmx_batch* b, int pre, double rtol2, int64_t max_iter, const
 	BFMX_HIP(hipEventRecord(b->ev[0], b->stream));
 	launch_assemble(b);
 	resident::ClusterLock const lock(b->device);
-	BFMX_CHECK(resident::plan_launch(b->plan, b->stream, pre, rtol2, max_iter, b->d_out));
+	BFMX_CHECK(resident::plan_launch(b->plan, b->stream, pre, rtol2, max_iter, b->d_out,
+	                               static_cast<int>(b->h_out.size())));
 	const int32_t* at = b->d_rest;
 	for (int c = kClasses - 1; c >= 0; c--) {
 		if (b->rest_count[c] > 0) {
@@ -1181,7 +1183,7 @@ int solve_resident(bfmx_batch* b, int pre, double rtol2, int64_t max_iter, const
 	                        b->stream));
 	BFMX_HIP(hipStreamSynchronize(b->stream));
 	*ran = std::none_of(b->h_out.begin(), b->h_out.end(),
-	                    [](BatchOut const& o) { return o.status == resident::kFailed; });
+	                    [](BatchOut const& o) { return o.gave_up != 0; });
 	return BFMX_OK;
 }
 

@@ -81,6 +81,7 @@ struct alignas(128) Scalars {
 	int32_t stall;   // consecutive tolerance checks without halving the true residual
 	int32_t checking;// a tolerance check has failed: check at every chunk end
 	int32_t updates; // true-residual recomputations
+	int32_t gave_up; // a workgroup of a register-resident run ran out of polls (resident.h)
 };
 
 // Segmented flexible CG: a system whose convergence segments (at least kBlock
@@ -581,7 +582,8 @@ int vector_out(bfmx_system* s, const double* d_v, hipStream_t st, double* d_stag
 // resident.hip: point or block Jacobi PCG of s->d_bsolve in the solver's
 // buffers, with the matrix held in registers, from x = 0 or (warm) from
 // s->d_x; *ran is false (and nothing but the buffers changed) when the system
-// does not fit or the device could not run it. *out: the final scalars.
+// does not fit or the device could not run it: s->d_x is then as it was, or in
+// part or whole a later iterate, a start as good. *out: the final scalars.
 int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double delta2, int64_t cap, bool warm,
                  Scalars* out, bool* ran);
 // MINRES of s->d_bsolve the same way (status 0: iteration limit, 1: converged,

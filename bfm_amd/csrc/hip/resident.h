@@ -36,8 +36,11 @@
 // thread holds the device's ClusterLock from their launch to their end (an
 // ordinary launch under the lock costs 11 us with its synchronization, a
 // cooperative one 20 us). Between processes nothing prevents that, so every
-// wait is bounded (kSpinLimit polls): each workgroup ends whatever happens, and
-// the caller then solves with the streaming kernels.
+// wait is bounded (kSpinLimit polls): each workgroup ends whatever happens. A
+// vector's node that did not arrive counts as NaN, so that the sums end the run
+// in every workgroup; a workgroup whose wait ran out raises the launch's gave_up
+// flag, and the host then drops the run, whatever it reports, and solves with the
+// streaming kernels.
 #pragma once
 
 #include <mutex>
@@ -94,6 +97,7 @@ struct View {
 	u64* w[4];
 	u64* slots;
 	double* save;           // 4 doubles a node: r and p of a run cut at its iteration limit
+	int32_t* gave_up;       // set by a workgroup whose wait ran out; zeroed before the launch
 	int64_t n;
 };
 
@@ -175,7 +179,10 @@ struct Shared {
 	double tot[3][3][4];     // the gathered sums of up to four polling waves
 	int lo, hi;          // the window
 	int below, above;    // own rows before below or from above on lie in another workgroup's window
-	int failed;
+	int late;            // a wait for a vector's words or the windows ran out
+	int failed;          // a wait of an all-gather did: written between the two barriers of gather() only, so
+	                     // that all waves read the same after it
+	uint32_t polls;      // of one wait at most (set by the kernel; read where a wait goes on)
 };
 
 // Blocks of a row held in registers, by threads of the workgroup: six FP64
@@ -241,6 +248,7 @@ struct Cluster {
 			sh.hi = r1;
 			sh.below = 0;
 			sh.above = n;
+			sh.late = 0;
 			sh.failed = 0;
 		}
 		__syncthreads();
@@ -321,8 +329,8 @@ struct Cluster {
 				if (static_cast<uint32_t>(a) == sep && static_cast<uint32_t>(c) == sep) {
 					break;
 				}
-				if (++spin >= kSpinLimit) {
-					sh.failed = 1;
+				if (++spin >= sh.polls) {
+					sh.late = 1;
 					break;
 				}
 			}
@@ -345,12 +353,20 @@ struct Cluster {
 		a11 = top[2 * kSlice + 1];
 	}
 
+	// At the end of a run (a gather after the last wait made the flags visible).
+	__device__ __forceinline__ void report() const {
+		if (t == 0 && (sh.late || sh.failed)) {
+			*V.gave_up = 1;
+		}
+	}
+
 	// Addresses are formed anew in every iteration: held in registers they would
 	// push the matrix out.
 	__device__ __forceinline__ void forget_addresses() {
 		asm volatile("" : "+v"(t), "+v"(row));
 	}
 
+	// After a gather.
 	__device__ __forceinline__ bool failed() const {
 		return __builtin_amdgcn_readfirstlane(sh.failed) != 0;
 	}
@@ -386,8 +402,9 @@ struct Cluster {
 			    static_cast<uint32_t>(q2) == ep && static_cast<uint32_t>(q3) == ep) {
 				break;
 			}
-			if (++spin >= kSpinLimit) {
-				sh.failed = 1;
+			if (++spin >= sh.polls) {
+				sh.late = 1;
+				q0 = q1 = q2 = q3 = ~u64{0};   // NaN
 				break;
 			}
 		}
@@ -464,7 +481,7 @@ struct Cluster {
 					if (ok) {
 						break;
 					}
-					if (++spin >= kSpinLimit) {
+					if (++spin >= sh.polls) {
 						sh.failed = 1;
 						break;
 					}
@@ -569,7 +586,8 @@ struct Cluster {
 // the run's scalars (in every thread) and V.x the solution of the workgroup's
 // rows. lds: the spare blocks and the window. mode 0 starts from x = 0, 1 from
 // the x in V.x, 2 continues a run cut at its limit (R as it was left, r and p in
-// V.save). Runs until R.iter >= stop.
+// V.save). Runs until R.iter >= stop. A workgroup that left because a wait ran
+// out leaves its part of V.x as it was.
 template <typename MT, int W, int PRE, int NT>
 __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, double delta2, int64_t stop,
                         bool final_check, Shared& sh, dbl2* lds, Run& R) {
@@ -763,7 +781,8 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 		}
 	}
 	R.status = status;
-	if (C.live) {
+	C.report();
+	if (C.live && status != kFailed) {
 		st2(V.x + 2 * static_cast<int64_t>(C.row), x_get());
 		if (status == 0) {
 			st2(V.save + 2 * static_cast<int64_t>(C.row), r);
@@ -911,7 +930,8 @@ __device__ void run_minres(View const& V, int g, int G, bool fresh, double rtol,
 			}
 		}
 	}
-	if (C.live) {
+	C.report();
+	if (C.live && R.status != kFailed) {
 		int64_t const i = 2 * static_cast<int64_t>(C.row);
 		st2(V.x + i, x);
 		if (R.status == 0) {
@@ -953,6 +973,7 @@ struct Out {
 	double bb;
 	int32_t status;   // 1 converged, 2 breakdown, 3 stagnated, 0 iteration limit, kFailed
 	int32_t checks;
+	int32_t gave_up;  // a workgroup's wait ran out: the rest does not count
 };
 
 struct Plan;
@@ -964,8 +985,9 @@ void plan_destroy(Plan* p);
 // Systems the plan does not take, largest first.
 const std::vector<int32_t>& plan_rest(const Plan* p);
 // Queues the runs of the plan's systems (the caller holds a ClusterLock until
-// st is drained). A system whose status is kFailed afterwards was not solved.
-int plan_launch(Plan* p, hipStream_t st, int precond, double rtol2, int64_t max_iter, Out* d_out);
+// st is drained). If any of the n systems of d_out has gave_up set afterwards,
+// some of the plan's were not solved.
+int plan_launch(Plan* p, hipStream_t st, int precond, double rtol2, int64_t max_iter, Out* d_out, int n);
 
 }  // namespace resident
 }  // namespace bfmx

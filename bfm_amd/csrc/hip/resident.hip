@@ -26,13 +26,25 @@ __global__ __launch_bounds__(kBlock) void k_clear(View V, int64_t nw, int64_t ns
 	if (i < nslots) {
 		V.slots[i] = 0;
 	}
+	if (i == 0) {
+		*V.gave_up = 0;
+	}
+}
+
+// Polls of one wait (tests let waits run out early).
+uint32_t poll_limit() {
+	const char* e = std::getenv("BFMX_RESIDENT_POLLS");
+	return e && std::atoi(e) > 0 ? static_cast<uint32_t>(std::atoi(e)) : kSpinLimit;
 }
 
 template <typename MT, int W, int PRE, int NT>
-__global__ __launch_bounds__(NT) void k_resident_pcg(View V, int mode, double rtol2, double delta2, int64_t stop,
-                                                     Scalars* __restrict__ S) {
+__global__ __launch_bounds__(NT) void k_resident_pcg(View V, uint32_t polls, int mode, double rtol2,
+                                                     double delta2, int64_t stop, Scalars* __restrict__ S) {
 	extern __shared__ __align__(16) double dyn[];
 	__shared__ Shared sh;
+	if (threadIdx.x == 0) {
+		sh.polls = polls;
+	}
 	Run R;
 	if (mode == 2) {
 		R.rz = S->rz;
@@ -70,7 +82,7 @@ __global__ __launch_bounds__(NT) void k_resident_pcg(View V, int mode, double rt
 	}
 }
 
-typedef void (*PcgKernel)(View, int, double, double, int64_t, Scalars*);
+typedef void (*PcgKernel)(View, uint32_t, int, double, double, int64_t, Scalars*);
 
 template <typename MT, int W, int PRE>
 PcgKernel pick_threads(int nt) {
@@ -157,7 +169,8 @@ int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double d
 	int64_t const n = s->n_nodes;
 	auto words = [](double* p) { return reinterpret_cast<u64*>(p); };
 	View V{s->d_slice_ptr, s->d_col, s->d_diag_blk, s->d_val, s->d_val32, s->d_bsolve, s->d_x,
-	       {words(s->d_r), words(s->d_z), words(s->d_q), words(s->d_p[0])}, words(s->d_p[1]), s->d_dinv, n};
+	       {words(s->d_r), words(s->d_z), words(s->d_q), words(s->d_p[0])}, words(s->d_p[1]), s->d_dinv,
+	       &s->d_scal->gave_up, n};
 	int const nt = n <= 512 ? 512 : 1024;
 	PcgKernel const kernel = pick(mixed, s->res_width, precond, nt);
 	size_t const lds = static_cast<size_t>(s->res_window) * sizeof(resident::dbl2) + fixed(mixed, s->res_width, nt);
@@ -178,11 +191,11 @@ int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double d
 			lock.emplace(s->device);
 			k_clear<<<static_cast<int>((2 * n + kBlock - 1) / kBlock), kBlock, 0, st>>>(V, 2 * n, nslots);
 		}
-		kernel<<<G, nt, lds, st>>>(V, mode, rtol2, delta2, stop, s->d_scal);
+		kernel<<<G, nt, lds, st>>>(V, poll_limit(), mode, rtol2, delta2, stop, s->d_scal);
 		BFMX_HIP(hipGetLastError());
 		BFMX_HIP(hipMemcpyAsync(out, s->d_scal, sizeof(Scalars), hipMemcpyDeviceToHost, st));
 		BFMX_HIP(hipStreamSynchronize(st));
-		if (out->done == kFailed) {
+		if (G > 1 && out->gave_up) {
 			return BFMX_OK;
 		}
 		if (out->done != 0 || out->iter >= cap) {
@@ -204,12 +217,22 @@ namespace {
 
 constexpr int kMinresThreads = 512;
 
+// What a launch leaves.
+struct MinresState {
+	MinresRun run;
+	int32_t gave_up;
+};
+
 template <int W>
-__global__ __launch_bounds__(kMinresThreads) void k_resident_minres(View V, int fresh, double rtol, int64_t stop,
-                                                                    int64_t cap, double* __restrict__ more,
+__global__ __launch_bounds__(kMinresThreads) void k_resident_minres(View V, uint32_t polls, int fresh, double rtol,
+                                                                    int64_t stop, int64_t cap,
+                                                                    double* __restrict__ more,
                                                                     MinresRun* __restrict__ run) {
 	extern __shared__ __align__(16) double dyn[];
 	__shared__ Shared sh;
+	if (threadIdx.x == 0) {
+		sh.polls = polls;
+	}
 	MinresRun R;
 	if (!fresh) {
 		R = *run;
@@ -234,14 +257,17 @@ int resident_minres(bfmx_system* s, double rtol, int64_t cap, MinresResult* out,
 	}
 	hipStream_t const st = s->stream;
 	double* more = nullptr;       // w and w2 of a run cut at its limit
-	MinresRun* d_run = nullptr;
-	MinresRun R{};
+	MinresState* d_run = nullptr;
+	MinresState last{};
+	MinresRun& R = last.run;
+	bool gave_up = false;
 	int const rc = [&]() -> int {
 		BFMX_CHECK(palloc(&more, 4 * static_cast<size_t>(n)));
 		BFMX_CHECK(palloc(&d_run, 1));
 		auto words = [](double* p) { return reinterpret_cast<u64*>(p); };
 		View V{s->d_slice_ptr, s->d_col, s->d_diag_blk, s->d_val, nullptr, s->d_bsolve, s->d_x,
-		       {words(s->d_r), words(s->d_z), words(s->d_q), words(s->d_p[0])}, words(s->d_p[1]), s->d_dinv, n};
+		       {words(s->d_r), words(s->d_z), words(s->d_q), words(s->d_p[0])}, words(s->d_p[1]), s->d_dinv,
+		       &d_run->gave_up, n};
 		int const width = *std::max_element(s->row_len.begin(), s->row_len.end());
 		auto const kernel = width <= 7 ? k_resident_minres<7> : k_resident_minres<9>;
 		size_t const lds = static_cast<size_t>(win) * sizeof(resident::dbl2);
@@ -251,7 +277,7 @@ int resident_minres(bfmx_system* s, double rtol, int64_t cap, MinresResult* out,
 		}
 		const char* cut = std::getenv("BFMX_RESIDENT_ITERS");
 		int64_t const per_launch = cut && std::atoll(cut) > 0 ? std::atoll(cut) : kPerLaunch;
-		for (int fresh = 1; R.status == 0 && (fresh || R.iter < cap); fresh = 0) {
+		for (int fresh = 1; !gave_up && R.status == 0 && (fresh || R.iter < cap); fresh = 0) {
 			int64_t const stop = std::min(cap, R.iter + per_launch);
 			std::optional<ClusterLock> lock;
 			if (G > 1) {
@@ -259,10 +285,12 @@ int resident_minres(bfmx_system* s, double rtol, int64_t cap, MinresResult* out,
 				k_clear<<<static_cast<int>((2 * n + kBlock - 1) / kBlock), kBlock, 0, st>>>(V, 2 * n,
 				                                                                         2 * G * kSlotWords);
 			}
-			kernel<<<static_cast<unsigned>(G), kMinresThreads, lds, st>>>(V, fresh, rtol, stop, cap, more, d_run);
+			kernel<<<static_cast<unsigned>(G), kMinresThreads, lds, st>>>(V, poll_limit(), fresh, rtol, stop, cap, more,
+			                                                              &d_run->run);
 			BFMX_HIP(hipGetLastError());
-			BFMX_HIP(hipMemcpyAsync(&R, d_run, sizeof R, hipMemcpyDeviceToHost, st));
+			BFMX_HIP(hipMemcpyAsync(&last, d_run, sizeof last, hipMemcpyDeviceToHost, st));
 			BFMX_HIP(hipStreamSynchronize(st));
+			gave_up = G > 1 && last.gave_up;
 		}
 		return BFMX_OK;
 	}();
@@ -270,7 +298,7 @@ int resident_minres(bfmx_system* s, double rtol, int64_t cap, MinresResult* out,
 	pfree(more);
 	pfree(d_run);
 	BFMX_CHECK(rc);
-	*ran = R.status != kFailed;
+	*ran = !gave_up;
 	*out = MinresResult{R.status, R.iter, R.rr, R.bb, R.checks};
 	return BFMX_OK;
 }
@@ -307,7 +335,7 @@ __global__ __launch_bounds__(kBlock) void k_clear_batch(const View* __restrict__
                                                         const int32_t* __restrict__ order,
                                                         const int32_t* __restrict__ groups,
                                                         Queue* __restrict__ queues, int nq, u64* __restrict__ post,
-                                                        int npost) {
+                                                        int npost, Out* __restrict__ out, int nout) {
 	int const k = blockIdx.x / kClearParts, part = blockIdx.x % kClearParts;
 	int const gid = part * kBlock + threadIdx.x, step = kClearParts * kBlock;
 	if (k == 0) {
@@ -316,6 +344,9 @@ __global__ __launch_bounds__(kBlock) void k_clear_batch(const View* __restrict__
 		}
 		for (int i = gid; i < npost; i += step) {
 			post[i] = 0;
+		}
+		for (int i = gid; i < nout; i += step) {
+			out[i].gave_up = 0;
 		}
 	}
 	int const G = groups[k];
@@ -336,10 +367,14 @@ __global__ __launch_bounds__(kRows) void k_resident_batch(const View* __restrict
                                                           const int32_t* __restrict__ order,
                                                           const Member* __restrict__ members,
                                                           Queue* __restrict__ queues, u64* __restrict__ post,
-                                                          double rtol2, int64_t max_iter, Out* __restrict__ out) {
+                                                          uint32_t polls, double rtol2, int64_t max_iter,
+                                                          Out* __restrict__ out) {
 	extern __shared__ __align__(16) double dyn[];
 	__shared__ Shared sh;
 	__shared__ int job;
+	if (threadIdx.x == 0) {
+		sh.polls = polls;
+	}
 	Member const M = members[blockIdx.x];
 	for (uint32_t round = 1;; round++) {
 		if (threadIdx.x == 0) {
@@ -353,7 +388,7 @@ __global__ __launch_bounds__(kRows) void k_resident_batch(const View* __restrict
 					put(at, (static_cast<u64>(static_cast<uint32_t>(k)) << 32) | round);
 				}
 			} else {
-				for (uint32_t spin = 0; spin < kSpinLimit; spin++) {
+				for (uint32_t spin = 0; spin < sh.polls; spin++) {
 					u64 const v = get(at);
 					if (static_cast<uint32_t>(v) == round) {
 						k = static_cast<int>(v >> 32);
@@ -582,7 +617,7 @@ int plan_create(Plan** out, const std::vector<bfmx_system*>& systems, const std:
 	return BFMX_OK;
 }
 
-int plan_launch(Plan* p, hipStream_t st, int precond, double rtol2, int64_t max_iter, Out* d_out) {
+int plan_launch(Plan* p, hipStream_t st, int precond, double rtol2, int64_t max_iter, Out* d_out, int n) {
 	bool const point = precond == BFMX_PRECOND_JACOBI;
 	auto const kernel = p->width <= 7
 	                        ? (point ? k_resident_batch<7, BFMX_PRECOND_JACOBI> : k_resident_batch<7, BFMX_PRECOND_BLOCK_JACOBI>)
@@ -590,11 +625,11 @@ int plan_launch(Plan* p, hipStream_t st, int precond, double rtol2, int64_t max_
 	BFMX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
 	                             static_cast<int>(p->lds)));
 	k_clear_batch<<<p->taken * kClearParts, kBlock, 0, st>>>(p->d_views, p->d_order, p->d_groups, p->d_queues, p->queues,
-	                                                   p->d_post, p->clusters);
+	                                                         p->d_post, p->clusters, d_out, n);
 	BFMX_HIP(hipGetLastError());
 	for (auto const& L : p->launches) {
 		kernel<<<L.blocks, kRows, p->lds, st>>>(p->d_views, p->d_order, p->d_members + L.first, p->d_queues, p->d_post,
-		                                        rtol2, max_iter, d_out);
+		                                        poll_limit(), rtol2, max_iter, d_out);
 		BFMX_HIP(hipGetLastError());
 	}
 	return BFMX_OK;

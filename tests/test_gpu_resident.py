@@ -10,6 +10,7 @@ import threading
 import numpy as np
 import pytest
 
+import mpnn as M
 from conftest import rel_err
 
 from bfm_amd import device as D
@@ -193,20 +194,75 @@ def test_a_system_after_a_broken_one(pre):
         assert np.array_equal(b.get_u(8 + k), alone.get_u(k))
 
 
-@pytest.mark.parametrize("nx,ny,kind", [(3, 2, 3), (16, 5, 4), (40, 10, 4), (42, 11, 3), (51, 9, 4), (60, 14, 4)])
-def test_minres(monkeypatch, nx, ny, kind):
-    """Axisymmetric rings of 12 to 915 nodes (one workgroup of 512, and two) against the recurrences on the host;
-    a run cut into launches is the same run. K is indefinite with a condition number of about 1e5 here: two
-    solutions whose residuals meet 1e-8 agree to 1e-3; seen 1e-9."""
+def ring(nx, ny, kind=4):
+    """An axisymmetric ring (indefinite: MINRES)."""
     m = meshgen.beam(nx, ny, kind=kind, length=4.0, height=1.0, jitter=0.2, seed=12)
     m.coords = m.coords + np.array([1.0, 0.0])
     s = D.System.from_mesh(m)
     s.assemble(D.AXISYMMETRIC, 2.0e11, 0.3, 7850.0, g=(0.0, -9.81))
     sets = m.node_sets
     s.apply_conditions([1, 0, 3], [0.0, 0.0, -1e6], [sets["bottom"], sets["left"], sets["top"]])
+    return s
+
+
+# A wait that runs out is forced by a limit of one poll: every workgroup still ends, some of them on sums to which a
+# failed one contributed. What comes back is bitwise the streaming kernels' solution and report.
+
+@pytest.mark.parametrize("pre,precision,nx", [(D.PRECOND_JACOBI, D.FP64, 80), (D.PRECOND_BLOCK_JACOBI, D.FP64, 500),
+                                              (D.PRECOND_JACOBI, D.MIXED, 120), (D.PRECOND_MINRES, D.FP64, 60)])
+def test_a_wait_that_runs_out(monkeypatch, pre, precision, nx):
+    s = ring(nx, 14) if pre == D.PRECOND_MINRES else D.beam_system(meshgen.beam(nx, 20, kind=4, jitter=0.2, seed=3))
+    kw = dict(precond=pre, precision=precision, rtol=1e-7)
+    ref, st_ref, u, st = both(monkeypatch, s, **kw)
+    assert not np.array_equal(u, ref)          # the two paths differ in rounding
+    monkeypatch.setenv("BFMX_RESIDENT_POLLS", "1")
+    got, st_got = s.solve(**kw)
+    assert np.array_equal(got, ref)
+    assert [st_got[k] for k in ("status", "iterations", "rel_residual", "restarts")] == \
+        [st_ref[k] for k in ("status", "iterations", "rel_residual", "restarts")]
+
+
+def test_a_wait_that_runs_out_in_a_warm_start(monkeypatch):
+    """The learned solve's block-Jacobi run from the iterate where a network that returns NaN broke down."""
+    s = D.beam_system(meshgen.beam(80, 20, kind=4, jitter=0.2, seed=3))
+    m = D.Model(seed=5)
+    p = m.get_params()
+    p[M.OFF_W0 + 3] = np.nan
+    m.set_params(p)
+    s.set_model(m)
+    kw = dict(precond=D.PRECOND_LEARNED, rtol=1e-7)
+    ref, st_ref, u, st = both(monkeypatch, s, **kw)
+    assert st["fallback"] == 1 and not np.array_equal(u, ref)
+    monkeypatch.setenv("BFMX_RESIDENT_POLLS", "1")
+    got, st_got = s.solve(**kw)
+    assert np.array_equal(got, ref) and st_got["iterations"] == st_ref["iterations"]
+
+
+def test_a_wait_that_runs_out_in_a_batch(monkeypatch):
+    systems = [D.beam_system(strip(n, 3 + k % 2, het=False, seed=k))
+               for k, n in enumerate((64, 1026, 2050, 5000, 5100, 9000, 20600, 30002, 30002))]
+    b = D.Batch(systems)
+    monkeypatch.setenv("BFMX_RESIDENT", "0")
+    st_ref, _ = b.solve(rtol=1e-6)
+    ref = [b.get_u(k) for k in range(len(systems))]
+    monkeypatch.delenv("BFMX_RESIDENT")
+    monkeypatch.setenv("BFMX_RESIDENT_POLLS", "1")
+    st, _ = b.solve(rtol=1e-6)
+    for k in range(len(systems)):
+        assert [st[k][x] for x in ("status", "iterations", "rel_residual")] == \
+            [st_ref[k][x] for x in ("status", "iterations", "rel_residual")], k
+        assert np.array_equal(b.get_u(k), ref[k]), k
+
+
+@pytest.mark.parametrize("nx,ny,kind", [(3, 2, 3), (16, 5, 4), (40, 10, 4), (42, 11, 3), (51, 9, 4), (60, 14, 4)])
+def test_minres(monkeypatch, nx, ny, kind):
+    """Axisymmetric rings of 12 to 915 nodes (one workgroup of 512, and two) against the recurrences on the host;
+    a run cut into launches is the same run. K is indefinite with a condition number of about 1e5 here: two
+    solutions whose residuals meet 1e-8 agree to 1e-3; seen 1e-9."""
+    s = ring(nx, ny, kind)
     kw = dict(precond=D.PRECOND_MINRES, rtol=1e-8)
     ref, st_ref, u, st = both(monkeypatch, s, **kw)
-    print(f"{m.n_nodes} nodes: {st_ref['iterations']} / {st['iterations']} iterations, difference {rel_err(u, ref):.1e}")
+    print(f"{s.n_nodes} nodes: {st_ref['iterations']} / {st['iterations']} iterations, difference {rel_err(u, ref):.1e}")
     assert abs(st["iterations"] - st_ref["iterations"]) <= 0.1 * st_ref["iterations"] + 10
     A, b = s.get_csr_scipy(), s.get_rhs()
     assert st["status"] == 0 and np.linalg.norm(b - A @ u) <= 1.1e-8 * np.linalg.norm(b)

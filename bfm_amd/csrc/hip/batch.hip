@@ -638,6 +638,7 @@ struct bfmx_batch {
 	// fit, made at the first solve; the streaming kernel takes the others
 	bool planned = false;
 	bfmx::resident::Plan* plan = nullptr;
+	std::chrono::steady_clock::time_point res_retry{};   // no clusters before this time
 	int32_t* d_rest = nullptr;              // those others, by class, largest first
 	int rest_count[bfmx::kClasses] = {};
 	// batches built from meshes: the systems are the batch's own (host
@@ -1158,7 +1159,7 @@ int make_plan(bfmx_batch* b) {
 int solve_resident(bfmx_batch* b, int pre, double rtol2, int64_t max_iter, const int* picks, bool* ran) {
 	*ran = false;
 	const char* e = std::getenv("BFMX_RESIDENT");
-	if (e && e[0] == '0') {
+	if ((e && e[0] == '0') || std::chrono::steady_clock::now() < b->res_retry) {
 		return BFMX_OK;
 	}
 	BFMX_CHECK(make_plan(b));
@@ -1184,6 +1185,9 @@ int solve_resident(bfmx_batch* b, int pre, double rtol2, int64_t max_iter, const
 	BFMX_HIP(hipStreamSynchronize(b->stream));
 	*ran = std::none_of(b->h_out.begin(), b->h_out.end(),
 	                    [](BatchOut const& o) { return o.gave_up != 0; });
+	if (!*ran) {
+		b->res_retry = std::chrono::steady_clock::now() + resident::kRetryAfter;
+	}
 	return BFMX_OK;
 }
 

@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdarg>
+#include <chrono>
 #include <cstdint>
 #include <cstdio>
 #include <functional>
@@ -398,6 +399,7 @@ struct bfmx_system {
 	int res_groups = -1;
 	int res_window = 0;
 	int res_width = 0;
+	std::chrono::steady_clock::time_point res_retry{};   // not tried before this time (resident.h)
 
 	bool assembled = false;
 	bool finalized = false;

@@ -43,6 +43,7 @@
 // streaming kernels.
 #pragma once
 
+#include <chrono>
 #include <mutex>
 
 #include "internal.h"
@@ -82,6 +83,9 @@ constexpr int kMaxWidth = 9;                // blocks of a row held in registers
 constexpr int kCheckEvery = 16;             // iterations between true-residual checks once one has failed
 constexpr int kStall = 8;                   // such checks without halving before the run counts as stalled
 constexpr int kFailed = 5;                  // status: a bounded wait ran out
+// A wait runs out after seconds, when something else holds the GPU's CUs: the
+// system's or batch's solves of the next minute stream without trying again.
+constexpr std::chrono::seconds kRetryAfter{60};
 
 // One system's arrays. The exchange uses the solver's vector buffers (16
 // bytes a node each): words 0 and 1, 2 and 3 of the two parities in w[0..3],

@@ -152,6 +152,9 @@ int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double d
 	if ((e && e[0] == '0') || s->n_conv_seg > 0 || (precond != BFMX_PRECOND_JACOBI && precond != BFMX_PRECOND_BLOCK_JACOBI)) {
 		return BFMX_OK;
 	}
+	if (std::chrono::steady_clock::now() < s->res_retry) {
+		return BFMX_OK;
+	}
 	if (s->res_groups < 0) {
 		int64_t const groups = (s->n_nodes + kRows - 1) / kRows;
 		s->res_window = groups <= compute_units(s->device) ? window_of(s, groups) : 0;
@@ -196,6 +199,7 @@ int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double d
 		BFMX_HIP(hipMemcpyAsync(out, s->d_scal, sizeof(Scalars), hipMemcpyDeviceToHost, st));
 		BFMX_HIP(hipStreamSynchronize(st));
 		if (G > 1 && out->gave_up) {
+			s->res_retry = std::chrono::steady_clock::now() + kRetryAfter;
 			return BFMX_OK;
 		}
 		if (out->done != 0 || out->iter >= cap) {
@@ -251,7 +255,8 @@ int resident_minres(bfmx_system* s, double rtol, int64_t cap, MinresResult* out,
 	*ran = false;
 	const char* e = std::getenv("BFMX_RESIDENT");
 	int64_t const n = s->n_nodes, G = (n + kMinresThreads - 1) / kMinresThreads;
-	int const win = (e && e[0] == '0') || G > compute_units(s->device) ? 0 : window_of(s, G, kMinresThreads);
+	bool const off = (e && e[0] == '0') || std::chrono::steady_clock::now() < s->res_retry;
+	int const win = off || G > compute_units(s->device) ? 0 : window_of(s, G, kMinresThreads);
 	if (win == 0) {
 		return BFMX_OK;
 	}
@@ -291,6 +296,9 @@ int resident_minres(bfmx_system* s, double rtol, int64_t cap, MinresResult* out,
 			BFMX_HIP(hipMemcpyAsync(&last, d_run, sizeof last, hipMemcpyDeviceToHost, st));
 			BFMX_HIP(hipStreamSynchronize(st));
 			gave_up = G > 1 && last.gave_up;
+			if (gave_up) {
+				s->res_retry = std::chrono::steady_clock::now() + kRetryAfter;
+			}
 		}
 		return BFMX_OK;
 	}();

@@ -186,7 +186,7 @@ int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double d
 	int64_t const per_launch = cut && std::atoll(cut) > 0 ? std::atoll(cut) : kPerLaunch;
 	int64_t const nslots = G > 1 ? 2 * static_cast<int64_t>(G) * kSlotWords : 0;
 	int mode = warm ? 1 : 0;
-	cap = (cap + kCheckEvery - 1) / kCheckEvery * kCheckEvery;
+	cap = (std::min(cap, INT64_MAX - kCheckEvery) + kCheckEvery - 1) / kCheckEvery * kCheckEvery;
 	while (true) {
 		int64_t const stop = std::min(cap, (mode == 2 ? out->iter : 0) + per_launch);
 		std::optional<ClusterLock> lock;

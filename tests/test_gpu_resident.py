@@ -125,6 +125,9 @@ def test_zero_load_limit_and_floor():
     with pytest.raises(D.BfmxError) as e:
         s.solve(rtol=1e-17)
     assert e.value.code == -8
+    u, st = s.solve(rtol=RTOL)
+    u2, st2 = s.solve(rtol=RTOL, max_iter=2**63 - 1)   # as good as no limit
+    assert st2["status"] == 0 and np.array_equal(u, u2)
 
 
 def test_clusters_on_several_threads():

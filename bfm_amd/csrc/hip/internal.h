@@ -585,9 +585,10 @@ int vector_out(bfmx_system* s, const double* d_v, hipStream_t st, double* d_stag
 // buffers, with the matrix held in registers, from x = 0 or (warm) from
 // s->d_x; *ran is false (and nothing but the buffers changed) when the system
 // does not fit or the device could not run it: s->d_x is then as it was, or in
-// part or whole a later iterate, a start as good. *out: the final scalars.
+// part or whole a later iterate, a start as good. no_scratch: with a kernel that
+// needs no scratch memory. *out: the final scalars.
 int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double delta2, int64_t cap, bool warm,
-                 Scalars* out, bool* ran);
+                 bool no_scratch, Scalars* out, bool* ran);
 // MINRES of s->d_bsolve the same way (status 0: iteration limit, 1: converged,
 // 2: breakdown, 3: exhausted above rtol).
 struct MinresResult {

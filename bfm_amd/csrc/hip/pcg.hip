@@ -1067,7 +1067,7 @@ int run_chunks(bfmx_system* s, int precond, bool mixed, double rtol2, int64_t ca
 	if (!is_fcg(precond)) {
 		// in one launch, where the matrix fits the GPU's registers
 		bool ran = false;
-		BFMX_CHECK(resident_pcg(s, precond, mixed, rtol2, mixed ? kDelta2 : 0.0, cap, warm, out, &ran));
+		BFMX_CHECK(resident_pcg(s, precond, mixed, rtol2, mixed ? kDelta2 : 0.0, cap, warm, false, out, &ran));
 		if (ran) {
 			return BFMX_OK;
 		}
@@ -1825,7 +1825,7 @@ int pcg_in_buffers(bfmx_system* s, PcgBuffers const& w, int precond, double rtol
 	s->d_scal = w.scal;
 	double const rtol2 = rtol * rtol;
 	bool ran = false;
-	BFMX_CHECK(resident_pcg(s, precond, false, rtol2, 0.0, cap, false, out, &ran));
+	BFMX_CHECK(resident_pcg(s, precond, false, rtol2, 0.0, cap, false, true, out, &ran));
 	if (ran) {
 		return BFMX_OK;
 	}

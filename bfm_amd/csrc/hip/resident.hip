@@ -37,7 +37,7 @@ uint32_t poll_limit() {
 	return e && std::atoi(e) > 0 ? static_cast<uint32_t>(std::atoi(e)) : kSpinLimit;
 }
 
-template <typename MT, int W, int PRE, int NT>
+template <typename MT, int W, int PRE, int NT, bool LEAN>
 __global__ __launch_bounds__(NT) void k_resident_pcg(View V, uint32_t polls, int mode, double rtol2,
                                                      double delta2, int64_t stop, Scalars* __restrict__ S) {
 	extern __shared__ __align__(16) double dyn[];
@@ -62,7 +62,7 @@ __global__ __launch_bounds__(NT) void k_resident_pcg(View V, uint32_t polls, int
 		R.updates = S->updates;
 		R.checks = S->updates - 1;
 	}
-	run_pcg<MT, W, PRE, NT>(V, blockIdx.x, gridDim.x, mode, rtol2, delta2, stop, false, sh,
+	run_pcg<MT, W, PRE, NT, LEAN>(V, blockIdx.x, gridDim.x, mode, rtol2, delta2, stop, false, sh,
 	                        reinterpret_cast<resident::dbl2*>(dyn), R);
 	if (blockIdx.x == 0 && threadIdx.x == 0) {
 		S->rz = R.rz;
@@ -86,7 +86,7 @@ typedef void (*PcgKernel)(View, uint32_t, int, double, double, int64_t, Scalars*
 
 template <typename MT, int W, int PRE>
 PcgKernel pick_threads(int nt) {
-	return nt == 512 ? k_resident_pcg<MT, W, PRE, 512> : k_resident_pcg<MT, W, PRE, 1024>;
+	return nt == 512 ? k_resident_pcg<MT, W, PRE, 512, false> : k_resident_pcg<MT, W, PRE, 1024, false>;
 }
 
 template <typename MT, int W>
@@ -95,7 +95,12 @@ PcgKernel pick_precond(int pre, int nt) {
 	                                  : pick_threads<MT, W, BFMX_PRECOND_BLOCK_JACOBI>(nt);
 }
 
-PcgKernel pick(bool mixed, int width, int pre, int nt) {
+// no_scratch: a kernel that spills no register.
+PcgKernel pick(bool mixed, int width, int pre, int nt, bool no_scratch) {
+	if (no_scratch && !mixed && pre == BFMX_PRECOND_BLOCK_JACOBI && nt == 1024) {
+		return width <= 7 ? k_resident_pcg<double, 7, BFMX_PRECOND_BLOCK_JACOBI, 1024, true>
+		                  : k_resident_pcg<double, 9, BFMX_PRECOND_BLOCK_JACOBI, 1024, true>;
+	}
 	if (mixed) {
 		return width <= 7 ? pick_precond<float, 7>(pre, nt) : pick_precond<float, 9>(pre, nt);
 	}
@@ -146,7 +151,7 @@ int window_of(const bfmx_system* s, int64_t G, int threads) {
 }  // namespace resident
 
 int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double delta2, int64_t cap, bool warm,
-                 Scalars* out, bool* ran) {
+                 bool no_scratch, Scalars* out, bool* ran) {
 	*ran = false;
 	const char* e = std::getenv("BFMX_RESIDENT");
 	if ((e && e[0] == '0') || s->n_conv_seg > 0 || (precond != BFMX_PRECOND_JACOBI && precond != BFMX_PRECOND_BLOCK_JACOBI)) {
@@ -175,7 +180,7 @@ int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double d
 	       {words(s->d_r), words(s->d_z), words(s->d_q), words(s->d_p[0])}, words(s->d_p[1]), s->d_dinv,
 	       &s->d_scal->gave_up, n};
 	int const nt = n <= 512 ? 512 : 1024;
-	PcgKernel const kernel = pick(mixed, s->res_width, precond, nt);
+	PcgKernel const kernel = pick(mixed, s->res_width, precond, nt, no_scratch);
 	size_t const lds = static_cast<size_t>(s->res_window) * sizeof(resident::dbl2) + fixed(mixed, s->res_width, nt);
 	if (lds > 48 * 1024) {
 		BFMX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),

@@ -1168,7 +1168,7 @@ int solve_resident(bfmx_batch* b, int pre, double rtol2, int64_t max_iter, const
 	}
 	BFMX_HIP(hipEventRecord(b->ev[0], b->stream));
 	launch_assemble(b);
-	resident::ClusterLock const lock(b->device);
+	resident::ClusterLock const lock(b->device, resident::plan_workgroups(b->plan));
 	BFMX_CHECK(resident::plan_launch(b->plan, b->stream, pre, rtol2, max_iter, b->d_out,
 	                               static_cast<int>(b->h_out.size())));
 	const int32_t* at = b->d_rest;

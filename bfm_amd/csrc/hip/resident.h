@@ -33,9 +33,9 @@
 // The workgroups of a cluster must be resident together. A launch has at most
 // one workgroup a CU, kernels on other streams end and leave their CUs to it,
 // and clusters that could wait for each other's CUs do not run at once: a host
-// thread holds the device's ClusterLock from their launch to their end (an
-// ordinary launch under the lock costs 11 us with its synchronization, a
-// cooperative one 20 us). Between processes nothing prevents that, so every
+// thread holds a ClusterLock for their CUs (cu_budget.h) from their launch to
+// their end (an ordinary launch under the lock costs 11 us with its
+// synchronization, a cooperative one 20 us). Between processes nothing prevents that, so every
 // wait is bounded (kSpinLimit polls): each workgroup ends whatever happens. A
 // vector's node that did not arrive counts as NaN, so that the sums end the run
 // in every workgroup; a workgroup whose wait ran out raises the launch's gave_up
@@ -44,8 +44,8 @@
 #pragma once
 
 #include <chrono>
-#include <mutex>
 
+#include "cu_budget.h"
 #include "internal.h"
 
 namespace bfmx {
@@ -962,14 +962,18 @@ constexpr int kRows = 1024;
 // Compute units of a device: the most workgroups of a launch of clusters.
 int compute_units(int device);
 
-// One thread at a time launches clusters of several workgroups on a device; it
-// holds this until they have ended (its stream drained).
+// Held by a thread from its launch of `workgroups` workgroups in clusters until
+// they have ended (its stream drained).
 class ClusterLock {
 public:
-	explicit ClusterLock(int device);
+	ClusterLock(int device, int64_t workgroups);
+	~ClusterLock();
+	ClusterLock(ClusterLock const&) = delete;
+	ClusterLock& operator=(ClusterLock const&) = delete;
 
 private:
-	std::unique_lock<std::mutex> m_lock;
+	CuBudget& m_budget;
+	int const m_share;
 };
 
 // The nodes of the widest window when G workgroups of at most `threads` rows
@@ -997,8 +1001,10 @@ int plan_create(Plan** out, const std::vector<bfmx_system*>& systems, const std:
 void plan_destroy(Plan* p);
 // Systems the plan does not take, largest first.
 const std::vector<int32_t>& plan_rest(const Plan* p);
-// Queues the runs of the plan's systems (the caller holds a ClusterLock until
-// st is drained). If any of the n systems of d_out has gave_up set afterwards,
+// Workgroups of the plan's largest launch.
+int plan_workgroups(const Plan* p);
+// Queues the runs of the plan's systems (the caller holds a ClusterLock for
+// plan_workgroups until st is drained). If any of the n systems of d_out has gave_up set afterwards,
 // some of the plan's were not solved.
 int plan_launch(Plan* p, hipStream_t st, int precond, double rtol2, int64_t max_iter, Out* d_out, int n);
 

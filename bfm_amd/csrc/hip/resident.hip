@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <map>
 #include <optional>
 
 #include "resident.h"
@@ -121,9 +122,25 @@ int compute_units(int device) {
 	return hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess ? cus : 0;
 }
 
-ClusterLock::ClusterLock(int device) {
-	static std::mutex m[64];   // of the devices; two that share one only wait for each other
-	m_lock = std::unique_lock<std::mutex>(m[device & 63]);
+namespace {
+
+CuBudget& budget_of(int device) {
+	static std::mutex m;
+	// never destroyed: threads may still hold shares while the process exits
+	static auto* budgets = new std::map<int, CuBudget>;
+	std::lock_guard<std::mutex> const lock(m);
+	return budgets->try_emplace(device, compute_units(device)).first->second;
+}
+
+}  // namespace
+
+ClusterLock::ClusterLock(int device, int64_t workgroups)
+    : m_budget(budget_of(device)), m_share(CuBudget::share(workgroups)) {
+	m_budget.take(m_share);
+}
+
+ClusterLock::~ClusterLock() {
+	m_budget.give(m_share);
 }
 
 int window_of(const bfmx_system* s, int64_t G, int threads) {
@@ -196,7 +213,7 @@ int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double d
 		int64_t const stop = std::min(cap, (mode == 2 ? out->iter : 0) + per_launch);
 		std::optional<ClusterLock> lock;
 		if (G > 1) {
-			lock.emplace(s->device);
+			lock.emplace(s->device, G);
 			k_clear<<<static_cast<int>((2 * n + kBlock - 1) / kBlock), kBlock, 0, st>>>(V, 2 * n, nslots);
 		}
 		kernel<<<G, nt, lds, st>>>(V, poll_limit(), mode, rtol2, delta2, stop, s->d_scal);
@@ -291,7 +308,7 @@ int resident_minres(bfmx_system* s, double rtol, int64_t cap, MinresResult* out,
 			int64_t const stop = std::min(cap, R.iter + per_launch);
 			std::optional<ClusterLock> lock;
 			if (G > 1) {
-				lock.emplace(s->device);
+				lock.emplace(s->device, G);
 				k_clear<<<static_cast<int>((2 * n + kBlock - 1) / kBlock), kBlock, 0, st>>>(V, 2 * n,
 				                                                                         2 * G * kSlotWords);
 			}
@@ -499,6 +516,7 @@ struct Plan {
 	std::vector<Launch> launches;
 	std::vector<int32_t> rest;
 	int taken = 0, queues = 0, clusters = 0, width = 0;
+	int workgroups = 0;   // of the largest launch
 	size_t lds = 0;
 	View* d_views = nullptr;
 	int32_t* d_order = nullptr;
@@ -523,6 +541,10 @@ void plan_destroy(Plan* p) {
 
 const std::vector<int32_t>& plan_rest(const Plan* p) {
 	return p->rest;
+}
+
+int plan_workgroups(const Plan* p) {
+	return p->workgroups;
 }
 
 int plan_create(Plan** out, const std::vector<bfmx_system*>& systems, const std::vector<View>& views,
@@ -601,7 +623,9 @@ int plan_create(Plan** out, const std::vector<bfmx_system*>& systems, const std:
 			}
 			queues.push_back(Queue{begin, static_cast<int32_t>(order.size()), begin, 0});
 		}
-		p->launches.push_back(Plan::Launch{first, static_cast<int>(members.size()) - first});
+		int const blocks = static_cast<int>(members.size()) - first;
+		p->launches.push_back(Plan::Launch{first, blocks});
+		p->workgroups = std::max(p->workgroups, blocks);
 	}
 	p->queues = static_cast<int>(queues.size());
 	int const rc = [&]() -> int {

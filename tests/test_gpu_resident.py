@@ -6,6 +6,7 @@ compared to 1e-6, a hundred times what was seen, and the residual of the
 register-resident solution is formed again from the matrix."""
 
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -146,6 +147,64 @@ def test_clusters_on_several_threads():
     for t in threads:
         t.join()
     assert all(np.array_equal(a, g) for a, g in zip(alone, got))
+
+
+def test_clusters_beside_each_other():
+    """Clusters of 2 to 59 workgroups from twelve threads and a batch: each run is its own, bitwise, so that no
+    wait ran out."""
+    systems = [D.beam_system(meshgen.beam(60 + 50 * k, 20 + 7 * k, kind=3 + k % 2, jitter=0.2, seed=k))
+               for k in range(12)]
+    alone = [s.solve(rtol=1e-5)[0] for s in systems]
+    batch = D.Batch(systems[::4])
+    batch.solve(rtol=1e-5)
+    in_batch = [batch.get_u(k) for k in range(3)]
+    wrong = []
+
+    def work(k):
+        for _ in range(6):
+            if k == 12:
+                batch.solve(rtol=1e-5)
+                ok = all(np.array_equal(batch.get_u(j), in_batch[j]) for j in range(3))
+            else:
+                ok = np.array_equal(systems[k].solve(rtol=1e-5)[0], alone[k])
+            if not ok:
+                wrong.append(k)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(13)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+
+
+def test_a_small_solve_does_not_wait_for_a_large_one():
+    """5,124 nodes (six workgroups) beside a thread that solves 201,051 nodes (197) over and over: on average well
+    under the time of a large solve (4 of 38 ms seen, 39 when clusters ran one at a time)."""
+    large = D.beam_system(meshgen.beam(800, 250, kind=4, jitter=0.2, seed=1))
+    small = D.beam_system(meshgen.beam(182, 27, kind=4, jitter=0.2, seed=2))
+    want, _ = small.solve(rtol=1e-6)
+    large.solve(rtol=1e-4)
+    t = time.perf_counter()
+    large.solve(rtol=1e-4)
+    t_large = time.perf_counter() - t
+    stop = threading.Event()
+
+    def work():
+        while not stop.is_set():
+            large.solve(rtol=1e-4)
+
+    thread = threading.Thread(target=work)
+    thread.start()
+    time.sleep(0.5 * t_large)
+    t = time.perf_counter()
+    got = [small.solve(rtol=1e-6)[0] for _ in range(10)]
+    t_small = (time.perf_counter() - t) / 10
+    stop.set()
+    thread.join()
+    print(f"large {t_large * 1e3:.1f} ms, small beside it {t_small * 1e3:.1f} ms")
+    assert all(np.array_equal(u, want) for u in got)
+    assert t_small < 0.5 * t_large
 
 
 @pytest.mark.parametrize("pre", [D.PRECOND_JACOBI, D.PRECOND_BLOCK_JACOBI])

@@ -552,7 +552,8 @@ struct Cluster {
 
 	// b - A x of the own row with the FP64 matrix, compensated (row_residual in
 	// pcg.hip). x is published for it; the own rows of the window are left
-	// holding keep.
+	// holding keep. HALVES: one half of a block at a time, in fewer registers.
+	template <bool HALVES = false>
 	__device__ __forceinline__ dbl2 true_residual(dbl2 x, dbl2 keep) {
 		publish(x);
 		dbl2 res = {0, 0};
@@ -569,10 +570,18 @@ struct Cluster {
 			for (int blk = beg; blk < end; blk += kSlice) {
 				int const c = V.col[blk];
 				int64_t const o = 4 * static_cast<int64_t>(blk) - 2 * r64;
-				dbl2 const a = ld2(V.val + o), d = ld2(V.val + o + 2 * kSlice);
+				dbl2 const a = ld2(V.val + o);
+				dbl2 d = {0, 0};
+				if (!HALVES) {
+					d = ld2(V.val + o + 2 * kSlice);
+				}
 				dbl2 const xv = c >= r0 && c < r1 ? win[c - lo] : receive(c);
 				sub_exact(s0, c0, a.x, xv.x);
 				sub_exact(s0, c0, a.y, xv.y);
+				if (HALVES) {
+					asm volatile("" : "+v"(s0), "+v"(c0)::"memory");
+					d = ld2(V.val + o + 2 * kSlice);
+				}
 				sub_exact(s1, c1, d.x, xv.x);
 				sub_exact(s1, c1, d.y, xv.y);
 			}
@@ -592,11 +601,16 @@ struct Cluster {
 // the x in V.x, 2 continues a run cut at its limit (R as it was left, r and p in
 // V.save). Runs until R.iter >= stop. A workgroup that left because a wait ran
 // out leaves its part of V.x as it was.
-// LEAN forms z = M^-1 r again where p needs it instead of keeping it. Block Jacobi
-// with 1024 threads otherwise spills 12 registers, outside its loop but for one
-// load and store, which hide: 5,124 nodes 4.78 us an iteration, LEAN 4.96. It is
-// for the solve that allocates nothing: for the first launch that needs scratch
-// memory the runtime takes some from the device (16 MiB).
+// LEAN forms z = M^-1 r again where p needs it instead of keeping it, and takes the
+// blocks of a true residual by halves. One system's block Jacobi with 1024 threads
+// otherwise spills 12 registers, outside its loop but for one load and store,
+// which hide: 5,124 nodes 4.78 us an iteration, LEAN 4.96. There it is for the
+// solve that allocates nothing: for the first launch that needs scratch memory
+// the runtime takes some from the device (16 MiB). The batch kernels carry more
+// state and spill 20 to 27 registers, LEAN 10 to 13, most of them in the true
+// residual: 256 panels of 500 to 4,000 nodes 15.7 ms with point and 15.2 with
+// block Jacobi, LEAN 14.9 and 14.3; 24 of 10,000 to 30,000 45.9 and 45.5, LEAN
+// 42.8 and 41.5.
 template <typename MT, int W, int PRE, int NT, bool LEAN = false>
 __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, double delta2, int64_t stop,
                         bool final_check, Shared& sh, dbl2* lds, Run& R) {
@@ -662,7 +676,7 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 			}
 		}
 		if (mode == 1) {
-			r = C.true_residual(x_get(), pn);
+			r = C.template true_residual<LEAN>(x_get(), pn);
 		}
 		z = precond(r);
 		dbl2 const bv = C.live ? ld2(V.b + 2 * static_cast<int64_t>(C.row)) : dbl2{0, 0};
@@ -751,7 +765,7 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 		if ((at_tol && !R.checking) || (every && (R.checking || R.rr <= delta2 * R.rr_ref))) {
 			// the true residual replaces the recursive one (the directions are
 			// kept) and decides about the end
-			r = C.true_residual(x_get(), pn);
+			r = C.template true_residual<LEAN>(x_get(), pn);
 			z = precond(r);
 			double v3[2] = {r.x * z.x + r.y * z.y, r.x * r.x + r.y * r.y};
 			C.gather(v3, 2);
@@ -785,7 +799,7 @@ __device__ void run_pcg(View const& V, int g, int G, int mode, double rtol2, dou
 	}
 	R.beta = beta;
 	if (status == 0 && final_check && R.checks == 0) {
-		dbl2 const rt = C.true_residual(x_get(), pn);
+		dbl2 const rt = C.template true_residual<LEAN>(x_get(), pn);
 		double v[1] = {rt.x * rt.x + rt.y * rt.y};
 		C.gather(v, 2);
 		R.rr_true = v[0];

@@ -435,7 +435,7 @@ __global__ __launch_bounds__(kRows) void k_resident_batch(const View* __restrict
 		}
 		View const V = views[k];
 		Run R;
-		run_pcg<double, W, PRE, kRows>(V, M.g, M.G, 0, rtol2, 0.0, max_iter, true, sh,
+		run_pcg<double, W, PRE, kRows, true>(V, M.g, M.G, 0, rtol2, 0.0, max_iter, true, sh,
 		                               reinterpret_cast<resident::dbl2*>(dyn), R);
 		if (M.g == 0 && threadIdx.x == 0) {
 			out[k].iter = R.iter;

@@ -640,8 +640,9 @@ int pool_alloc_bytes(void** p, size_t bytes);
 void pool_free_bytes(void* p);
 
 // A pinned (device-visible) host buffer of at least `bytes`, one per host
-// thread and slot (0 .. kStagingSlots - 1), grown as needed and kept until
-// the process ends; valid until the thread's next call for the same slot.
+// thread and slot (0 .. kStagingSlots - 1), grown as needed and passed on to
+// another thread when this one ends; valid until the thread's next call for the
+// same slot.
 // Slots: 0 a level's graph and 1 counts read back (the multigrid build), 2 a
 // small system's load or solution.
 constexpr int kStagingSlots = 3;

@@ -168,13 +168,49 @@ int pinned_staging(void** out, size_t bytes, int slot) {
 		void* p = nullptr;
 		size_t cap = 0;
 	};
-	// not freed at thread exit: the HIP runtime may already be gone then
-	thread_local Staging* slots = new Staging[kStagingSlots];
+	// A thread's buffers pass to the next thread that needs some: never freed at
+	// its exit, when the HIP runtime may already be gone, and never more of them
+	// than threads at once used (a buffer too small is freed for a larger one).
+	struct Left {
+		std::mutex m;
+		std::vector<Staging> of[kStagingSlots];
+	};
+	static Left* const left = new Left;   // never destroyed, as the pool
+	struct Mine {
+		Staging of[kStagingSlots];
+		~Mine() {
+			std::lock_guard<std::mutex> const lock(left->m);
+			for (int k = 0; k < kStagingSlots; k++) {
+				if (of[k].p) {
+					try {
+						left->of[k].push_back(of[k]);
+					} catch (const std::bad_alloc&) {   // lost
+					}
+					of[k] = Staging{};
+				}
+			}
+		}
+	};
+	thread_local Mine mine;
 	if (slot < 0 || slot >= kStagingSlots) {
 		set_error("pinned staging slot %d out of range", slot);
 		return BFMX_E_ARG;
 	}
-	Staging* const st = &slots[slot];
+	Staging* const st = &mine.of[slot];
+	if (!st->p) {
+		std::lock_guard<std::mutex> const lock(left->m);
+		auto& v = left->of[slot];
+		if (!v.empty()) {
+			// the smallest that holds the request, else the largest
+			auto const better = [&](Staging const& a, Staging const& b) {
+				bool const fa = a.cap >= bytes, fb = b.cap >= bytes;
+				return fa != fb ? fa : fa ? a.cap < b.cap : a.cap > b.cap;
+			};
+			auto const at = std::min_element(v.begin(), v.end(), better);
+			*st = *at;
+			v.erase(at);
+		}
+	}
 	if (st->cap < bytes) {
 		if (st->p) {
 			(void) hipHostFree(st->p);

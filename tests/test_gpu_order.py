@@ -32,6 +32,38 @@ def test_given_loads_and_solutions(nx, ny):
     assert np.linalg.norm(b3 - A @ u3) <= 1.1e-8 * np.linalg.norm(b3)
 
 
+def test_a_thread_leaves_its_pinned_buffer_to_the_next():
+    """Below 16,384 nodes a load and a solution go through a pinned buffer of the calling thread (256 KB here). Sixty
+    threads one after another use one of them, not sixty: the process maps no more device memory than after the first
+    few."""
+    s = D.beam_system(meshgen.beam(127, 120, kind=4, jitter=0.2, seed=2))
+    small = D.beam_system(meshgen.beam(8, 3, kind=4))
+    b, b_small = s.get_rhs(), small.get_rhs()
+    want, _ = s.solve(b=b, precond=D.PRECOND_AMG, rtol=1e-6)
+    want_small, _ = small.solve(b=b_small, rtol=1e-6)
+    wrong = []
+
+    def mapped():
+        with open("/proc/self/maps") as f:
+            return sum("/dev/dri/" in line or "/dev/kfd" in line for line in f)
+
+    def work(k):
+        u, _ = s.solve(b=b, precond=D.PRECOND_AMG, rtol=1e-6)
+        v, _ = small.solve(b=b_small, rtol=1e-6)
+        if not (np.array_equal(u, want) and np.array_equal(s.get_u(), want) and np.array_equal(v, want_small)):
+            wrong.append(k)
+
+    counts = []
+    for k in range(60):
+        t = threading.Thread(target=work, args=(k,))
+        t.start()
+        t.join()
+        counts.append(mapped())
+    print(f"mapped: {counts[4]} after 5 threads, {counts[-1]} after {len(counts)}")
+    assert not wrong
+    assert counts[4] > 0 and counts[-1] <= counts[4] + 4
+
+
 def test_batches_on_two_threads_share_a_large_system():
     """Both batches read the solution of the same system, whose permutation goes to the device at the first read."""
     s = D.beam_system(meshgen.beam(255, 64, kind=3, jitter=0.2, seed=2))

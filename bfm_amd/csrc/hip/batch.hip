@@ -1123,7 +1123,12 @@ int batch_solve_amg(bfmx_batch* b, double rtol, int64_t max_iter, bfmx_stats_t* 
 
 namespace {
 
-// The batch's clusters (at its first Jacobi solve): the systems that fit, and
+bool clusters_allowed(const bfmx_batch* b) {
+	const char* e = std::getenv("BFMX_RESIDENT");
+	return !(e && e[0] == '0') && std::chrono::steady_clock::now() >= b->res_retry;
+}
+
+// The batch's clusters (at its first Jacobi solve or tuning): the systems that fit, and
 // the rest by class for the streaming kernel.
 int make_plan(bfmx_batch* b) {
 	if (b->planned) {
@@ -1158,8 +1163,7 @@ int make_plan(bfmx_batch* b) {
 // to take them all.
 int solve_resident(bfmx_batch* b, int pre, double rtol2, int64_t max_iter, const int* picks, bool* ran) {
 	*ran = false;
-	const char* e = std::getenv("BFMX_RESIDENT");
-	if ((e && e[0] == '0') || std::chrono::steady_clock::now() < b->res_retry) {
+	if (!clusters_allowed(b)) {
 		return BFMX_OK;
 	}
 	BFMX_CHECK(make_plan(b));
@@ -1304,20 +1308,33 @@ int batch_autotune(bfmx_batch* b, int pre, int sample, int iters, int32_t* picks
 		set_error("batched solves use Jacobi or block-Jacobi PCG");
 		return BFMX_E_UNSUPPORTED;
 	}
+	// only what a solve gives to the streaming kernel is timed
+	bool const clusters = clusters_allowed(b);
+	if (clusters) {
+		BFMX_CHECK(make_plan(b));
+	}
+	bool const rest = clusters && b->plan;
+	const int32_t* first[kClasses];
+	int all[kClasses];
+	const int32_t* at = b->d_rest;
+	for (int c = kClasses - 1; c >= 0; c--) {
+		all[c] = rest ? b->rest_count[c] : b->class_off[c + 1] - b->class_off[c];
+		first[c] = rest ? at : b->d_order + b->class_off[c];
+		at += b->rest_count[c];
+	}
 	launch_assemble(b);
 	BFMX_HIP(hipGetLastError());
 	for (int c = 0; c < kClasses; c++) {
-		int const all = b->class_off[c + 1] - b->class_off[c];
-		int const cnt = sample > 0 ? std::min(sample, all) : all;
+		int const cnt = sample > 0 ? std::min(sample, all[c]) : all[c];
 		int best = kDefaultPick[c];
 		float best_ms = 0;
 		for (int cfg = 0; cfg < kConfigs; cfg++) {
 			float ms = 0;
 			if (cnt > 0) {
 				// tiny rtol: every sampled system runs exactly `iters` iterations
-				launch(pre, cfg, cnt, b->stream, b->d_inst, b->d_order + b->class_off[c], 1e-300, iters, b->d_out);
+				launch(pre, cfg, cnt, b->stream, b->d_inst, first[c], 1e-300, iters, b->d_out);
 				BFMX_HIP(hipEventRecord(b->ev[0], b->stream));
-				launch(pre, cfg, cnt, b->stream, b->d_inst, b->d_order + b->class_off[c], 1e-300, iters, b->d_out);
+				launch(pre, cfg, cnt, b->stream, b->d_inst, first[c], 1e-300, iters, b->d_out);
 				BFMX_HIP(hipEventRecord(b->ev[1], b->stream));
 				BFMX_HIP(hipEventSynchronize(b->ev[1]));
 				BFMX_HIP(hipGetLastError());

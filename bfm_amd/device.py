@@ -501,7 +501,8 @@ class Batch:
 
     def autotune(self, precond=PRECOND_JACOBI, sample=0, iters=32):
         """(picks (3,), times_ms (3, 5)): the fastest configuration of each size
-        class, timed on `sample` systems of the class (0: all)."""
+        class, timed on `sample` systems of the class (0: all) that no cluster
+        takes (a class without any: the default, times 0)."""
         picks = np.zeros(BATCH_CLASSES, np.int32)
         times = np.zeros(BATCH_CLASSES * BATCH_CONFIGS)
         _check(lib().bfmx_batch_autotune(self.h, precond, sample, iters, picks, times))

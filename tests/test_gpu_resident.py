@@ -256,6 +256,32 @@ def test_a_system_after_a_broken_one(pre):
         assert np.array_equal(b.get_u(8 + k), alone.get_u(k))
 
 
+def test_autotune_times_what_streams(monkeypatch):
+    """Configurations apply to the systems that fit no cluster; only these are timed, each in its size class."""
+    fit = [D.beam_system(strip(n, 4, het=False)) for n in (200, 3000, 9000)]
+    wide = meshgen.beam(120, 50, kind=4, jitter=0.2, seed=4)     # 6,171 nodes in no order: the middle class
+    p = np.random.default_rng(1).permutation(wide.n_nodes)
+    q = np.empty_like(p)
+    q[p] = np.arange(p.size)
+    wide.coords, wide.elems = wide.coords[p], q[wide.elems.astype(np.int64)].astype(np.uint64)
+    wide.edges = q[wide.edges.astype(np.int64)]
+    wide.node_sets = {name: v[p] for name, v in wide.node_sets.items()}
+    streams = D.beam_system(wide, renumber=False)
+    b = D.Batch(fit)
+    default, times = b.autotune(iters=8)
+    assert not times.any()
+    u = [b.solve(rtol=1e-6, picks=default) and b.get_u(k) for k in range(3)]
+    picks, times = D.Batch([fit[2], streams, fit[0], fit[1]]).autotune(iters=8)
+    assert (times[1] > 0).all() and not times[0].any() and not times[2].any()
+    assert picks[1] == times[1].argmin() and picks[0] == default[0] and picks[2] == default[2]
+    monkeypatch.setenv("BFMX_RESIDENT", "0")
+    _, times = b.autotune(iters=8)
+    assert (times > 0).all()
+    monkeypatch.delenv("BFMX_RESIDENT")
+    b.solve(rtol=1e-6)
+    assert all(np.array_equal(b.get_u(k), u[k]) for k in range(3))
+
+
 def ring(nx, ny, kind=4):
     """An axisymmetric ring (indefinite: MINRES)."""
     m = meshgen.beam(nx, ny, kind=kind, length=4.0, height=1.0, jitter=0.2, seed=12)

@@ -1143,6 +1143,11 @@ int make_plan(bfmx_batch* b) {
 		                               {words(I.r), words(I.z), words(I.q), words(I.p0)}, words(I.p1), I.dinv,
 		                               &b->d_out[views.size()].gave_up, I.n});
 	}
+	// an attempt that failed half-way (no memory for the rest) leaves nothing
+	resident::plan_destroy(b->plan);
+	b->plan = nullptr;
+	dfree(b->d_rest);
+	std::fill(std::begin(b->rest_count), std::end(b->rest_count), 0);
 	BFMX_CHECK(resident::plan_create(&b->plan, b->systems, views, b->stream));
 	if (b->plan && !resident::plan_rest(b->plan).empty()) {
 		std::vector<int32_t> rest = resident::plan_rest(b->plan);

@@ -22,9 +22,9 @@ pytestmark = pytest.mark.gpu
 RTOL = 1e-9
 
 
-def strip(n, kind, het, seed=5):
+def strip(n, kind, het, seed=5, h=None):
     """A beam of exactly n nodes: a grid h nodes high, cut off along its last column."""
-    h = 4 if n < 256 else 16 if n < 1000 else 32 if n < 4000 else 96
+    h = h or (4 if n < 256 else 16 if n < 1000 else 32 if n < 4000 else 96)
     nx = -(-n // h)
     m = meshgen.beam(nx, h - 1, kind=kind, length=nx / h, height=1.0, jitter=0.2, seed=seed)
     # nodes column by column, so that the first n of them are a prefix of the grid
@@ -62,14 +62,15 @@ def check(s, u, ref, st, rtol):
     assert rel_err(u, ref) <= 1e-6
 
 
-# one workgroup of 512 and of 1024 threads, then clusters: full, one row over, an uneven last one
-@pytest.mark.parametrize("n", [8, 64, 511, 512, 514, 1022, 1024, 1026, 2048, 2050, 3200])
+# one workgroup of 512 and of 1024 threads, then clusters: full, a few rows less and over, an uneven last one
+@pytest.mark.parametrize("n", [8, 64, 511, 512, 514, 515, 1022, 1023, 1024, 1026, 1027, 2047, 2048, 2050, 2051, 3200])
 @pytest.mark.parametrize("kind,pre,precision", [(4, D.PRECOND_JACOBI, D.FP64), (3, D.PRECOND_BLOCK_JACOBI, D.FP64),
                                                 (4, D.PRECOND_BLOCK_JACOBI, D.MIXED)])
 def test_workgroup_edges(monkeypatch, n, kind, pre, precision):
-    if precision == D.MIXED and n < 512:
+    if precision == D.MIXED and n < 500:
         pytest.skip("the FP32 operator stalls above rtol on the smallest strips, on either path")
-    m = strip(n + n % 2, kind, het=pre == D.PRECOND_BLOCK_JACOBI and precision == D.FP64)
+    m = strip(n, kind, het=pre == D.PRECOND_BLOCK_JACOBI and precision == D.FP64)
+    assert m.n_nodes == n
     s = D.beam_system(m)
     rtol = 1e-8 if precision == D.MIXED else RTOL
     ref, st_ref, u, st = both(monkeypatch, s, precond=pre, precision=precision, rtol=rtol)
@@ -77,6 +78,47 @@ def test_workgroup_edges(monkeypatch, n, kind, pre, precision):
     check(s, u, ref, st, rtol)
     again, st2 = s.solve(precond=pre, precision=precision, rtol=rtol)
     assert np.array_equal(u, again) and st2["iterations"] == st["iterations"]
+
+
+# Columns of 600 and 900 nodes in their own order: a workgroup of 1,024 rows reads some 1,200 and 1,800 nodes of
+# others (more than one a thread; 2,826 is near the widest window), one of MINRES's 512 rows the same.
+@pytest.mark.parametrize("n,h,pre,precision",
+                         [(6000, 600, D.PRECOND_JACOBI, D.FP64), (6005, 600, D.PRECOND_BLOCK_JACOBI, D.FP64),
+                          (6050, 600, D.PRECOND_JACOBI, D.MIXED), (7200, 900, D.PRECOND_BLOCK_JACOBI, D.FP64),
+                          (6000, 600, D.PRECOND_MINRES, D.FP64)])
+def test_wide_windows(monkeypatch, n, h, pre, precision):
+    s = D.beam_system(strip(n, 4, het=False, h=h), renumber=False)
+    kw = dict(precond=pre, precision=precision, rtol=1e-8, max_iter=20000)
+    ref, st_ref, u, st = both(monkeypatch, s, **kw)
+    print(f"{n} nodes: {st_ref['iterations']} / {st['iterations']} iterations, difference {rel_err(u, ref):.1e}")
+    assert not np.array_equal(u, ref)        # it was not streamed
+    check(s, u, ref, st, 1e-8)
+    monkeypatch.setenv("BFMX_RESIDENT_ITERS", "48")
+    u2, st2 = s.solve(**kw)
+    assert st2["iterations"] == st["iterations"] and np.array_equal(u, u2)
+
+
+@pytest.mark.parametrize("nx,ny", [(70, 20), (480, 69), (1200, 100)])
+def test_minres_of_many_workgroups(monkeypatch, nx, ny):
+    """Three, 66 and 237 workgroups of 512 rows (most with neighbours on both sides; the sums over more than 64 are
+    gathered by several wavefronts). Both paths are cut after 100 iterations, before the Lanczos vectors lose their
+    orthogonality: the same recurrences in another order of summation, whose iterates agree to 1e-10 (seen 1e-12)."""
+    s = D.beam_system(meshgen.beam(nx, ny, kind=4, jitter=0.2, seed=3))
+
+    def iterate():
+        with pytest.raises(D.BfmxError) as e:
+            s.solve(precond=D.PRECOND_MINRES, rtol=1e-10, max_iter=100)
+        assert e.value.code == -5 and "100 iterations" in str(e.value)
+        return s.get_u()
+
+    monkeypatch.setenv("BFMX_RESIDENT", "0")
+    ref = iterate()
+    monkeypatch.delenv("BFMX_RESIDENT")
+    u = iterate()
+    print(f"{s.n_nodes} nodes: difference {rel_err(u, ref):.1e}")
+    assert not np.array_equal(u, ref) and rel_err(u, ref) <= 1e-10
+    monkeypatch.setenv("BFMX_RESIDENT_ITERS", "7")
+    assert np.array_equal(iterate(), u)
 
 
 @pytest.mark.parametrize("nx,ny,precision", [(24, 6, D.FP64), (80, 20, D.FP64), (80, 20, D.MIXED)])
@@ -355,7 +397,7 @@ def test_a_wait_that_runs_out_in_a_batch(monkeypatch):
 def test_minres(monkeypatch, nx, ny, kind):
     """Axisymmetric rings of 12 to 915 nodes (one workgroup of 512, and two) against the recurrences on the host;
     a run cut into launches is the same run. K is indefinite with a condition number of about 1e5 here: two
-    solutions whose residuals meet 1e-8 agree to 1e-3; seen 1e-9."""
+    solutions whose residuals meet 1e-8 agree to 1e-3 at the worst; seen 2e-9, of which a hundred times is allowed."""
     s = ring(nx, ny, kind)
     kw = dict(precond=D.PRECOND_MINRES, rtol=1e-8)
     ref, st_ref, u, st = both(monkeypatch, s, **kw)
@@ -363,7 +405,7 @@ def test_minres(monkeypatch, nx, ny, kind):
     assert abs(st["iterations"] - st_ref["iterations"]) <= 0.1 * st_ref["iterations"] + 10
     A, b = s.get_csr_scipy(), s.get_rhs()
     assert st["status"] == 0 and np.linalg.norm(b - A @ u) <= 1.1e-8 * np.linalg.norm(b)
-    assert rel_err(u, ref) <= 1e-3
+    assert rel_err(u, ref) <= 2e-7
     monkeypatch.setenv("BFMX_RESIDENT_ITERS", "7")
     u2, st2 = s.solve(**kw)
     assert st2["iterations"] == st["iterations"] and np.array_equal(u, u2)

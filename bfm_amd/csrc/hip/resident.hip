@@ -108,6 +108,20 @@ PcgKernel pick(bool mixed, int width, int pre, int nt, bool no_scratch) {
 	return width <= 7 ? pick_precond<double, 7>(pre, nt) : pick_precond<double, 9>(pre, nt);
 }
 
+// The kernel may be launched with lds bytes of dynamic LDS. The limit belongs to
+// the kernel, not to the launch: always the same one, the CU's 160 KB without
+// Shared and the batch kernel's word, so that threads do not lower it for each
+// other.
+int allow_lds(const void* kernel, size_t lds) {
+	constexpr int kMost = 160 * 1024 - 2048;
+	static_assert(sizeof(Shared) + 64 <= 2048 &&
+	              kMaxWindow * sizeof(resident::dbl2) + fixed_bytes<double, kMaxWidth, kRows>() <= kMost);
+	if (lds > 48 * 1024) {
+		BFMX_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kMost));
+	}
+	return BFMX_OK;
+}
+
 // LDS bytes beside the window.
 int fixed(bool mixed, int width, int nt) {
 	return mixed || nt <= 512 ? 0 : width <= 7 ? fixed_bytes<double, 7, 1024>() : fixed_bytes<double, 9, 1024>();
@@ -199,10 +213,7 @@ int resident_pcg(bfmx_system* s, int precond, bool mixed, double rtol2, double d
 	int const nt = n <= 512 ? 512 : 1024;
 	PcgKernel const kernel = pick(mixed, s->res_width, precond, nt, no_scratch);
 	size_t const lds = static_cast<size_t>(s->res_window) * sizeof(resident::dbl2) + fixed(mixed, s->res_width, nt);
-	if (lds > 48 * 1024) {
-		BFMX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-		                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-	}
+	BFMX_CHECK(allow_lds(reinterpret_cast<const void*>(kernel), lds));
 	// (tests cut runs into many launches)
 	const char* cut = std::getenv("BFMX_RESIDENT_ITERS");
 	int64_t const per_launch = cut && std::atoll(cut) > 0 ? std::atoll(cut) : kPerLaunch;
@@ -298,10 +309,7 @@ int resident_minres(bfmx_system* s, double rtol, int64_t cap, MinresResult* out,
 		int const width = *std::max_element(s->row_len.begin(), s->row_len.end());
 		auto const kernel = width <= 7 ? k_resident_minres<7> : k_resident_minres<9>;
 		size_t const lds = static_cast<size_t>(win) * sizeof(resident::dbl2);
-		if (lds > 48 * 1024) {
-			BFMX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-			                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-		}
+		BFMX_CHECK(allow_lds(reinterpret_cast<const void*>(kernel), lds));
 		const char* cut = std::getenv("BFMX_RESIDENT_ITERS");
 		int64_t const per_launch = cut && std::atoll(cut) > 0 ? std::atoll(cut) : kPerLaunch;
 		for (int fresh = 1; !gave_up && R.status == 0 && (fresh || R.iter < cap); fresh = 0) {
@@ -659,8 +667,7 @@ int plan_launch(Plan* p, hipStream_t st, int precond, double rtol2, int64_t max_
 	auto const kernel = p->width <= 7
 	                        ? (point ? k_resident_batch<7, BFMX_PRECOND_JACOBI> : k_resident_batch<7, BFMX_PRECOND_BLOCK_JACOBI>)
 	                        : (point ? k_resident_batch<9, BFMX_PRECOND_JACOBI> : k_resident_batch<9, BFMX_PRECOND_BLOCK_JACOBI>);
-	BFMX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-	                             static_cast<int>(p->lds)));
+	BFMX_CHECK(allow_lds(reinterpret_cast<const void*>(kernel), p->lds));
 	k_clear_batch<<<p->taken * kClearParts, kBlock, 0, st>>>(p->d_views, p->d_order, p->d_groups, p->d_queues, p->queues,
 	                                                         p->d_post, p->clusters, d_out, n);
 	BFMX_HIP(hipGetLastError());

@@ -209,9 +209,9 @@ def copy_calibration(nbytes):
 def batched_leg(D, meshgen, count, rtol):
     """The batched workload: `count` seeded holed panels (1k-60k DOFs, plane
     strain, traction U(1e5, 1e7) N/m on top, bottom corners pinned), built
-    into one batch from their meshes; one timed launch assembles every panel
-    (a launch per colour over all of them) and solves it by block-Jacobi PCG
-    to rtol (a cluster of workgroups each; the autotuner's configurations are
+    into one batch from their meshes; one timed call assembles every panel
+    (above 1,024 panels one workgroup each, else a launch per colour over all
+    of them) and solves it by block-Jacobi PCG to rtol (a cluster of workgroups each; the autotuner's configurations are
     for panels that do not fit one)."""
     t = time.perf_counter()
     inst, sizes, dofs = [], [], 0
@@ -231,7 +231,7 @@ def batched_leg(D, meshgen, count, rtol):
     picks, times = b.autotune(precond=pre)
     t_tune = time.perf_counter() - t
     log(f"batched: autotune {t_tune:.1f} s, picks {picks.tolist()}")
-    b.solve(precond=pre, rtol=rtol, picks=picks)         # graph capture + first launch
+    b.solve(precond=pre, rtol=rtol, picks=picks)         # clusters planned, first launch
     t = time.perf_counter()
     st, ms = b.solve(precond=pre, rtol=rtol, picks=picks)
     wall = time.perf_counter() - t
@@ -263,7 +263,7 @@ def batched_leg(D, meshgen, count, rtol):
     worst = max(x["rel_residual"] for x in st_mg)
     log(f"batched multigrid: {ms_mg:.1f} ms device ({wall_mg * 1e3:.1f} ms wall), {dofs / (ms_mg / 1e3):.3e} DOF/s, "
         f"{st_mg[0]['iterations']} iterations, worst instance residual {worst:.2e}, {ms / ms_mg:.2f}x the "
-        f"persistent launch; first launch (union and hierarchy build) {t_mg_setup:.1f} s")
+        f"block-Jacobi solve; first launch (union and hierarchy build) {t_mg_setup:.1f} s")
     return {
         "workload": f"{count} holed panels (seeds 0-{count - 1}), 1k-60k DOFs, plane strain, block-Jacobi PCG "
                     f"to rtol {rtol:g}, assembled and solved from one call",
@@ -274,7 +274,8 @@ def batched_leg(D, meshgen, count, rtol):
                                                                               "autotune": t_tune},
         "roofline": {"bound": "latency of the clusters' exchanges and issue (the matrix stays in registers)",
                      "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS,
-                     "traffic": None, "kernel": "k_resident_batch (block Jacobi) + k_batch_elements (whole launch)",
+                     "traffic": None, "kernel": "k_resident_batch (block Jacobi) + "
+                                               f"{'k_batch_colors' if count > 1024 else 'k_batch_elements'} (whole call)",
                      "algorithmic_bytes": byt, "streamed_bytes_of_its_iterations": streamed},
         "multigrid": {
             "solver": "the batch as one block-diagonal system: flexible CG (FP64) + FP32 smoothed-aggregation "

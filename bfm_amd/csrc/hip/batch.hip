@@ -1,10 +1,11 @@
 // Batched solves: many independent planar systems of uneven sizes.
 //
-// Systems whose matrix fits the registers of a cluster of workgroups (rows of
-// at most nine blocks, up to 262,144 nodes) are solved by resident.hip, each
-// cluster taking one system after another. The others, and all of them where a
-// cluster's bounded wait ran out, are solved by the streaming kernel below, one persistent launch per size class (captured in
-// one HIP graph when it solves the whole batch).
+// Systems whose matrix fits the registers of a cluster of workgroups (up to
+// 262,144 nodes, rows of at most nine blocks, windows of at most 2,900 nodes:
+// resident.h) are solved by resident.hip, each cluster taking one system after
+// another. The others, and all of them where a cluster's bounded wait ran out,
+// are solved by the streaming kernel below, one persistent launch per size class
+// (captured in one HIP graph when it solves the whole batch).
 //
 // In the streaming kernel one workgroup runs the whole Jacobi or block-Jacobi
 // PCG of one system: its passes over the rows (SpMV with the direction update
@@ -18,8 +19,9 @@
 //
 // Tuning: the workgroup size and the rows each thread takes per step (the
 // independent row chains in flight per thread) are template parameters. The
-// autotuner times every configuration on a sample of each size class and
-// records its picks, which bfmx_batch_solve replays.
+// autotuner times every configuration on a sample of each size class, of the
+// systems that no cluster takes, and records its picks, which bfmx_batch_solve
+// replays.
 //
 // Workspace: one packed FP64 allocation, per system x, r, z, p0, p1, q (2 per
 // node each) and the Jacobi inverses (4 per node).

@@ -1,9 +1,9 @@
 // Preconditioned conjugate gradients on the device.
 //
 // Point and block Jacobi PCG of a system whose matrix fits the GPU's registers
-// (up to 262,144 nodes, rows of at most nine blocks) runs in one launch
-// (resident.hip, three to five times as fast); the kernels here take the
-// larger systems and those it refuses.
+// (up to 262,144 nodes, rows of at most nine blocks, windows of at most 2,900
+// nodes: resident.h) runs in one launch (resident.hip; an iteration is 2.6 to 8
+// times as fast); the kernels here take the others.
 //
 // One CG iteration is four kernels:
 //   k_cg_spmv    p_new = z + beta p_old and q = A p_new for its rows, gathering

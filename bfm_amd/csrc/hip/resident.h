@@ -15,7 +15,8 @@
 //     every workgroup forms p = z + beta p for its whole window, so that only
 //     z is exchanged;
 //   * z and the partial dot products travel through memory in 8-byte words of
-//     32 data bits and the 32-bit number of the exchange, written and read with
+//     32 data bits and the 32-bit number of the exchange (the low-latency protocol
+//     of collective libraries), written and read with
 //     agent-scope relaxed atomics (which pass by the XCDs' incoherent L2s). A
 //     reader polls the word itself until it carries the expected number, so an
 //     exchange costs one store-to-load latency (1.3 us up to 4 workgroups, 1.8
@@ -604,9 +605,10 @@ struct Cluster {
 // LEAN forms z = M^-1 r again where p needs it instead of keeping it, and takes the
 // blocks of a true residual by halves. One system's block Jacobi with 1024 threads
 // otherwise spills 12 registers, outside its loop but for one load and store,
-// which hide: 5,124 nodes 4.78 us an iteration, LEAN 4.96. There it is for the
-// solve that allocates nothing: for the first launch that needs scratch memory
-// the runtime takes some from the device (16 MiB). The batch kernels carry more
+// which hide: 915 nodes 2.65 us an iteration, LEAN 2.69; 5,124 4.72 either way;
+// 22,857 4.87, LEAN 4.98. There it is for the solve that allocates nothing: for
+// the first launch that needs scratch memory the runtime takes some from the
+// device (16 MiB). The batch kernels carry more
 // state and spill 20 to 27 registers, LEAN 10 to 13, most of them in the true
 // residual: 256 panels of 500 to 4,000 nodes 15.7 ms with point and 15.2 with
 // block Jacobi, LEAN 14.9 and 14.3; 24 of 10,000 to 30,000 45.9 and 45.5, LEAN

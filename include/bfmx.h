@@ -292,10 +292,16 @@ int bfmx_system_apply_model(bfmx_system_t* s, const double* r, double* z);
  * persistent launch per size class (systems of < 2048, < 8192, >= 8192 nodes).
  * A batch holds either existing assembled systems (bfmx_batch_create) or
  * meshes that every launch assembles before solving
- * (bfmx_batch_create_planar). Systems of at most 262,144 nodes and nine blocks
- * a row are solved by clusters of workgroups that hold the matrix in registers,
- * whatever the configuration; configurations apply to the others. A
- * configuration is a workgroup size x rows-per-thread pair:
+ * (bfmx_batch_create_planar). Clusters of workgroups that hold the matrix in
+ * registers solve the systems that fit them, whatever the configuration:
+ * at most 262,144 nodes, at most nine blocks in any row (a node and eight
+ * neighbours, as structured Q1 meshes have; unstructured meshes often have a
+ * row of ten or more), and at most 2,900 nodes, in the solver's RCM order,
+ * between the first and the last that the rows of one workgroup reach (a beam
+ * of 500 x 400 cells fits, one of 500 x 480 does not). The same holds for
+ * bfmx_system_solve with point or block Jacobi, and with MINRES up to 131,072
+ * nodes. Configurations apply to the others. A configuration is a workgroup
+ * size x rows-per-thread pair:
  * 0 = 256 x 1, 1 = 256 x 2, 2 = 512 x 1, 3 = 512 x 2, 4 = 1024 x 1. A
  * system's solution does not depend on the rest of the batch (bitwise, for
  * the same configuration). The systems must outlive the batch and stay

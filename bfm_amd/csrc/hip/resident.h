@@ -358,7 +358,8 @@ struct Cluster {
 		a11 = top[2 * kSlice + 1];
 	}
 
-	// At the end of a run (a gather after the last wait made the flags visible).
+	// At the end of a run. A gather after the last wait made the flags visible,
+	// but for waits at an iteration limit whose values are not used any more.
 	__device__ __forceinline__ void report() const {
 		if (t == 0 && (sh.late || sh.failed)) {
 			*V.gave_up = 1;

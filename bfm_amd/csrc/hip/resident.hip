@@ -350,8 +350,8 @@ int resident_minres(bfmx_system* s, double rtol, int64_t cap, MinresResult* out,
 // its work: in the streaming kernel, one workgroup a system, the largest one's
 // time on one CU is the least a launch can take.
 // Measured, whole launch with the assembly, block Jacobi to 1e-8: 256 panels of
-// 500 to 4,000 nodes 63.2 -> 14.8 ms, 64 panels of 3,000 to 30,000 nodes 835 ->
-// 73 ms, 512 of 500 to 30,000 1,911 -> 466 ms.
+// 500 to 4,000 nodes 63.2 -> 14.5 ms, 64 panels of 3,000 to 30,000 nodes 835 ->
+// 70 ms, 512 of 500 to 30,000 1,911 -> 456 ms.
 
 namespace resident {
 namespace {
